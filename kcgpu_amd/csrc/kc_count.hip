@@ -59,7 +59,7 @@ constexpr int ACC = 8;  // per-class accumulator slots
 // accumulators that, and not the work, bound launches of many small tasks
 // (970,000 node tasks of 96 small graphs, one grab per four: 3.0 ms).
 constexpr uint32_t NQUEUE = 32, QSTRIDE = 16;  // heads, u32 from one to the next
-constexpr uint32_t NSTRIPE = 16;
+constexpr uint32_t NSTRIPE = 32;
 constexpr uint32_t PIVOT_TOP2 = 256;  // largest pivoting task of the four-word register kernel
 
 // one query of a launch: the oriented graph it runs on and its k
@@ -80,6 +80,7 @@ struct CountArgs {
     const QDesc *qd;
     const uint64_t *tasks;  // (query << 32) | vertex-or-edge id
     uint32_t ntasks;
+    const uint32_t *ntasks_p;  // where the device has the number of tasks, when the host does not know it (or null)
     uint32_t nparts;        // partitions per wave the orientation DFS stacks are laid out for
     uint32_t chunk_log;     // log2 of the tasks per queue grab
     uint32_t rmax;          // row capacity of the workspace
@@ -89,10 +90,11 @@ struct CountArgs {
     const uint8_t *binom_ovf;
     uint32_t bstride;       // binom[n * bstride + r]
     uint32_t *qhead;        // NQUEUE heads: chunks taken
-    uint64_t *acc;          // [0] count [1] bytes [2] tasks [3] tree nodes [4] max task ticks [5] sum task ticks
+    uint32_t direct;        // 1: one block per chunk, block i takes chunk i (no queue)
+    uint32_t single;        // 1: one query, its count is summed in acc[0] and acc[6] (below)
+    uint64_t *acc;          // [0] count [1] bytes [2] tasks [3] tree nodes [4] max task ticks [5] sum task ticks [6] count
     uint32_t acc_mask;      // copies of acc - 1 (a wave adds to copy blockIdx & acc_mask)
-    uint32_t q_mask;        // copies of qcount - 1
-    uint64_t *qcount;       // per query (per copy and query, 64 bytes apart, when there are several copies)
+    uint64_t *qcount;       // per query two sums: of the low and of the high 32 bits of what the waves add
     uint32_t *qovf;         // per query
     uint64_t *gscr;
     uint64_t gscr_words;
@@ -1512,13 +1514,15 @@ struct WaveAcc {
 __device__ __attribute__((always_inline)) void flush_query(const CountArgs &a, WaveAcc &w)
 {
     if (w.q == INF32) return;
-    if (lane_id() == 0) {
-        const uint64_t at = a.q_mask ? ((uint64_t)w.q * (a.q_mask + 1) + (blockIdx.x & a.q_mask)) * 8 : w.q;
-        unsigned long long old = atomicAdd((unsigned long long *)&a.qcount[at], (unsigned long long)w.run);
-        if (old + w.run < old || w.run_ovf) {
-            atomicOr(&a.qovf[w.q], 1u);
-        }
+    // low and high half into sums of their own, in one instruction: neither can
+    // wrap, so nothing has to come back, and the host joins them and sees an
+    // overflow of the whole
+    const int lane = lane_id();
+    if (lane < 2 && w.run) {
+        uint64_t *at = a.single ? a.acc + (uint64_t)(blockIdx.x & a.acc_mask) * ACC + 6 * lane : a.qcount + 2ull * w.q + lane;
+        atomicAdd((unsigned long long *)at, (unsigned long long)(lane ? w.run >> 32 : w.run & 0xFFFFFFFFull));
     }
+    if (lane == 0 && w.run_ovf) atomicOr(&a.qovf[w.q], 1u);
     w.any_ovf |= w.run_ovf;
     w.run = 0;
     w.run_ovf = 0;
@@ -1539,17 +1543,15 @@ __device__ __attribute__((always_inline)) Cur select_task(const CountArgs &a, ui
 
 __device__ __attribute__((always_inline)) void finish_wave(const CountArgs &a, WaveAcc &w)
 {
+    if (w.ntask == 0 && w.q == INF32) return;  // (a wide block's other waves have a query, no tasks)
     flush_query(a, w);
     uint32_t nd_wrap = 0;
     const uint64_t nd = wave_sum64_checked(w.nodes, nd_wrap);  // tree nodes are per-lane shares
-    if (lane_id() == 0) {
-        unsigned long long *acc = reinterpret_cast<unsigned long long *>(a.acc + (uint64_t)(blockIdx.x & a.acc_mask) * ACC);
-        atomicAdd(&acc[1], (unsigned long long)w.bytes);
-        atomicAdd(&acc[2], (unsigned long long)w.ntask);
-        atomicAdd(&acc[3], (unsigned long long)nd);
-        atomicMax(&acc[4], (unsigned long long)w.tmax);
-        atomicAdd(&acc[5], (unsigned long long)w.tsum);
-    }
+    unsigned long long *acc = reinterpret_cast<unsigned long long *>(a.acc + (uint64_t)(blockIdx.x & a.acc_mask) * ACC);
+    const int lane = lane_id();
+    const uint64_t v = lane == 1 ? w.bytes : lane == 2 ? w.ntask : lane == 3 ? nd : lane == 5 ? w.tsum : 0ull;
+    if (v) atomicAdd(&acc[lane], (unsigned long long)v);
+    if (lane == 4) atomicMax(&acc[4], (unsigned long long)w.tmax);
 }
 
 __device__ inline uint32_t ld_head(uint32_t *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -1563,9 +1565,13 @@ __device__ inline uint32_t ld_head(uint32_t *p) { return __hip_atomic_load(p, __
 // tasks of blocks that had to wait for a slot started last (Chung-Lu n=1.2M,
 // k=5..8: 330 -> 357 ms).
 // One head -> NQUEUE heads: 970,000 node tasks of 96 small graphs at k = 4..7
-// 3.8 -> 2.4 ms a call, 9,208 node tasks of a 10,000-vertex graph 723 -> 226 us.
+// 3.8 -> 2.4 ms a call.
+// Few tasks (host: at most DIRECT_ROUNDS per block slot) need no queue: the
+// launch has one block per chunk and the device starts the blocks in order.
+// 8,192 waves that look at the heads once and leave take 80 us: 9,208 node
+// tasks of a 10,000-vertex graph 559 us with one head, 77 with NQUEUE, 23 so.
 struct TaskQueue {
-    uint32_t queue;
+    uint32_t queue, left = 1;
     __device__ explicit TaskQueue(uint32_t block) : queue(block % NQUEUE) {}
 };
 
@@ -1582,6 +1588,11 @@ __device__ __attribute__((always_inline)) uint32_t next_tasks(const CountArgs &a
 {
     const uint32_t lane = (uint32_t)lane_id();
     uint32_t c = INF32;
+    if (a.direct) {
+        const bool mine = tq.left && ((uint64_t)blockIdx.x << a.chunk_log) < a.ntasks;
+        tq.left = 0;
+        return mine ? uni32(blockIdx.x << a.chunk_log) : INF32;
+    }
     for (;;) {
         uint32_t i = 0;
         if (lane == 0) i = atomicAdd(&a.qhead[tq.queue * QSTRIDE], 1u);
@@ -1617,6 +1628,7 @@ void k_pivot_reg(CountArgs a)
     // list and starts (256 u32 each, dead once the bitmap is built)
     uint64_t *crows = lds + L.list;
     WaveAcc w;
+    if (a.ntasks_p) a.ntasks = uni32(*a.ntasks_p);
     TaskQueue tq(blockIdx.x);
     for (;;) {
         const uint32_t start = uni32(next_tasks(a, tq));
@@ -1884,6 +1896,7 @@ __global__ __launch_bounds__(64) void k_count(CountArgs a)
     uint64_t *lacc = ws + L.lacc;
     uint32_t *path = reinterpret_cast<uint32_t *>(ws + L.path);
     WaveAcc w;
+    if (a.ntasks_p) a.ntasks = uni32(*a.ntasks_p);
     TaskQueue tq(blockIdx.x);
     for (;;) {
         const uint32_t start = uni32(next_tasks(a, tq));
@@ -2190,7 +2203,7 @@ __device__ inline uint32_t query_of(const uint64_t *qoff, uint32_t nq, uint64_t 
     return lo;
 }
 
-// size of a task: d+(u) for a node, |T| = |N+(u) & N+(v)| for an edge (merge)
+// size of an edge task: |T| = |N+(u) & N+(v)| (merge)
 __global__ __launch_bounds__(256) void k_task_size(const QDesc *qd, const uint64_t *qoff, uint32_t nq, uint64_t total,
                                                     uint32_t *size)
 {
@@ -2199,10 +2212,7 @@ __global__ __launch_bounds__(256) void k_task_size(const QDesc *qd, const uint64
         const uint32_t q = query_of(qoff, nq, gi);
         const QDesc d = qd[q];
         const uint32_t t = (uint32_t)(gi - qoff[q]);
-        if (!d.gran) {
-            size[gi] = d.rowptr[t + 1] - d.rowptr[t];
-            continue;
-        }
+        if (!d.gran) continue;  // (a node task's size is its row length)
         const uint32_t u = d.src[t], v = d.col[t];
         uint32_t i = d.rowptr[u], ie = d.rowptr[u + 1], j = d.rowptr[v], je = d.rowptr[v + 1];
         uint32_t c = 0;
@@ -2228,11 +2238,20 @@ __device__ inline int class_of(uint32_t s, uint32_t top2)
 // Each class from 65 to 1024 vertices is cut into NSUB slices of its size
 // range, largest first, and a class's slices are contiguous in the task
 // array, so a class launch drains its largest tasks first and the long ones
-// do not start last.  Pass 0 counts per slice and takes the max size of the
-// unbounded class and of the launch (bin_max[15]), pass 1 scatters
-// (query << 32 | task).  A wave handles the distinct slices among its lanes
-// one at a time (ballot per slice, one atomic per slice).
+// do not start last.  k_bin_count counts per slice and takes the max size of
+// the unbounded class and of the launch (bin_max[15]), k_bin_offsets places the
+// slices, k_bin_scatter writes (query << 32 | task).
+// A block adds up its tiles (or one tile) in LDS and touches the device's
+// counters once per slice it met: with an atomic per wave and slice, the few
+// counters -- one of them takes most tasks -- bound both passes (0.8 ms each
+// over 7.8 M edge tasks; 970,000 node tasks of 96 graphs: two passes of 176 us
+// -> one of 29 us).
 constexpr int NSUB = 16;
+constexpr int NSLICE = 2 * NCLASS * NSUB;
+constexpr int BIN_T = 256;
+// tasks per thread: 16 keep the device's counters quiet where tasks are many,
+// 2 fill the device where they are few
+constexpr int BIN_I = 16, BIN_I_FEW = 2;
 
 __device__ inline int slice_of(uint32_t s, int c, uint32_t top2)
 {
@@ -2242,54 +2261,190 @@ __device__ inline int slice_of(uint32_t s, int c, uint32_t top2)
     return sl < NSUB ? (int)sl : NSUB - 1;
 }
 
-__global__ __launch_bounds__(256) void k_classify(const QDesc *qd, const uint8_t *qalgo, const uint64_t *qoff,
-                                                   uint32_t nq, uint64_t total, const uint32_t *size, uint32_t *sub_cnt,
-                                                   uint32_t *bin_max, uint32_t *sub_pos, const uint32_t *sub_off,
-                                                   uint64_t *out, int scatter, uint32_t pivot_top2)
+struct BinArgs {
+    const QDesc *qd;
+    const uint8_t *qalgo;
+    const uint64_t *qoff;
+    uint32_t nq;
+    uint32_t pivot_top2;
+    uint64_t total;
+    const uint32_t *size;   // edge tasks' sizes (a node task's is its row length)
+    uint32_t *sub_cnt;      // [NSLICE] tasks of each slice
+    uint32_t *bin_max;      // [16] largest task of the unbounded bins, [15] of the launch
+    uint32_t *sub_pos;      // [NSLICE] tasks of each slice written so far
+    uint32_t *sub_off;      // [NSLICE] first task of each slice
+    uint64_t *out;
+    uint64_t *binom;        // C(n, r), then a byte per entry: over 64 bits (null: not needed)
+    uint32_t brows, bstride;
+};
+
+// the query of the tasks a thread goes through in ascending order
+struct BinCursor {
+    uint32_t q;
+    uint64_t begin, end;  // its global tasks
+    QDesc d;
+    uint32_t algo;
+    __device__ BinCursor(const BinArgs &b, uint64_t gi) { load(b, b.nq == 1 ? 0 : query_of(b.qoff, b.nq, gi)); }
+    __device__ void load(const BinArgs &b, uint32_t qq)
+    {
+        q = qq;
+        begin = b.qoff[q];
+        end = b.qoff[q + 1];
+        d = b.qd[q];
+        algo = b.qalgo[q] ? 1 : 0;
+    }
+    __device__ void seek(const BinArgs &b, uint64_t gi)  // gi < total
+    {
+        while (gi >= end) load(b, q + 1);
+    }
+};
+
+// the slice of global task gi < total of size s, -1 when the task does not run
+__device__ inline int bin_of(const BinArgs &b, const BinCursor &c, uint64_t gi, uint32_t s)
 {
-    const int lane = threadIdx.x & 63;
-    for (uint64_t base = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) & ~63ull; base < total;
-         base += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t gi = base + lane;
-        int fb = -1;
-        uint32_t s = 0, q = 0;
-        if (gi < total) {
-            q = query_of(qoff, nq, gi);
-            const QDesc d = qd[q];
-            const uint32_t need = d.gran ? d.k - 2 : d.k - 1;
-            s = size[gi];
-            if (s >= need && (d.sample <= 1 || (uint32_t)(gi - qoff[q]) % d.sample == d.offset)) {
-                const uint32_t top2 = qalgo[q] ? pivot_top2 : CLASS_ROWS[2];
-                const int c = class_of(s, top2);
-                fb = ((qalgo[q] ? NCLASS : 0) + c) * NSUB + slice_of(s, c, top2);
-            }
+    const QDesc &d = c.d;
+    if (s < (d.gran ? d.k - 2 : d.k - 1) || (d.sample > 1 && (uint32_t)(gi - c.begin) % d.sample != d.offset)) return -1;
+    const uint32_t top2 = c.algo ? b.pivot_top2 : CLASS_ROWS[2];
+    const int cl = class_of(s, top2);
+    return (int)(c.algo * NCLASS + cl) * NSUB + slice_of(s, cl, top2);
+}
+
+__device__ inline uint32_t task_size(const BinArgs &b, const BinCursor &c, uint64_t gi)
+{
+    const uint32_t t = (uint32_t)(gi - c.begin);
+    return c.d.gran ? b.size[gi] : c.d.rowptr[t + 1] - c.d.rowptr[t];
+}
+
+// the sizes of a thread's I tasks of a tile (task i at base + i * BIN_T), all
+// loads in flight together where the tile lies in one query
+template <int I>
+__device__ inline void tile_sizes(const BinArgs &b, BinCursor c, uint64_t base, uint32_t (&s)[I])
+{
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+        const uint64_t gi = base + (uint64_t)i * BIN_T;
+        s[i] = 0;
+        if (gi >= b.total) continue;
+        if (gi >= c.end) c.seek(b, gi);
+        s[i] = task_size(b, c, gi);
+    }
+}
+
+template <int I>
+__global__ __launch_bounds__(BIN_T) void k_bin_count(BinArgs b)
+{
+    __shared__ uint32_t cnt[NSLICE], mx[3];
+    for (int i = threadIdx.x; i < NSLICE; i += BIN_T) cnt[i] = 0;
+    if (threadIdx.x < 3) mx[threadIdx.x] = 0;
+    __syncthreads();
+    uint32_t m[3] = {0, 0, 0};  // largest task; of the unbounded orientation and pivoting bins
+    for (uint64_t base = (uint64_t)blockIdx.x * BIN_T * I; base < b.total; base += (uint64_t)gridDim.x * BIN_T * I) {
+        BinCursor c(b, base);
+        uint32_t s[I];
+        tile_sizes(b, c, base + threadIdx.x, s);
+#pragma unroll
+        for (int i = 0; i < I; ++i) {
+            const uint64_t gi = base + (uint64_t)i * BIN_T + threadIdx.x;
+            if (gi >= b.total) continue;
+            c.seek(b, gi);
+            const int fb = bin_of(b, c, gi, s[i]);
+            if (fb < 0) continue;
+            atomicAdd(&cnt[fb], 1u);
+            m[0] = max(m[0], s[i]);
+            if (fb / NSUB == NCLASS - 1) m[1] = max(m[1], s[i]);
+            if (fb / NSUB == 2 * NCLASS - 1) m[2] = max(m[2], s[i]);
         }
-        if (!scatter) {  // the largest task size of the launch (binomial table rows)
-            uint32_t mx = fb >= 0 ? s : 0;
-            for (int dd = 32; dd >= 1; dd >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, dd, 64));
-            if (lane == 0 && mx) atomicMax(&bin_max[15], mx);
+    }
+    for (int i = 0; i < 3; ++i)
+        if (m[i]) atomicMax(&mx[i], m[i]);
+    __syncthreads();
+    for (int i = threadIdx.x; i < NSLICE; i += BIN_T)
+        if (cnt[i]) atomicAdd(&b.sub_cnt[i], cnt[i]);
+    if (threadIdx.x < 3 && mx[threadIdx.x])
+        atomicMax(&b.bin_max[threadIdx.x == 0 ? 15 : threadIdx.x * NCLASS - 1], mx[threadIdx.x]);
+}
+
+// exact C(n, r) for n <= nmax, r < bstride <= 64, one row a step, by one wave
+// (lane r); the byte after the table is 1 where the value exceeds 2^64-1
+__device__ inline void binom_rows(const BinArgs &b, uint32_t nmax)
+{
+    const uint32_t r = (uint32_t)lane_id();
+    uint8_t *ovf = reinterpret_cast<uint8_t *>(b.binom + (uint64_t)(b.brows) * b.bstride);
+    uint64_t v = r == 0 ? 1 : 0;
+    uint32_t o = 0;
+    for (uint32_t n = 0;; ++n) {
+        if (r < b.bstride) {
+            b.binom[(uint64_t)n * b.bstride + r] = v;
+            ovf[(uint64_t)n * b.bstride + r] = (uint8_t)o;
         }
-        for (uint64_t pend = __ballot(fb >= 0); pend;) {
-            const int leader = __ffsll((unsigned long long)pend) - 1;
-            const int cur = __builtin_amdgcn_readlane(fb, leader);
-            const uint64_t bal = __ballot(fb == cur);
-            pend &= ~bal;
-            if (!scatter) {
-                if (lane == leader) atomicAdd(&sub_cnt[cur], (uint32_t)__popcll(bal));
-                if ((cur / NSUB) % NCLASS == NCLASS - 1) {  // the unbounded class sizes its rows by its max
-                    uint32_t mx = (fb == cur) ? s : 0;
-                    for (int dd = 32; dd >= 1; dd >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, dd, 64));
-                    if (lane == leader) atomicMax(&bin_max[cur / NSUB], mx);
-                }
-            } else {
-                uint32_t b0 = 0;
-                if (lane == leader) b0 = atomicAdd(&sub_pos[cur], (uint32_t)__popcll(bal));
-                b0 = __shfl(b0, leader, 64);
-                if (fb == cur)
-                    out[sub_off[cur] + b0 + (uint32_t)__popcll(bal & lanemask_lt())] =
-                        ((uint64_t)q << 32) | (uint32_t)(gi - qoff[q]);
-            }
+        if (n == nmax) break;
+        const uint64_t w = __shfl_up(v, 1u, 64);
+        const uint32_t ow = __shfl_up(o, 1u, 64);
+        if (r > 0) {
+            const uint64_t sum = v + w;
+            o |= ow | (sum < v ? 1u : 0u);
+            v = sum;
         }
+    }
+}
+
+// block 0: where each slice's tasks go; block 1: the binomial table, for
+// every task size of the launch
+__global__ __launch_bounds__(64) void k_bin_offsets(BinArgs b)
+{
+    if (blockIdx.x == 1) {
+        if (b.binom) binom_rows(b, min(b.brows - 1, b.bin_max[15] + 1));
+        return;
+    }
+    uint32_t carry = 0;
+    for (int base = 0; base < NSLICE; base += 64) {
+        const uint32_t c = b.sub_cnt[base + lane_id()], inc = wave_incl_scan32(c);
+        b.sub_off[base + lane_id()] = carry + inc - c;
+        carry += __shfl(inc, 63, 64);
+    }
+}
+
+// One tile a block.  With ONE the launch has a single slice (every task of at
+// most 64 vertices, one algorithm): no counting pass is needed, its tasks
+// start at 0 and sub_pos ends as their number; the block after the last tile
+// makes the binomial table.
+template <bool ONE, int I>
+__global__ __launch_bounds__(BIN_T) void k_bin_scatter(BinArgs b)
+{
+    __shared__ uint32_t cnt[NSLICE], at[NSLICE];
+    const uint64_t base = (uint64_t)blockIdx.x * BIN_T * I;
+    if (ONE && base >= b.total) {
+        if (b.binom && threadIdx.x < 64) binom_rows(b, b.brows - 1);
+        return;
+    }
+    for (int i = threadIdx.x; i < NSLICE; i += BIN_T) cnt[i] = 0;
+    __syncthreads();
+    BinCursor c(b, base);
+    int fb[I];
+    uint32_t rank[I], s[I];
+    tile_sizes(b, c, base + threadIdx.x, s);
+    {
+        BinCursor cc = c;
+#pragma unroll
+        for (int i = 0; i < I; ++i) {
+            const uint64_t gi = base + (uint64_t)i * BIN_T + threadIdx.x;
+            fb[i] = -1;
+            if (gi >= b.total) continue;
+            cc.seek(b, gi);
+            fb[i] = bin_of(b, cc, gi, s[i]);
+            if (fb[i] >= 0) rank[i] = atomicAdd(&cnt[fb[i]], 1u);
+        }
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < NSLICE; i += BIN_T)
+        if (cnt[i]) at[i] = (ONE ? 0u : b.sub_off[i]) + atomicAdd(&b.sub_pos[ONE ? 0 : i], cnt[i]);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+        if (fb[i] < 0) continue;
+        const uint64_t gi = base + (uint64_t)i * BIN_T + threadIdx.x;
+        c.seek(b, gi);
+        b.out[at[fb[i]] + rank[i]] = ((uint64_t)c.q << 32) | (uint32_t)(gi - c.begin);
     }
 }
 
@@ -2417,14 +2572,22 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     // sub_cnt[NS] bin_max[16] sub_pos[NS] sub_off[NS] qhead[NB][NQUEUE]
     const size_t meta_u32 = 3 * NS + 16 + NB * NQUEUE * QSTRIDE;
     const size_t acc_bytes = sizeof(uint64_t) * NB * NSTRIPE * ACC;
-    // the sums of one query take every wave's flush: they are kept in copies
-    // like the accumulators; many queries spread over their own words
-    const uint32_t q_copies = nq == 1 ? NSTRIPE : 1;
-    const size_t q_words = q_copies > 1 ? (size_t)nq * q_copies * 8 : nq;
-    const size_t q_bytes = sizeof(uint64_t) * q_words + sizeof(uint32_t) * nq;
+    // per query: two sums, then a flag (the sums of a single query are in the accumulators)
+    const size_t q_bytes = sizeof(uint64_t) * 2 * nq + sizeof(uint32_t) * nq;
+    bool any_pivot = false, any_edge = false, one_algo = true;
+    uint32_t max_out = 0;  // bounds every task's size
+    for (uint32_t i = 0; i < nq; ++i) {
+        any_pivot |= halgo[i] != 0;
+        any_edge |= hq[i].gran == KC_GRAN_EDGE;
+        one_algo &= halgo[i] == halgo[0];
+        max_out = std::max(max_out, qs[i].o->max_out);
+    }
+    const uint32_t bstride = kmax + 1, brows = max_out + 2;
+    const size_t nbin = (size_t)brows * bstride;
     if ((rc = scr.qdesc.ensure(qd_bytes + off_bytes + nq + 16)) ||
         (rc = scr.meta.ensure(meta_u32 * 4 + acc_bytes + q_bytes + 16)) ||
-        (rc = scr.size.ensure(sizeof(uint32_t) * (total + 1))))
+        (rc = scr.tasks.ensure(sizeof(uint64_t) * (total + 1))) || (any_pivot && (rc = scr.binom.ensure(nbin * 9 + 16))) ||
+        (any_edge && (rc = scr.size.ensure(sizeof(uint32_t) * (total + 1)))))
         return rc;
     QDesc *dq = scr.qdesc.as<QDesc>();
     uint64_t *doff = reinterpret_cast<uint64_t *>(scr.qdesc.as<uint8_t>() + qd_bytes);
@@ -2433,10 +2596,13 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     uint32_t *sub_cnt = m32, *bin_max = m32 + NS, *sub_pos = bin_max + 16, *sub_off = sub_pos + NS, *qhead = sub_off + NS;
     uint64_t *dacc = reinterpret_cast<uint64_t *>(m32 + meta_u32);
     uint64_t *qcount = dacc + NB * NSTRIPE * ACC;
-    uint32_t *qovf = reinterpret_cast<uint32_t *>(qcount + q_words);
-    KC_HIP(hipMemcpyAsync(dq, hq.data(), qd_bytes, hipMemcpyHostToDevice, s));
-    KC_HIP(hipMemcpyAsync(doff, hoff.data(), off_bytes, hipMemcpyHostToDevice, s));
-    KC_HIP(hipMemcpyAsync(dalgo, halgo.data(), nq, hipMemcpyHostToDevice, s));
+    uint32_t *qovf = reinterpret_cast<uint32_t *>(qcount + 2 * (size_t)nq);
+    // descriptors, task offsets and algorithms side by side: one copy
+    std::vector<uint8_t> up(qd_bytes + off_bytes + nq);
+    std::memcpy(up.data(), hq.data(), qd_bytes);
+    std::memcpy(up.data() + qd_bytes, hoff.data(), off_bytes);
+    std::memcpy(up.data() + qd_bytes + off_bytes, halgo.data(), nq);
+    KC_HIP(hipMemcpyAsync(dq, up.data(), up.size(), hipMemcpyHostToDevice, s));
     {  // counters, queue heads and per-query sums start at zero (a fill kernel, no memset node)
         const uint64_t nz = (meta_u32 * 4 + acc_bytes + q_bytes) / 4;
         hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)std::min<uint64_t>(1024, (nz + 255) / 256)), dim3(256), 0, s,
@@ -2455,58 +2621,61 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     if (!scr.fixed && (rc = evs.create())) return rc;
     evs.record(evs.start, s);
     const int gs = (int)std::max<uint64_t>(1, std::min<uint64_t>((total + 255) / 256, (uint64_t)ctx->cu * 16));
-    // task sizes of a single query on the graph they were last computed for are reused
-    const bool sizes_cached = nq == 1 && scr.size_uid == qs[0].o->uid && scr.size_gran == qs[0].q.gran &&
-                              scr.size_total == total;
+    // edge task sizes of a single query on the graph they were last computed for are reused
+    const bool sizes_cached = nq == 1 && any_edge && scr.size_uid == qs[0].o->uid && scr.size_total == total;
     scr.size_uid = 0;
+    // Every task of at most 64 vertices and one algorithm: a single bin, filled
+    // by one pass, and the launch reads its number of tasks on the device, so
+    // that the host waits for the device once, for the result.  Otherwise it
+    // reads the bins' sizes first: they choose the launches.
+    const bool one_bin = one_algo && max_out <= CLASS_ROWS[0] && total < 0xFFFFFFFFull;
+    BinArgs ba{dq, dalgo, doff, nq, pivot_top2, total, any_edge ? scr.size.as<uint32_t>() : nullptr, sub_cnt, bin_max,
+               sub_pos, sub_off, scr.tasks.as<uint64_t>(), any_pivot ? scr.binom.as<uint64_t>() : nullptr, brows, bstride};
     if (total > 0) {
-        if (!sizes_cached)
+        if (any_edge && !sizes_cached)
             hipLaunchKernelGGL(k_task_size, dim3(gs), dim3(256), 0, s, dq, doff, nq, total, scr.size.as<uint32_t>());
-        hipLaunchKernelGGL(k_classify, dim3(gs), dim3(256), 0, s, dq, dalgo, doff, nq, total, scr.size.as<uint32_t>(),
-                           sub_cnt, bin_max, sub_pos, sub_off, scr.tasks.as<uint64_t>(), 0, pivot_top2);
-    }
-    KC_HIP(hipGetLastError());
-    scr.size_uid = nq == 1 ? qs[0].o->uid : 0;
-    scr.size_gran = qs[0].q.gran;
-    scr.size_total = total;
-    uint32_t h[NS + 16];
-    KC_HIP(hipMemcpyAsync(h, m32, sizeof h, hipMemcpyDeviceToHost, s));
-    KC_HIP(hipStreamSynchronize(s));
-    uint32_t bcnt[NB], bmax[NB], boff[NB], soff[NS];
-    uint64_t tot = 0;
-    uint32_t maxsize = 0;
-    for (int b = 0; b < NB; ++b) {
-        boff[b] = (uint32_t)tot;
-        bcnt[b] = 0;
-        for (int sl = 0; sl < NSUB; ++sl) {
-            soff[b * NSUB + sl] = (uint32_t)tot;
-            bcnt[b] += h[b * NSUB + sl];
-            tot += h[b * NSUB + sl];
+        const bool few = total < (uint64_t)BIN_T * BIN_I * ctx->cu;  // (less than a full tile per CU)
+        const int per = BIN_T * (few ? BIN_I_FEW : BIN_I);
+        const unsigned tiles = (unsigned)((total + per - 1) / per);
+        void *args[] = {&ba};
+        auto go = [&](const void *kern, unsigned blocks, unsigned threads) {
+            return hipLaunchKernel(kern, dim3(blocks), dim3(threads), args, 0, s);
+        };
+        if (one_bin) {
+            KC_HIP(go(few ? (const void *)&k_bin_scatter<true, BIN_I_FEW> : (const void *)&k_bin_scatter<true, BIN_I>,
+                      tiles + 1, BIN_T));
+        } else {
+            KC_HIP(go(few ? (const void *)&k_bin_count<BIN_I_FEW> : (const void *)&k_bin_count<BIN_I>,
+                      std::min<unsigned>(tiles, (unsigned)ctx->cu * 4), BIN_T));
+            KC_HIP(go((const void *)&k_bin_offsets, 2, 64));
+            KC_HIP(go(few ? (const void *)&k_bin_scatter<false, BIN_I_FEW> : (const void *)&k_bin_scatter<false, BIN_I>,
+                      tiles, BIN_T));
         }
-        bmax[b] = h[NS + b];  // (kept for the unbounded classes only)
     }
-    maxsize = h[NS + 15];
-    if (tot >= 0xFFFFFFFFull) return fail(KC_ERR_LIMIT, "more than 2^32 tasks in one launch");
-    if ((rc = scr.tasks.ensure(sizeof(uint64_t) * ((size_t)tot + 1)))) return rc;
-    KC_HIP(hipMemcpyAsync(sub_off, soff, sizeof soff, hipMemcpyHostToDevice, s));
-    if (tot > 0)
-        hipLaunchKernelGGL(k_classify, dim3(gs), dim3(256), 0, s, dq, dalgo, doff, nq, total, scr.size.as<uint32_t>(),
-                           sub_cnt, bin_max, sub_pos, sub_off, scr.tasks.as<uint64_t>(), 1, pivot_top2);
     KC_HIP(hipGetLastError());
-    evs.record(evs.cls, s);
-
-    // --- binomial table for the pivot leaves ---
-    const uint32_t bstride = kmax + 1;
-    const size_t nbin = (size_t)(maxsize + 2) * bstride;
-    {
-        std::vector<uint64_t> bv;
-        std::vector<uint8_t> bo;
-        binom_table(maxsize + 1, kmax, bv, bo);
-        if ((rc = scr.binom.ensure(nbin * 9 + 16))) return rc;
-        KC_HIP(hipMemcpyAsync(scr.binom.p, bv.data(), nbin * 8, hipMemcpyHostToDevice, s));
-        KC_HIP(hipMemcpyAsync(scr.binom.as<uint8_t>() + nbin * 8, bo.data(), nbin, hipMemcpyHostToDevice, s));
-        KC_HIP(hipStreamSynchronize(s));  // the host vectors go out of scope
+    if (nq == 1 && any_edge) {
+        scr.size_uid = qs[0].o->uid;
+        scr.size_total = total;
     }
+    uint32_t bcnt[NB] = {0}, bmax[NB] = {0}, boff[NB] = {0};
+    if (one_bin) {
+        bcnt[halgo[0] ? NCLASS : 0] = (uint32_t)total;  // (at most)
+    } else {
+        uint32_t h[NS + 16] = {0};
+        KC_HIP(hipMemcpyAsync(h, m32, sizeof h, hipMemcpyDeviceToHost, s));
+        KC_HIP(hipStreamSynchronize(s));
+        uint64_t tot = 0;
+        for (int b = 0; b < NB; ++b) {
+            boff[b] = (uint32_t)tot;
+            for (int sl = 0; sl < NSUB; ++sl) {
+                bcnt[b] += h[b * NSUB + sl];
+                tot += h[b * NSUB + sl];
+            }
+            bmax[b] = h[NS + b];  // (kept for the unbounded classes only)
+        }
+        if (tot >= 0xFFFFFFFFull) return fail(KC_ERR_LIMIT, "more than 2^32 tasks in one launch");
+    }
+    evs.record(evs.cls, s);
 
     // --- one persistent launch per non-empty bin, largest tasks first ---
     // The bins of tasks of at most 256 vertices can run side by side on the
@@ -2566,6 +2735,7 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         a.qd = dq;
         a.tasks = scr.tasks.as<uint64_t>() + boff[b];
         a.ntasks = bcnt[b];
+        a.ntasks_p = one_bin ? sub_pos : nullptr;
         a.binom = scr.binom.as<uint64_t>();
         a.binom_ovf = scr.binom.as<uint8_t>() + nbin * 8;
         a.bstride = bstride;
@@ -2573,7 +2743,7 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         a.acc = dacc + (size_t)b * NSTRIPE * ACC;
         a.acc_mask = NSTRIPE - 1;
         a.qcount = qcount;
-        a.q_mask = q_copies - 1;
+        a.single = nq == 1;
         a.qovf = qovf;
         a.local = local;
         const bool lc = local != nullptr;
@@ -2636,8 +2806,14 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         KC_HIP_L(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, (int)(64 * nw), lds));
         if (per_cu < 1) per_cu = 1;
         uint64_t blocks = std::max<uint64_t>(1, (uint64_t)per_cu * ctx->cu / std::max<uint32_t>(1, grid_share));
+        // one block per task while the tasks are few, else the persistent grid
+        // and its queues (a server worker's share of the device is a grid size,
+        // an HBM slice belongs to a block: those stay persistent)
+        constexpr uint64_t DIRECT_ROUNDS = 4;
+        a.direct = grid_share <= 1 && !global && bcnt[b] <= blocks * DIRECT_ROUNDS;
         a.chunk_log = (c == 0 && bcnt[b] > blocks * 64) ? 2 : 0;  // (the wide kernel takes one task per grab)
-        blocks = std::min<uint64_t>(blocks, ((uint64_t)bcnt[b] + (1u << a.chunk_log) - 1) >> a.chunk_log);
+        const uint64_t chunks = ((uint64_t)bcnt[b] + (1u << a.chunk_log) - 1) >> a.chunk_log;
+        blocks = a.direct ? chunks : std::min<uint64_t>(blocks, chunks);
         if (global) {
             a.gscr_words = L.total;
             // a fixed scratch holds as many slices as fit in what it has left
@@ -2691,8 +2867,10 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
                 uint64_t &h = hacc[b * ACC + i];
                 h = i == 4 ? std::max(h, v) : h + v;  // [4] is the longest task
             }
+    for (int b = 0; b < NB; ++b)
+        if (one_bin && hacc[ACC * b + 2] == 0) launched[b] = false;  // the bin was empty
     const uint64_t *hq_sum = back.data() + NB * NSTRIPE * ACC;
-    const uint32_t *hq_flag = reinterpret_cast<const uint32_t *>(hq_sum + q_words);
+    const uint32_t *hq_flag = reinterpret_cast<const uint32_t *>(hq_sum + 2 * (size_t)nq);
     float bin_ms[NB] = {0};
     const float prep_ms = evs.ms(evs.start, evs.cls), total_ms = evs.ms(evs.go, evs.end);
     for (int b = 0; b < NB; ++b)
@@ -2704,11 +2882,13 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     for (uint32_t i = 0; i < nq; ++i) {
         kc_result &r = res[i];
         r.overflow = hq_flag[i] ? 1 : 0;
-        for (uint32_t c = 0; c < q_copies; ++c) {
-            const uint64_t v = hq_sum[q_copies > 1 ? ((size_t)i * q_copies + c) * 8 : i];
-            r.count += v;
-            if (r.count < v) r.overflow = 1;
-        }
+        unsigned __int128 sum = 0;
+        if (nq == 1)
+            for (int b = 0; b < NB; ++b) sum += hacc[ACC * b] + ((unsigned __int128)hacc[ACC * b + 6] << 32);
+        else
+            sum = hq_sum[2 * i] + ((unsigned __int128)hq_sum[2 * i + 1] << 32);
+        r.count = (uint64_t)sum;
+        if (sum >> 64) r.overflow = 1;
         r.algo = qs[i].q.algo;
         r.gran = qs[i].q.gran;
         r.part_size = qs[i].q.part_size;

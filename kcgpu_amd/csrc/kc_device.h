@@ -65,12 +65,11 @@ int scan_exclusive_u32(const uint32_t *in, uint32_t *out, uint32_t n, DevBuf &tm
 struct Scratch {
     DevBuf tasks, meta, binom, gscr, size, qdesc, local;
     bool fixed = false;
-    // what `size` holds when it was filled for one query: the oriented graph
-    // (its uid), the granularity and the task count; task sizes (d+(u), or
-    // |N+(u) & N+(v)|) do not depend on k, so the next query on that graph
-    // reuses them
+    // what `size` holds when it was filled for one query of edge tasks: the
+    // oriented graph (its uid) and the task count; an edge task's size
+    // |N+(u) & N+(v)| does not depend on k, so the next query on that graph
+    // reuses it
     uint64_t size_uid = 0;
-    uint32_t size_gran = 0;
     uint64_t size_total = 0;
 };
 
