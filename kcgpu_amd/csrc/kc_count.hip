@@ -139,6 +139,16 @@ __host__ __device__ inline Layout make_layout(uint32_t rmax, uint32_t wmax, uint
 // ---- wave helpers ------------------------------------------------------------
 __device__ inline int lane_id() { return threadIdx.x & 63; }
 
+// A value every lane holds alike, moved to scalar registers: the compiler then
+// treats what is derived from it as uniform (scalar ALU, scalar branches)
+// instead of masking the wave lane by lane.
+__device__ inline uint32_t uni32(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+
+__device__ inline uint64_t uni64(uint64_t v)
+{
+    return ((uint64_t)uni32((uint32_t)(v >> 32)) << 32) | uni32((uint32_t)v);
+}
+
 __device__ inline uint64_t lanemask_lt()
 {
     int l = lane_id();
@@ -366,24 +376,6 @@ __device__ uint64_t orient_count(const CountArgs &a, uint32_t P, const uint64_t 
     return cnt;
 }
 
-// per-lane gather: lane l gets v of lane src(l)
-__device__ inline uint64_t bperm64(uint64_t v, uint32_t src)
-{
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(src << 2), (int)(uint32_t)v);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(src << 2), (int)(uint32_t)(v >> 32));
-    return ((uint64_t)hi << 32) | lo;
-}
-
-// A value every lane holds alike, moved to scalar registers: the compiler then
-// treats what is derived from it as uniform (scalar ALU, scalar branches)
-// instead of masking the wave lane by lane.
-__device__ inline uint32_t uni32(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
-
-__device__ inline uint64_t uni64(uint64_t v)
-{
-    return ((uint64_t)uni32((uint32_t)(v >> 32)) << 32) | uni32((uint32_t)v);
-}
-
 __device__ inline uint64_t rdlane64(uint64_t v, uint32_t src)
 {
     uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, (int)src);
@@ -391,47 +383,7 @@ __device__ inline uint64_t rdlane64(uint64_t v, uint32_t src)
     return ((uint64_t)hi << 32) | lo;
 }
 
-// ---- closed forms over a one-word candidate set X (row = the lane's row) ----
-// All of them run with every lane active: rows of other lanes come in with
-// ds_bpermute, and loops run while any lane still has work (ballot).
-
-// triangles of G[X] through the complement (Goodman):
-//   t(G) = C(|X|,3) - 1/2 sum_x d_x (|X|-1-d_x) - t(complement),
-// each lane walking its complement neighbours above it (cmpl, at most cmax)
-__device__ inline uint32_t tri_complement(uint64_t row, uint64_t cmpl, uint32_t cmax, bool mem, uint32_t v, uint32_t cx)
-{
-    uint32_t gd = mem ? v * (cx - 1 - v) : 0u, tb = 0;
-    uint64_t rest = cmpl;
-    for (uint32_t it = 0; it < cmax; ++it) {
-        const uint32_t y = rest ? (uint32_t)__builtin_ctzll(rest) : 0u;
-        const uint64_t ry = bperm64(row, y);
-        if (rest) {
-            const uint64_t ay = y == 63 ? 0ull : (~0ull << (y + 1));
-            tb += (uint32_t)__popcll(cmpl & ~ry & ay);
-            rest &= rest - 1;
-        }
-    }
-    gd = (uint32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_add_u32(gd));
-    tb = (uint32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_add_u32(tb));
-    return cx * (cx - 1) * (cx - 2) / 6 - gd / 2 - tb;
-}
-
-// triangles of G[X], each i < j < l counted at i over a uniform walk of X
-__device__ inline uint32_t tri_direct(uint64_t X, uint64_t row, uint64_t lane_above)
-{
-    const uint32_t lane = (uint32_t)lane_id();
-    uint32_t tri = 0;
-    const uint64_t mine = X & row & lane_above;
-    for (uint64_t bits = X; bits; bits &= bits - 1) {
-        const uint32_t il = (uint32_t)__builtin_ctzll(bits);
-        const uint64_t above = il == 63 ? 0ull : (~0ull << (il + 1));
-        const uint64_t Y = X & rdlane64(row, il) & above;
-        if ((Y >> lane) & 1ull) tri += (uint32_t)__popcll(Y & mine);
-    }
-    return (uint32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_add_u32(tri));
-}
-
-
+// ---- closed forms over one- and two-word candidate sets ----------------------
 // |E|, triangles and 4-cliques of G[X] from its complement H (the non-edges
 // inside X), by inclusion-exclusion over the edge sets F of H that span at
 // most four vertices, sum_F (-1)^|F| C(n - |V(F)|, 4 - |V(F)|):
@@ -443,102 +395,198 @@ __device__ inline uint32_t tri_direct(uint64_t X, uint64_t row, uint64_t lane_ab
 // neighbours), paw = sum_x t_x (d_x-2) triangles with a pendant edge, dia =
 // sum_{xy in E} C(c_xy,2) four-cycles with a chord, K4 four-cliques; and
 // Goodman's c3 = C(n,3) - 1/2 sum_x d_x (n-1-d_x) - K3.
-// Lane x holds its complement row Hx.  One uniform walk over u in X (row u by
-// v_readlane) hands c_ux = |Hu & Hx| to every lane, which keeps
-//   q  = sum_u c_ux^2,   qE = sum_{u in Hx} c_ux^2,   t2 = sum_{u in Hx} c_ux = 2 t_x,
-//   sd = sum_{u in Hx} d_u  (= sum_u c_ux),
-// so that, summed over lanes, 8 C4 = sum (q - d^2) - (sd - d), 2 P4 + 6 K3 =
-// sum (d-1)(sd-d), 4 dia = sum qE - t2.  The lane shares are summed scaled by
-// 24 so each is an integer.  A K4 of H has every vertex in at least three
-// H-triangles, so the K4 walk (over the H-edges u < v, counting the H-edges
-// inside Hu & Hv above v) only visits such vertices and is empty in most
-// near-cliques.
+// With, per vertex x,
+//   q = sum_u c_ux^2,  qE = sum_{u in Hx} c_ux^2,  t2 = sum_{u in Hx} c_ux = 2 t_x,
+//   sd = sum_u c_ux = sum_{u in Hx} d_u
+// (8 C4 = sum (q - d^2) - (sd - d), 2 P4 + 6 K3 = sum (d-1)(sd-d), 4 dia = sum
+// qE - t2) the terms beyond the counts of edges come to
+//   24 c4 = n(n-1)(n-2)(n-3) - 12 m (n-2)(n-3) + 12 m (m-1) + 24 K4
+//           + sum_x t2 (12d - 4n + 6) - sd (12d - 9) + 3q - 6qE + d(d-1)(12n - 31 - 4d)
+//   6 c3  = n(n-1)(n-2) - sum_x 3d(n-1-d) + t2
+// (all modulo 2^32: 24 c4 <= 128^4 fits).  A K4 of H has every vertex in at
+// least three H-triangles, so the K4 walk (over the H-edges u < v, counting
+// the H-edges inside Hu & Hv above v) only visits such vertices.
+//
+// The c_ux are the matrix H H^T, which the matrix cores make 32 x 32 entries
+// at a time (v_mfma_i32_32x32x32_i8, the bits of H as bytes 0 and 1).  A lane
+// (j, b) = (lane & 31, lane >> 5) gets, of column j, the rows 8g + 4b + i (g, i
+// < 4) in entry 4g + i.  The order of the summed index is free as long as
+// both operands agree, so byte i of operand word g holds bit 8g + 4b + i: the
+// operand words of a column are then also the 0/1 masks of its four entries.
+// Entries are at most 127, so four pack into a word for the dot products.
+// The walk this replaces took ~17 vector instructions per vertex u of X
+// (~45 over two words); here a 32 x 32 block takes 4 x 10 and 8 matrix
+// passes per 32 of the summed index.
 struct CliqueCounts {
     uint32_t e, c3, c4;
 };
 
-__device__ inline CliqueCounts k34_complement(uint64_t X, uint64_t row, bool mem, uint32_t cx)
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+// the lane's bit of a uniform mask
+__device__ inline bool in_mask(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
+__device__ inline uint32_t wave_sum32(uint32_t x)
 {
-    const uint32_t lane = (uint32_t)lane_id();
-    const uint64_t Hl = mem ? (X & ~row & ~(1ull << lane)) : 0ull;
-    const int32_t d = (int32_t)__popcll(Hl), n = (int32_t)cx;
-    uint32_t q = 0, qE = 0, t2 = 0, sd = 0;
-    if ((X >> 32) == 0) {
-        // X within vertices 0..31: lanes l and l+32 both hold vertex l (32-bit
-        // rows) and walk two members u per step, one per half of the wave
-        const uint32_t lo = lane & 31, X32 = (uint32_t)X;
-        const bool upper = lane >= 32;
-        const uint32_t row32 = (uint32_t)__shfl((int)(uint32_t)row, (int)lo, 64);
-        const uint32_t H32 = ((X32 >> lo) & 1u) ? (X32 & ~row32 & ~(1u << lo)) : 0u;
-        for (uint32_t bits = X32; bits;) {
-            const uint32_t ua = (uint32_t)__builtin_ctz(bits);
-            bits &= bits - 1;
-            uint32_t Hb = 0;
-            if (bits) {
-                const uint32_t ub = (uint32_t)__builtin_ctz(bits);
-                bits &= bits - 1;
-                Hb = X32 & ~(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)row, (int)ub) & ~(1u << ub);
-            }
-            const uint32_t Ha = X32 & ~(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)row, (int)ua) & ~(1u << ua);
-            const uint32_t Hu = upper ? Hb : Ha;
-            const uint32_t du = upper ? (uint32_t)__popc(Hb) : (uint32_t)__popc(Ha);
-            const uint32_t c = (uint32_t)__popc(H32 & Hu), c2 = c * c;
-            const uint32_t in = (Hu >> lo) & 1u;  // the lane's vertex is a complement neighbour of u
-            q += c2;
-            qE += in * c2;
-            t2 += in * c;
-            sd += in * du;
-        }
-        q += (uint32_t)__shfl_xor((int)q, 32, 64);
-        qE += (uint32_t)__shfl_xor((int)qE, 32, 64);
-        t2 += (uint32_t)__shfl_xor((int)t2, 32, 64);
-        sd += (uint32_t)__shfl_xor((int)sd, 32, 64);
-        if (upper) q = qE = t2 = sd = 0;  // (Hl, d are 0 there: X has no member above 31)
-    } else {
-        for (uint64_t bits = X; bits; bits &= bits - 1) {
-            const uint32_t u = (uint32_t)__builtin_ctzll(bits);
-            const uint64_t Hu = X & ~rdlane64(row, u) & ~(1ull << u);
-            const uint32_t du = (uint32_t)__popcll(Hu);
-            const uint32_t c = (uint32_t)__popcll(Hl & Hu), c2 = c * c;
-            const uint32_t in = (uint32_t)(Hu >> lane) & 1u;
-            q += c2;
-            qE += in * c2;
-            t2 += in * c;
-            sd += in * du;
-        }
-    }
-    const int32_t t = (int32_t)(t2 / 2);  // H-triangles through the lane's vertex
-    // K4 of H among the vertices in >= 3 H-triangles
-    int32_t k4acc = 0;
-    const uint64_t T3 = __ballot(t >= 3);
-    if (__popcll(T3) >= 4) {
-        const uint64_t lane_above = lane == 63 ? 0ull : (~0ull << (lane + 1));
-        for (uint64_t ub = T3; ub; ub &= ub - 1) {
-            const uint32_t u = (uint32_t)__builtin_ctzll(ub);
-            const uint64_t Hu = T3 & ~rdlane64(row, u) & (u == 63 ? 0ull : (~0ull << (u + 1)));
-            for (uint64_t vb = Hu; vb; vb &= vb - 1) {
-                const uint32_t v = (uint32_t)__builtin_ctzll(vb);
-                const uint64_t S = Hu & ~rdlane64(row, v) & (v == 63 ? 0ull : (~0ull << (v + 1)));
-                if (__popcll(S) >= 2 && ((S >> lane) & 1ull)) k4acc += (int32_t)__popcll(S & Hl & lane_above);
-            }
-        }
-    }
-    const int32_t iq = (int32_t)q, iqE = (int32_t)qE, isd = (int32_t)sd, it2 = (int32_t)t2;
-    const int32_t c4l = 12 * (n - 4) * d * (d - 1) - 8 * (n - 3) * t - 12 * (d - 1) * (isd - d) + 24 * t -
-                        4 * d * (d - 1) * (d - 2) + 3 * ((iq - d * d) - (isd - d)) + 24 * t * (d - 2) -
-                        6 * (iqE - it2) + 24 * k4acc;
-    const int32_t c3l = -3 * d * (n - 1 - d) - 2 * t;
-    const int32_t s_d = (int32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_add_u32((uint32_t)d));
-    const int32_t s_4 = (int32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_add_u32((uint32_t)c4l));
-    const int32_t s_3 = (int32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_add_u32((uint32_t)c3l));
-    const int32_t m = s_d / 2;
-    const int32_t c4_24 = n * (n - 1) * (n - 2) * (n - 3) - 12 * m * (n - 2) * (n - 3) + 12 * m * (m - 1) + s_4;
-    const int32_t c3_6 = n * (n - 1) * (n - 2) + s_3;
-    CliqueCounts r;
-    r.e = (uint32_t)(n * (n - 1) / 2 - m);
-    r.c3 = (uint32_t)(c3_6 / 6);
-    r.c4 = (uint32_t)(c4_24 / 24);
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_add_u32(x));
+}
+
+// lower lanes' values (both halves), upper lanes' values (both halves)
+__device__ inline void halves(uint32_t x, uint32_t &lo, uint32_t &hi)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    lo = r[0];
+    hi = r[1];
+}
+
+// operand words of 32 bits of a row: byte i of word g = bit 8g + 4b + i
+__device__ inline v4i spread_bits(uint32_t x)
+{
+    const uint32_t y = x >> ((lane_id() >> 5) * 4);
+    v4i r;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) r[g] = (int)(__umul24((y >> (8 * g)) & 15u, 0x204081u) & 0x01010101u);
     return r;
+}
+
+// The lane's share of the sums above over blocks of 32 vertices: H[I][K] is
+// word K of the complement row of vertex 32 I + (lane & 31) (zero outside X).
+// s4 += the sum's terms of 24 c4, s3 += those of 6 c3, sd += degrees; T3[J] =
+// the block's vertices in three or more triangles of H.  live: blocks with a
+// member (the others are branched over, which also keeps the blocks' entries
+// from being in registers together).
+template <int NB>
+__device__ inline void complement_sums(const uint32_t (&H)[NB][NB], uint32_t live, uint32_t n, uint32_t &s4, uint32_t &s3,
+                                       uint32_t &sd, uint32_t (&T3)[NB])
+{
+    const bool once = lane_id() < 32;
+    v4i E[NB][NB];
+#pragma unroll
+    for (int I = 0; I < NB; ++I)
+#pragma unroll
+        for (int K = 0; K < NB; ++K) E[I][K] = spread_bits(H[I][K]);
+#pragma unroll
+    for (int J = 0; J < NB; ++J) {
+        T3[J] = 0;
+        if (NB > 1 && !((live >> J) & 1u)) continue;
+        uint32_t d = 0, q = 0, qE = 0, t2 = 0, sm = 0;
+#pragma unroll
+        for (int K = 0; K < NB; ++K) d += (uint32_t)__popc(H[J][K]);
+#pragma unroll
+        for (int I = 0; I < NB; ++I) {
+            if (NB > 1 && !((live >> I) & 1u)) continue;
+            v16i c = {0};
+#pragma unroll
+            for (int K = 0; K < NB; ++K) c = __builtin_amdgcn_mfma_i32_32x32x32_i8(E[I][K], E[J][K], c, 0, 0, 0);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const uint32_t cp = (uint32_t)c[4 * g] | ((uint32_t)c[4 * g + 1] << 8) | ((uint32_t)c[4 * g + 2] << 16) |
+                                    ((uint32_t)c[4 * g + 3] << 24);
+                const uint32_t hb = (uint32_t)E[J][I][g];
+                const uint32_t cm = cp & ((hb << 8) - hb);
+                t2 = __builtin_amdgcn_udot4(cp, hb, t2, false);
+                sm = __builtin_amdgcn_udot4(cp, 0x01010101u, sm, false);
+                q = __builtin_amdgcn_udot4(cp, cp, q, false);
+                qE = __builtin_amdgcn_udot4(cm, cm, qE, false);
+            }
+        }
+        s3 += t2 + (once ? 3u * d * (n - 1 - d) : 0u);
+        sd += once ? d : 0u;
+        s4 += t2 * (12 * d - 4 * n + 6) - sm * (12 * d - 9) + 3 * q - 6 * qE +
+              (once ? d * (d - 1) * (12 * n - 31 - 4 * d) : 0u);
+        uint32_t lo, hi;
+        halves(t2, lo, hi);
+        T3[J] = (uint32_t)__ballot(lo + hi >= 6);
+    }
+}
+
+// the counts from the wave's sums
+__device__ inline CliqueCounts complement_counts(uint32_t n, uint32_t m, uint32_t s3, uint32_t s4)
+{
+    CliqueCounts r;
+    r.e = n * (n - 1) / 2 - m;
+    r.c3 = (n * (n - 1) * (n - 2) - s3) / 6;
+    r.c4 = (n * (n - 1) * (n - 2) * (n - 3) - 12 * m * (n - 2) * (n - 3) + 12 * m * (m - 1) + s4) / 24;
+    return r;
+}
+
+// One-word sets.  U = uint64_t: lane l holds vertex l.  U = uint32_t: lanes l
+// and l + 32 both hold vertex l.  mask64: the lanes of a set's members.
+__device__ inline uint64_t mask64(uint64_t X) { return X; }
+__device__ inline uint64_t mask64(uint32_t X) { return ((uint64_t)X << 32) | X; }
+__device__ inline uint32_t bits_of(uint64_t x) { return (uint32_t)__popcll(x); }
+__device__ inline uint32_t bits_of(uint32_t x) { return (uint32_t)__popc(x); }
+__device__ inline uint32_t low_bit(uint64_t x) { return (uint32_t)__builtin_ctzll(x); }
+__device__ inline uint32_t low_bit(uint32_t x) { return (uint32_t)__builtin_ctz(x); }
+__device__ inline uint64_t rdlane(uint64_t v, uint32_t src) { return rdlane64(v, src); }
+__device__ inline uint32_t rdlane(uint32_t v, uint32_t src)
+{
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)src);
+}
+// bits above b (b < bits of U)
+template <class U>
+__device__ inline U above(uint32_t b)
+{
+    return (~(U)0 << b) << 1;
+}
+
+// c2, c3 and (with_c4) c4 of G[X], n = |X| >= 1 (row: the lane's vertex's row)
+// MM: 64-vertex sets go through the matrix cores too (48 more registers)
+template <bool MM, class U>
+__device__ __attribute__((always_inline)) CliqueCounts close_word(U X, U row, uint32_t n, bool with_c4)
+{
+    constexpr int BITS = 8 * sizeof(U);
+    const uint32_t v = (uint32_t)lane_id() & (BITS - 1);
+    const U Hl = in_mask(mask64(X)) ? (U)(X & ~row & ~((U)1 << v)) : (U)0;
+    if (__ballot(Hl != 0) == 0) return complement_counts(n, 0, 0, 0);  // X is a clique
+    uint32_t s4 = 0, s3 = 0, sd = 0;
+    U T3 = 0;
+    if constexpr (BITS == 32) {
+        uint32_t H[1][1], t3[1];
+        H[0][0] = Hl;
+        complement_sums<1>(H, 1, n, s4, s3, sd, t3);
+        T3 = t3[0];
+    } else if constexpr (MM) {
+        uint32_t H[2][2], t3[2];
+        halves((uint32_t)Hl, H[0][0], H[1][0]);
+        halves((uint32_t)(Hl >> 32), H[0][1], H[1][1]);
+        complement_sums<2>(H, ((uint32_t)X ? 1u : 0u) | ((uint32_t)(X >> 32) ? 2u : 0u), n, s4, s3, sd, t3);
+        T3 = ((uint64_t)t3[1] << 32) | t3[0];
+    } else {
+        // a uniform walk over u in X hands c_ux = |Hu & Hx| to every lane x
+        const uint32_t d = bits_of(Hl);
+        uint32_t q = 0, qE = 0, t2 = 0, sm = 0;
+        for (U b = X; b; b &= b - 1) {
+            const U Hu = rdlane(Hl, low_bit(b));
+            const uint32_t c = bits_of((U)(Hl & Hu)), cm = in_mask(Hu) ? c : 0u;
+            sm += c;
+            t2 += cm;
+            q += __umul24(c, c);
+            qE += __umul24(cm, cm);
+        }
+        s4 = t2 * (12 * d - 4 * n + 6) - sm * (12 * d - 9) + 3 * q - 6 * qE + d * (d - 1) * (12 * n - 31 - 4 * d);
+        s3 = in_mask(X) ? t2 + 3 * d * (n - 1 - d) : 0u;
+        sd = d;
+        T3 = __ballot(t2 >= 6);
+    }
+    if (with_c4 && bits_of(T3) >= 4) {  // K4 of H among the vertices in >= 3 H-triangles
+        uint32_t k4 = 0;
+        for (U ub = T3; ub; ub &= ub - 1) {
+            const uint32_t u = low_bit(ub);
+            const U Hu = T3 & rdlane(Hl, u) & above<U>(u);
+            if (bits_of(Hu) < 3) continue;
+            for (U vb = Hu; vb; vb &= vb - 1) {
+                const uint32_t w = low_bit(vb);
+                const U S = Hu & rdlane(Hl, w) & above<U>(w);
+                if (bits_of(S) >= 2) k4 += in_mask(mask64(S)) ? bits_of((U)(S & Hl & above<U>(v))) : 0u;
+            }
+        }
+        s4 += BITS == 32 ? 12 * k4 : 24 * k4;  // (32 vertices: both halves of the wave counted)
+    }
+    // n <= 64: s3 <= 6 C(64,3) < 2^20 and the degrees sum to less than 2^12
+    const uint32_t sum = wave_sum32(s3 + (sd << 20));
+    return complement_counts(n, (sum >> 20) / 2, sum & 0xFFFFFu, with_c4 ? wave_sum32(s4) : 0u);
 }
 
 __device__ inline uint64_t mul_chk(uint64_t x, uint64_t y, uint32_t &ovf)
@@ -568,111 +616,175 @@ __device__ inline uint64_t close_k3(const CountArgs &a, uint32_t p, uint32_t cx,
     return r;
 }
 
-// SCT of a subproblem of at most 64 vertices held one row per lane: lane i
-// keeps row i (bit j <=> vertex j of the subproblem is adjacent), X0 is the
-// candidate set, h0/p0 the held and pivot counts above it.  Every set is one
-// uniform 64-bit word, a score is one AND + popcount, a branch row is one
-// v_readlane pair, and the stack lives across the lanes (lane t = level t).
-// Nodes with h >= k-3 close in form as in pivot_reg, nodes with h = k-4 by
-// k34_complement.
-__device__ uint64_t sct64(const CountArgs &a, uint32_t k, uint64_t row, uint64_t X0, uint32_t h0, uint32_t p0,
-                          uint64_t &nodes, uint32_t &ovf)
+// The k-cliques of a subtree with `need` vertices to find and no 5-clique
+// wanted inside X: sum_{j <= min(need, 4)} C(p, need-j) c_j(X), c_0 = 1, c_1 = |X|.
+// Lane j adds term j to its own sum (the wave's share of a count is spread
+// over the lanes until the task ends).  The five binomials are one load,
+// issued before the counts are made: term by term they were five dependent
+// trips to memory, which a closing node waited for longer than it computed.
+struct CloseTerm {
+    uint64_t b = 0;
+    uint32_t o = 0;
+    __device__ CloseTerm(const CountArgs &a, uint32_t need, uint32_t p)
+    {
+        const uint32_t j = (uint32_t)lane_id();
+        if (j <= 4 && j <= need) {
+            const uint64_t idx = (uint64_t)p * a.bstride + (need - j);
+            b = a.binom[idx];
+            o = a.binom_ovf[idx];
+        }
+    }
+    __device__ void add(uint64_t &acc, uint32_t &ovf, uint32_t cx, const CliqueCounts &c) const
+    {
+        const uint32_t j = (uint32_t)lane_id();
+        const uint32_t m = j == 0 ? 1u : j == 1 ? cx : j == 2 ? c.e : j == 3 ? c.c3 : j == 4 ? c.c4 : 0u;
+        const uint64_t lo = (b & 0xFFFFFFFFull) * m, hi = (b >> 32) * m + (lo >> 32);
+        if (m && (o || (hi >> 32))) ovf = 1;
+        add_checked(acc, (hi << 32) | (lo & 0xFFFFFFFFull), ovf);
+    }
+};
+
+// the wave's total of per-lane shares, in every lane; ovf (uniform) with it
+__device__ inline uint64_t wave_total(uint64_t x, uint32_t lane_ovf, uint32_t &ovf)
 {
-    const uint32_t lane = (uint32_t)lane_id();
-    const uint64_t lane_above = lane == 63 ? 0ull : (~0ull << (lane + 1));
+    const uint64_t t = uni64(wave_sum64_checked(x, lane_ovf));
+    if (__ballot(lane_ovf != 0)) ovf = 1;
+    return t;
+}
+
+// SCT of a subproblem of at most 64 (U = uint64_t) or 32 (uint32_t) vertices
+// held one row per lane: X0 is the candidate set, h0/p0 the held and pivot
+// counts above it.  Every set is one uniform word, a score is one AND +
+// popcount.  The open level is in scalar registers (tC candidates, tB branches
+// left, the pivot, h, p); levels below it are put away across the lanes (lane
+// i = level i) when a node opens a new level over one that has branches left,
+// so the chain of pivot branches moves nothing.
+// Returns the lanes' shares of the count.  A node closes in form at h >= k-4
+// (close_word), and, at any h, once at most four candidates are left, which cannot hold a 5-clique.  Candidates
+// adjacent to all others lie in every maximal clique of X: they become pivots
+// together instead of one node each.  A 64-vertex subtree whose candidates
+// are at most 32 is re-encoded as a 32-vertex one.
+template <bool MM, class U>
+__device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32_t h0, uint32_t p0, uint64_t &nodes,
+                             uint32_t &ovf)
+{
+    constexpr uint32_t BITS = 8 * sizeof(U);
+    const uint32_t lane = (uint32_t)lane_id(), v = lane & (BITS - 1);
     k = uni32(k);
-    uint64_t X = uni64(X0), stkC = 0, stkB = 0;
-    uint32_t stkM = 0;
+    U X = BITS == 64 ? (U)uni64(X0) : (U)uni32((uint32_t)X0);
+    U tC = 0, tB = 0, stkC = 0, stkB = 0;
+    uint32_t tM = 0, stkM = 0;  // h | p << 8 | pivot << 20
+    bool open = false;
     int t = -1;
-    bool pending = true;
     uint32_t h = uni32(h0), p = uni32(p0);
     uint64_t acc = 0, my_nodes = 0;
     for (;;) {
-        if (pending) {
-            pending = false;
-            ++my_nodes;
-            const uint32_t cx = (uint32_t)__popcll(X);
-            if (cx == 0) {
-                if (k >= h && k - h <= p) {
-                    const uint64_t idx = (uint64_t)p * a.bstride + (k - h);
-                    if (a.binom_ovf[idx]) ovf = 1;
-                    add_checked(acc, a.binom[idx], ovf);
-                }
-            } else if (h >= k) {
-                add_checked(acc, 1, ovf);
-            } else if (h + 1 == k) {
-                add_checked(acc, (uint64_t)p + cx, ovf);
-            } else if (h + p + cx >= k) {
-                const bool mem = (X >> lane) & 1ull;
-                const uint32_t v = mem ? (uint32_t)__popcll(X & row) : 0u;
-                if (h + 3 >= k) {
-                    const uint32_t e2 = (uint32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_add_u32(v));
-                    const uint64_t pp = p;
-                    if (h + 2 == k) {
-                        add_checked(acc, pp * (pp - (pp ? 1 : 0)) / 2, ovf);
-                        add_checked(acc, pp * cx, ovf);
-                        add_checked(acc, e2 / 2, ovf);
+        ++my_nodes;
+        uint32_t cx = bits_of(X);
+        const uint32_t need = k - h;  // (h <= k)
+        if (p + cx >= need) {
+            if (BITS == 64 && cx <= 32 && need >= 3 && cx > 0 && (!MM || need >= 5 || (uint32_t)((uint64_t)X >> 32) == 0)) {
+                if constexpr (BITS == 64) {
+                    uint32_t row1 = 0, X1 = (uint32_t)X;
+                    if ((X >> 32) == 0) {
+                        uint32_t up;
+                        halves((uint32_t)row, row1, up);
                     } else {
-                        // triangles of G[X]: through the complement when X is nearly a
-                        // clique, else every triangle i < j < l counted at i
-                        const uint64_t cmpl = mem ? (X & ~row & lane_above) : 0ull;
-                        const uint32_t cmax =
-                            (uint32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_max_u32((uint32_t)__popcll(cmpl)));
-                        const uint32_t tri = (3 * cmax < 2 * cx) ? tri_complement(row, cmpl, cmax, mem, v, cx)
-                                                                 : tri_direct(X, row, lane_above);
-                        add_checked(acc, pp * (pp - (pp ? 1 : 0)) * (pp >= 2 ? pp - 2 : 0) / 6, ovf);
-                        add_checked(acc, pp * (pp - (pp ? 1 : 0)) / 2 * cx, ovf);
-                        add_checked(acc, pp * (e2 / 2), ovf);
-                        add_checked(acc, tri, ovf);
+                        // the members' rows to the lanes 0..cx-1 (the other rows to lane 63), then
+                        // new row j = ballot of bit x_j over them (the bitmap is symmetric)
+                        const int to = (int)((in_mask(X) ? (uint32_t)__popcll(X & lanemask_lt()) : 63u) << 2);
+                        uint32_t lo = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)(uint32_t)row);
+                        uint32_t hi = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)(uint32_t)(row >> 32));
+                        if (lane >= cx) lo = hi = 0;
+                        uint32_t j = 0;
+                        for (uint32_t bits = (uint32_t)X; bits; bits &= bits - 1, ++j) {
+                            const uint32_t col = (uint32_t)__ballot((lo & (bits & -bits)) != 0);
+                            row1 = (lane & 31) == j ? col : row1;
+                        }
+                        for (uint32_t bits = (uint32_t)(X >> 32); bits; bits &= bits - 1, ++j) {
+                            const uint32_t col = (uint32_t)__ballot((hi & (bits & -bits)) != 0);
+                            row1 = (lane & 31) == j ? col : row1;
+                        }
+                        X1 = cx >= 32 ? ~0u : (1u << cx) - 1;
                     }
-                } else if (h + 4 == k) {
-                    // h = k-4: the subtree holds
-                    // C(p,4) + C(p,3)|X| + C(p,2)|E(X)| + p c3(X) + c4(X) k-cliques
-                    const CliqueCounts cc = k34_complement(X, row, mem, cx);
-                    add_checked(acc, binom_chk(a, p, 4, ovf), ovf);
-                    add_checked(acc, mul_chk(binom_chk(a, p, 3, ovf), cx, ovf), ovf);
-                    add_checked(acc, mul_chk(binom_chk(a, p, 2, ovf), cc.e, ovf), ovf);
-                    add_checked(acc, mul_chk(p, cc.c3, ovf), ovf);
-                    add_checked(acc, cc.c4, ovf);
-                } else {
-                    // (score + 1, 63 - index): the max names the smallest index of the largest score
-                    uint32_t key = mem ? (((v + 1) << 8) | (63u - lane)) : 0u;
-                    key = (uint32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_max_u32(key));
-                    if ((key >> 8) + h + p >= k) {  // (key >> 8) = max score + 1 bounds the clique inside X
-                        const uint32_t pv = 63u - (key & 0xFFu);
-                        ++t;
-                        const uint64_t bw = X & ~rdlane64(row, pv);
-                        stkC = (lane == (uint32_t)t) ? X : stkC;
-                        stkB = (lane == (uint32_t)t) ? bw : stkB;
-                        const uint32_t M = h | (p << 8) | (pv << 20);
-                        stkM = (lane == (uint32_t)t) ? M : stkM;
+                    add_checked(acc, sct_word<MM, uint32_t>(a, k, row1, X1, h, p, nodes, ovf), ovf);
+                    --my_nodes;  // counted again as the subtree's root
+                }
+            } else {
+                bool close = need < 5 || cx == 0;
+                if (!close) {
+                    const uint32_t sc = bits_of((U)(X & row));
+                    const U all = (U)__ballot(in_mask(mask64(X)) && sc + 1 == cx);  // adjacent to every other candidate
+                    const uint32_t na = bits_of(all);
+                    X &= ~all;
+                    p += na;
+                    cx -= na;
+                    close = cx <= 4;
+                    if (!close) {
+                        // (score + 1, BITS-1 - index): the max names the smallest index of the largest score
+                        uint32_t key = in_mask(mask64(X)) ? ((sc - na + 1) << 8) | (BITS - 1 - v) : 0u;
+                        key = (uint32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_max_u32(key));
+                        if ((key >> 8) + p >= need) {  // (key >> 8) = max score + 1 bounds the clique inside X
+                            const uint32_t pv = BITS - 1 - (key & 0xFFu);
+                            if (open) {
+                                ++t;
+                                stkC = lane == (uint32_t)t ? tC : stkC;
+                                stkB = lane == (uint32_t)t ? tB : stkB;
+                                stkM = lane == (uint32_t)t ? tM : stkM;
+                            }
+                            open = true;
+                            tC = X;
+                            tB = X & ~rdlane(row, pv) & ~((U)1 << pv);
+                            tM = h | (p << 8) | (pv << 20);
+                        }
                     }
+                }
+                if (close) {
+                    const CloseTerm term(a, need, p);
+                    CliqueCounts c{0, 0, 0};
+                    if (cx >= 2 && need >= 3) {
+                        c = close_word<MM>(X, row, cx, need > 3);
+                    } else if (cx >= 2 && need == 2) {
+                        const uint32_t sc = in_mask(mask64(X)) ? bits_of((U)(X & row)) : 0u;
+                        c.e = wave_sum32(sc) / (BITS == 32 ? 4 : 2);
+                    }
+                    term.add(acc, ovf, cx, c);
                 }
             }
         }
-        if (t < 0) break;
-        // next branch of level t: non-pivot vertices first, the pivot last
-        uint64_t Cc = rdlane64(stkC, (uint32_t)t), B = rdlane64(stkB, (uint32_t)t);
-        const uint32_t M = (uint32_t)__builtin_amdgcn_readlane((int)stkM, t);
-        const uint32_t hh = M & 0xFF, pp = (M >> 8) & 0xFFF, pv = M >> 20;
-        const uint64_t nb = B & ~(1ull << pv);
-        const bool last = nb == 0;
-        const uint32_t b = last ? pv : (uint32_t)__builtin_ctzll(nb);
-        X = Cc & rdlane64(row, b);
-        h = hh + (last ? 0u : 1u);
-        p = pp + (last ? 1u : 0u);
-        if (last) {
-            --t;  // the pivot branch replaces its level
-        } else {
-            Cc &= ~(1ull << b);
-            B &= ~(1ull << b);
-            stkC = (lane == (uint32_t)t) ? Cc : stkC;
-            stkB = (lane == (uint32_t)t) ? B : stkB;
+        // next branch of the open level: non-pivot vertices first, the pivot last
+        if (!open) {
+            if (t < 0) break;
+            tC = rdlane(stkC, (uint32_t)t);
+            tB = rdlane(stkB, (uint32_t)t);
+            tM = (uint32_t)__builtin_amdgcn_readlane((int)stkM, t);
+            --t;
+            open = true;
         }
-        if (h <= k) pending = true;
+        h = tM & 0xFF;
+        p = (tM >> 8) & 0xFFF;
+        if (tB) {
+            const uint32_t b = low_bit(tB);
+            X = tC & rdlane(row, b);
+            tC &= ~((U)1 << b);
+            tB &= tB - 1;
+            ++h;
+        } else {  // the pivot branch replaces its level
+            X = tC & rdlane(row, tM >> 20);
+            ++p;
+            open = false;
+        }
     }
     if (lane == 0) nodes += my_nodes;
     return acc;
+}
+
+// SCT of a one-word subproblem (row = the lane's row, 0 beyond the subproblem)
+template <bool MM>
+__device__ inline uint64_t sct64(const CountArgs &a, uint32_t k, uint64_t row, uint64_t X0, uint32_t h0, uint32_t p0,
+                                 uint64_t &nodes, uint32_t &ovf)
+{
+    return sct_word<MM, uint64_t>(a, k, row, X0, h0, p0, nodes, ovf);
 }
 
 // ---- step 3b: pivoting (SCT) ----------------------------------------------
@@ -822,7 +934,9 @@ __device__ uint64_t pivot_count(const CountArgs &a, uint32_t P, uint32_t k, cons
                     const uint64_t col = __ballot((wv >> (xj & 63)) & 1ull);
                     row1 = (lane == j) ? col : row1;
                 }
-                add_checked(acc, sct64(a, k, row1, cx >= 64 ? ~0ull : ((1ull << cx) - 1), h, p, nodes, ovf), ovf);
+                uint32_t lo = 0;
+                const uint64_t part = sct64<true>(a, k, row1, cx >= 64 ? ~0ull : ((1ull << cx) - 1), h, p, nodes, lo);
+                add_checked(acc, wave_total(part, lo, ovf), ovf);
                 --my_nodes;  // counted again as the subtree's root
             } else if (!LOCAL && crows4 && cx > 128 && cx <= 256 && h + 3 <= k && h + p + cx >= k) {
                 // 129..256 candidates: re-encode three or four words per row the
@@ -844,7 +958,9 @@ __device__ uint64_t pivot_count(const CountArgs &a, uint32_t P, uint32_t k, cons
                     if (lane < Wc) crows4[(uint64_t)Wc * j + lane] = mine;
                 }
                 sync_tree<WIDE>();
-                add_checked(acc, pivot_reg<4, true>(a, k, crows4, cx, h, cand, nodes, ovf, p, crows2), ovf);
+                uint32_t lo = 0;
+                const uint64_t part = pivot_reg<4, true>(a, k, crows4, cx, h, cand, nodes, lo, p, crows2);
+                add_checked(acc, wave_total(part, lo, ovf), ovf);
                 --my_nodes;
             } else if (!LOCAL && crows2 && cx <= 128 && h + 3 <= k && h + p + cx >= k) {
                 // 65..128 candidates: re-encode two words per row (word t of new
@@ -859,7 +975,9 @@ __device__ uint64_t pivot_count(const CountArgs &a, uint32_t P, uint32_t k, cons
                     if (lane < 2) crows2[2 * j + lane] = lane ? c1 : c0;
                 }
                 sync_tree<WIDE>();
-                add_checked(acc, pivot_reg<2>(a, k, crows2, cx, h, cand, nodes, ovf, p, nullptr), ovf);
+                uint32_t lo = 0;
+                const uint64_t part = pivot_reg<2>(a, k, crows2, cx, h, cand, nodes, lo, p, nullptr);
+                add_checked(acc, wave_total(part, lo, ovf), ovf);
                 --my_nodes;
             } else if (h + p + cx >= k) {
                 // scores |X & row_j| for j in X: P lanes per candidate
@@ -1042,7 +1160,7 @@ __device__ uint64_t compact_and_count(const CountArgs &a, uint32_t k, const uint
         }
     }
     const uint64_t X1 = cx >= 64 ? ~0ull : ((1ull << cx) - 1);
-    return sct64(a, k, row1, X1, h, p, nodes, ovf);
+    return sct64<true>(a, k, row1, X1, h, p, nodes, ovf);
 }
 
 // Triangles of G[X] for X of up to 64*S vertices (rows of stride W in LDS) by
@@ -1120,13 +1238,14 @@ __device__ uint32_t tri_lanes(const uint64_t *rows, uint32_t W, const uint64_t (
     return comp ? cx * (cx - 1) * (cx - 2) / 6 - tot / 2 : tot / 2;
 }
 
-// k34_complement for X of up to 64*S vertices (rows of stride W in LDS): lane
-// l takes the vertices l + 64s, s < S, with their complement rows in S words
-// each; the same uniform walk over u in X, the same four running sums per
-// vertex and the same K4 walk over the vertices in three or more complement
-// triangles, with the lane shares summed in 64 bits (C(256,4) * 24 does not
-// fit 32).  Used at h = k-4 when X is a near-clique (the complement walks
-// stay short).
+// The counts of close_word for X of up to 64*S vertices (rows of stride W in
+// LDS): lane l takes the vertices l + 64s, s < S, with their complement rows in
+// S words each.  Two words go through the matrix cores like one; over four
+// (the wide kernel) the operands would not fit the registers, and a uniform
+// walk over u in X keeps the four running sums of each vertex, summed over
+// the lanes in 64 bits (C(256,4) * 24 does not fit 32).  Used at h = k-4 when X
+// is a near-clique (the K4 walk, over the vertices in three or more complement
+// triangles, stays short).
 template <int S>
 __device__ CliqueCounts k34_complement_rows(const uint64_t *rows, uint32_t W, const uint64_t (&X)[S], uint32_t cx)
 {
@@ -1146,41 +1265,57 @@ __device__ CliqueCounts k34_complement_rows(const uint64_t *rows, uint32_t W, co
             d[s] += __popcll(Hl[s][w]);
         }
     }
+    uint64_t T3[S];
+    uint32_t s4 = 0, s3 = 0, s2 = 0;  // (S = 2)
     uint32_t q[S], qE[S], t2[S], sd[S];
+    if constexpr (S == 2) {
+        uint32_t H[4][4], t3[4], live = 0;
 #pragma unroll
-    for (int s = 0; s < S; ++s) q[s] = qE[s] = t2[s] = sd[s] = 0;
+        for (int s = 0; s < 2; ++s)
 #pragma unroll
-    for (int wu = 0; wu < S; ++wu) {
-        for (uint64_t bits = X[wu]; bits; bits &= bits - 1) {
-            const uint32_t u = 64u * wu + (uint32_t)__builtin_ctzll(bits);
-            uint64_t Hu[S];
-            uint32_t du = 0;
-#pragma unroll
-            for (int w = 0; w < S; ++w) {
-                Hu[w] = X[w] & ~lds_row_word(rows, W, u, w) & (w == wu ? ~(1ull << (u & 63)) : ~0ull);
-                du += (uint32_t)__popcll(Hu[w]);
+            for (int w = 0; w < 2; ++w) {
+                halves((uint32_t)Hl[s][w], H[2 * s][2 * w], H[2 * s + 1][2 * w]);
+                halves((uint32_t)(Hl[s][w] >> 32), H[2 * s][2 * w + 1], H[2 * s + 1][2 * w + 1]);
             }
 #pragma unroll
-            for (int s = 0; s < S; ++s) {
-                uint32_t c = 0;
+        for (int J = 0; J < 4; ++J) live |= (uint32_t)(X[J >> 1] >> (32 * (J & 1))) ? 1u << J : 0u;
+        complement_sums<4>(H, live, cx, s4, s3, s2, t3);
+        T3[0] = ((uint64_t)t3[1] << 32) | t3[0];
+        T3[1] = ((uint64_t)t3[3] << 32) | t3[2];
+    } else {
 #pragma unroll
-                for (int w = 0; w < S; ++w) c += (uint32_t)__popcll(Hl[s][w] & Hu[w]);
-                const uint32_t c2 = c * c, in = (uint32_t)(Hu[s] >> lane) & 1u;
-                q[s] += c2;
-                qE[s] += in * c2;
-                t2[s] += in * c;
-                sd[s] += in * du;
+        for (int s = 0; s < S; ++s) q[s] = qE[s] = t2[s] = sd[s] = 0;
+#pragma unroll
+        for (int wu = 0; wu < S; ++wu) {
+            for (uint64_t bits = X[wu]; bits; bits &= bits - 1) {
+                const uint32_t u = 64u * wu + (uint32_t)__builtin_ctzll(bits);
+                uint64_t Hu[S];
+                uint32_t du = 0;
+#pragma unroll
+                for (int w = 0; w < S; ++w) {
+                    Hu[w] = X[w] & ~lds_row_word(rows, W, u, w) & (w == wu ? ~(1ull << (u & 63)) : ~0ull);
+                    du += (uint32_t)__popcll(Hu[w]);
+                }
+#pragma unroll
+                for (int s = 0; s < S; ++s) {
+                    uint32_t c = 0;
+#pragma unroll
+                    for (int w = 0; w < S; ++w) c += (uint32_t)__popcll(Hl[s][w] & Hu[w]);
+                    const uint32_t c2 = c * c, in = (uint32_t)(Hu[s] >> lane) & 1u;
+                    q[s] += c2;
+                    qE[s] += in * c2;
+                    t2[s] += in * c;
+                    sd[s] += in * du;
+                }
             }
         }
+#pragma unroll
+        for (int s = 0; s < S; ++s) T3[s] = __ballot(t2[s] >= 6);
     }
     // K4 of H among the vertices in >= 3 H-triangles (bit l of word s = vertex l + 64s)
-    uint64_t T3[S];
     uint32_t nt3 = 0;
 #pragma unroll
-    for (int s = 0; s < S; ++s) {
-        T3[s] = __ballot(t2[s] >= 6);
-        nt3 += (uint32_t)__popcll(T3[s]);
-    }
+    for (int s = 0; s < S; ++s) nt3 += (uint32_t)__popcll(T3[s]);
     int64_t k4acc[S];
 #pragma unroll
     for (int s = 0; s < S; ++s) k4acc[s] = 0;
@@ -1224,6 +1359,10 @@ __device__ CliqueCounts k34_complement_rows(const uint64_t *rows, uint32_t W, co
             }
         }
     }
+    if constexpr (S == 2) {
+        s4 += 24 * (uint32_t)(k4acc[0] + k4acc[1]);
+        return complement_counts(cx, wave_sum32(s2) / 2, wave_sum32(s3), wave_sum32(s4));
+    }
     int64_t c4l = 0, c3l = 0, sdl = 0;
 #pragma unroll
     for (int s = 0; s < S; ++s) {
@@ -1255,10 +1394,6 @@ __device__ CliqueCounts k34_complement_rows(const uint64_t *rows, uint32_t W, co
 // quarter of the four-word ones.  Lanes l and l+64 load the full rows of
 // members l and l+64; word t of new row j is the ballot over lanes of bit x_j
 // of the rows of members 64t + lane (the bitmap is symmetric).
-template <int S, bool CL4>
-__device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t R, uint32_t h0,
-                              uint32_t *idx, uint64_t &nodes, uint32_t &ovf, uint32_t p0, uint64_t *crows);
-
 template <int S>
 __device__ uint64_t compact2_and_count(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t W,
                                        const uint64_t (&X)[S], uint32_t *idx, uint64_t *crows, uint32_t h, uint32_t p,
@@ -1307,7 +1442,7 @@ __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *ro
     const uint32_t W = (R + 63) / 64;
     if (S == 1) {
         const uint64_t r1 = lane < R ? rows[lane] : 0ull;
-        return sct64(a, k, r1, R >= 64 ? ~0ull : ((1ull << R) - 1), h0, p0, nodes, ovf);
+        return sct64<false>(a, k, r1, R >= 64 ? ~0ull : ((1ull << R) - 1), h0, p0, nodes, ovf);
     }
     // rows of the lane in VGPRs for the two-word kernel; the four-word level
     // (a small share of the work once subtrees of <= 128 candidates are
@@ -1354,20 +1489,11 @@ __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *ro
             } else if (cx <= 64 && cx > 0 && h + 3 <= k && h + p + cx >= k) {
                 // a subtree of at most 64 candidates: one word per row from here on
                 add_checked(acc, compact_and_count<S>(a, k, rows, W, X, idx, h, p, nodes, ovf), ovf);
-            } else if ((++my_nodes, cx == 0)) {
-                if (k >= h && k - h <= p) {
-                    const uint64_t idx = (uint64_t)p * a.bstride + (k - h);
-                    if (a.binom_ovf[idx]) ovf = 1;
-                    add_checked(acc, a.binom[idx], ovf);
-                }
-            } else if (h >= k) {
-                add_checked(acc, 1, ovf);
-            } else if (h + 1 == k) {
-                add_checked(acc, (uint64_t)p + cx, ovf);
-            } else if (h + p + cx >= k) {
+            } else if (++my_nodes, h + p + cx >= k) {
                 // scores |X & row_j| of the lane's member rows; key packs
                 // (score + 1, 0xFFFF - j), so the wave max names the smallest j of
                 // the largest score
+                const uint32_t need = k - h;  // (h <= k)
                 uint32_t key = 0, lsum = 0;
 #pragma unroll
                 for (int s = 0; s < S; ++s) {
@@ -1380,31 +1506,18 @@ __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *ro
                         key = kk > key ? kk : key;
                     }
                 }
-                uint32_t e2 = 0;
-                if (h + 4 >= k) e2 = (uint32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_add_u32(lsum));
-                if ((S == 2 || (S == 4 && CL4)) && h + 4 == k && 4 * (uint64_t)e2 >= 3ull * cx * (cx - 1)) {
-                    // h = k-4 over a near-clique (complement density <= 1/4): closed form
-                    const CliqueCounts cc = k34_complement_rows<S>(rows, W, X, cx);
-                    add_checked(acc, binom_chk(a, p, 4, ovf), ovf);
-                    add_checked(acc, mul_chk(binom_chk(a, p, 3, ovf), cx, ovf), ovf);
-                    add_checked(acc, mul_chk(binom_chk(a, p, 2, ovf), cc.e, ovf), ovf);
-                    add_checked(acc, mul_chk(p, cc.c3, ovf), ovf);
-                    add_checked(acc, cc.c4, ovf);
-                } else if (h + 3 >= k) {
-                    // (e2 = twice the edges of G[X])
-                    const uint64_t pp = p;
-                    if (h + 2 == k) {
-                        add_checked(acc, pp * (pp - (pp ? 1 : 0)) / 2, ovf);
-                        add_checked(acc, pp * cx, ovf);
-                        add_checked(acc, e2 / 2, ovf);
-                    } else {
-                        // h = k-3: C(p,3) + C(p,2)|X| + p|E(X)| + triangles(X)
-                        const uint32_t tri = tri_lanes<S>(rows, W, X, cx, e2, idx);
-                        add_checked(acc, pp * (pp - (pp ? 1 : 0)) * (pp >= 2 ? pp - 2 : 0) / 6, ovf);
-                        add_checked(acc, pp * (pp - (pp ? 1 : 0)) / 2 * cx, ovf);
-                        add_checked(acc, pp * (e2 / 2), ovf);
-                        add_checked(acc, tri, ovf);
-                    }
+                uint32_t e2 = 0;  // twice the edges of G[X]
+                if (need <= 4) e2 = wave_sum32(lsum);
+                const bool near = (S == 2 || (S == 4 && CL4)) && need == 4 && 4 * (uint64_t)e2 >= 3ull * cx * (cx - 1);
+                if (near || need <= 3 || cx == 0) {
+                    // closed forms: h >= k-3, and h = k-4 over a near-clique (complement
+                    // density <= 1/4)
+                    const CloseTerm term(a, need, p);
+                    CliqueCounts c{0, 0, 0};
+                    if (near && cx) c = k34_complement_rows<S>(rows, W, X, cx);
+                    else if (need >= 2) c.e = e2 / 2;
+                    if (need == 3 && cx) c.c3 = tri_lanes<S>(rows, W, X, cx, e2, idx);
+                    term.add(acc, ovf, cx, c);
                 } else if ((((key = (uint32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_max_u32(key))) >> 16) +
                             h + p) >= k) {  // (key >> 16) = max score + 1 bounds the clique inside X
                     const uint32_t pv = 0xFFFFu - (key & 0xFFFFu);
@@ -1505,11 +1618,13 @@ __device__ __attribute__((always_inline)) uint32_t stage_task(const Cur &g, uint
 // changes and at the end), and the launch statistics.
 struct WaveAcc {
     uint32_t q = INF32;
-    uint64_t run = 0;
-    uint32_t run_ovf = 0;
+    uint64_t run = 0;      // this lane's share of the query's count
+    uint32_t run_ovf = 0;  // this lane saw an overflow
     uint64_t bytes = 0, ntask = 0, nodes = 0, tmax = 0, tsum = 0;
-    uint32_t any_ovf = 0;
 };
+
+// add a value every lane holds alike to the wave's running count
+__device__ inline void run_add(WaveAcc &w, uint64_t v) { add_checked(w.run, lane_id() == 0 ? v : 0ull, w.run_ovf); }
 
 __device__ __attribute__((always_inline)) void flush_query(const CountArgs &a, WaveAcc &w)
 {
@@ -1518,12 +1633,13 @@ __device__ __attribute__((always_inline)) void flush_query(const CountArgs &a, W
     // wrap, so nothing has to come back, and the host joins them and sees an
     // overflow of the whole
     const int lane = lane_id();
-    if (lane < 2 && w.run) {
+    uint32_t ovf = 0;
+    const uint64_t run = wave_total(w.run, w.run_ovf, ovf);
+    if (lane < 2 && run) {
         uint64_t *at = a.single ? a.acc + (uint64_t)(blockIdx.x & a.acc_mask) * ACC + 6 * lane : a.qcount + 2ull * w.q + lane;
-        atomicAdd((unsigned long long *)at, (unsigned long long)(lane ? w.run >> 32 : w.run & 0xFFFFFFFFull));
+        atomicAdd((unsigned long long *)at, (unsigned long long)(lane ? run >> 32 : run & 0xFFFFFFFFull));
     }
-    if (lane == 0 && w.run_ovf) atomicOr(&a.qovf[w.q], 1u);
-    w.any_ovf |= w.run_ovf;
+    if (lane == 0 && ovf) atomicOr(&a.qovf[w.q], 1u);
     w.run = 0;
     w.run_ovf = 0;
 }
@@ -1614,7 +1730,7 @@ __device__ __attribute__((always_inline)) uint32_t next_tasks(const CountArgs &a
 // register-bitmap pivoting kernel for tasks of at most 64*S vertices
 // waves per SIMD the register budget is held to: 4 for S = 4 (<= 128 VGPRs), 6 for S = 2, 8 for S = 1
 template <int S>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S == 4 ? 4 : S == 2 ? 6 : 8)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S == 4 ? 4 : S == 2 ? 4 : 8)))
 void k_pivot_reg(CountArgs a)
 {
     extern __shared__ uint64_t lds[];
@@ -1627,6 +1743,10 @@ void k_pivot_reg(CountArgs a)
     // (S = 4) the two-word rows of a compacted subtree, 128 x 2 words, over
     // list and starts (256 u32 each, dead once the bitmap is built)
     uint64_t *crows = lds + L.list;
+    // the launch statistics are kept in LDS (lane 0; as acc, [6] the task's
+    // start): they are touched once a task and would hold registers through it
+    uint64_t *st = lds + L.misc;
+    if (lane < 8) st[lane] = 0;
     WaveAcc w;
     if (a.ntasks_p) a.ntasks = uni32(*a.ntasks_p);
     TaskQueue tq(blockIdx.x);
@@ -1635,26 +1755,39 @@ void k_pivot_reg(CountArgs a)
         if (start == INF32) break;
         const uint32_t stop = start + min(a.ntasks - start, 1u << a.chunk_log);
         for (uint32_t ti = start; ti < stop; ++ti) {
-            const uint64_t t0 = wall_clock64();
+            if (lane == 0) st[6] = wall_clock64();
             uint32_t task;
             const Cur g = select_task(a, a.tasks[ti], w, task);
-            ++w.ntask;
-            const uint32_t R = stage_task(g, task, list, w.bytes);
+            uint64_t bytes = 0;
+            const uint32_t R = stage_task(g, task, list, bytes);
+            if (lane == 0) ++st[2];
             if (g.gran && g.k == 3) {  // an edge task at k=3 adds |T| (no bitmap needed)
-                add_checked(w.run, R, w.run_ovf);
+                run_add(w, R);
+                if (lane == 0) st[1] += bytes;
                 __syncthreads();
                 continue;
             }
             __syncthreads();
-            build_rows<true>(g, list, offs, starts, rows, R, (R + 63) / 64, w.bytes);
-            add_checked(w.run, pivot_reg<S>(a, g.k, rows, R, g.gran ? 2u : 1u, offs, w.nodes, w.run_ovf, 0u, crows),
+            build_rows<true>(g, list, offs, starts, rows, R, (R + 63) / 64, bytes);
+            if (lane == 0) st[1] += bytes;
+            uint64_t nodes = 0;
+            add_checked(w.run, pivot_reg<S>(a, g.k, rows, R, g.gran ? 2u : 1u, offs, nodes, w.run_ovf, 0u, crows),
                         w.run_ovf);
             __syncthreads();
-            const uint64_t dt = wall_clock64() - t0;
-            w.tmax = dt > w.tmax ? dt : w.tmax;
-            w.tsum += dt;
+            if (lane == 0) {
+                const uint64_t dt = wall_clock64() - st[6];
+                st[3] += nodes;
+                st[4] = dt > st[4] ? dt : st[4];
+                st[5] += dt;
+            }
         }
     }
+    __syncthreads();
+    w.bytes = st[1];
+    w.ntask = st[2];
+    w.nodes = lane == 0 ? st[3] : 0;
+    w.tmax = st[4];
+    w.tsum = st[5];
     finish_wave(a, w);
 }
 
@@ -1743,10 +1876,12 @@ __device__ __attribute__((always_inline)) void open_flush(const OpenArgs &oa, Wa
 {
     if (w.q == INF32) return;
     const CountArgs &a = oa.c;
+    uint32_t run_ovf = 0;
+    const uint64_t run = wave_total(w.run, w.run_ovf, run_ovf);
     if (lane_id() == 0 && pend) {
         const uint32_t q = w.q;
-        const unsigned long long old = atomicAdd((unsigned long long *)&a.qcount[q], (unsigned long long)w.run);
-        if (old + w.run < old || w.run_ovf) atomicOr(&a.qovf[q], 1u);
+        const unsigned long long old = atomicAdd((unsigned long long *)&a.qcount[q], (unsigned long long)run);
+        if (old + run < old || run_ovf) atomicOr(&a.qovf[q], 1u);
         const uint64_t before = __hip_atomic_fetch_add(&oa.qdone[q], (uint64_t)pend, __ATOMIC_ACQ_REL,
                                                        __HIP_MEMORY_SCOPE_AGENT);
         if (before + pend == total) {
@@ -1760,7 +1895,6 @@ __device__ __attribute__((always_inline)) void open_flush(const OpenArgs &oa, Wa
             __hip_atomic_store(&oa.mail[q].seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
-    w.any_ovf |= w.run_ovf;
     w.run = 0;
     w.run_ovf = 0;
     pend = 0;
@@ -1842,7 +1976,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) void k_
         const uint32_t need = g.gran ? g.k - 2 : g.k - 1;
         if (R >= need) {
             if (g.gran && g.k == 3) {
-                add_checked(w.run, R, w.run_ovf);
+                run_add(w, R);
             } else {
                 __syncthreads();
                 build_rows<true>(g, list, offs, starts, rows, R, (R + 63) / 64, w.bytes);
@@ -1912,7 +2046,7 @@ __global__ __launch_bounds__(64) void k_count(CountArgs a)
             if (LOCAL)
                 for (uint32_t i = lane; i < R; i += 64) lacc[i] = 0;
             if (g.gran && k == 3) {  // an edge task at k=3 adds |T| (no bitmap needed)
-                add_checked(w.run, R, w.run_ovf);
+                run_add(w, R);
                 if (LOCAL) {
                     for (uint32_t i = lane; i < R; i += 64) lacc[i] = 1;
                     __syncthreads();
@@ -1931,15 +2065,15 @@ __global__ __launch_bounds__(64) void k_count(CountArgs a)
                 uint32_t povf = 0;
                 uint64_t part = orient_count<LOCAL>(a, g.psize, rows, stk, misc, R, W, g.gran ? k - 2 : k - 1,
                                                     w.nodes, povf, lacc, path);
-                task_count = wave_sum64_checked(part, povf);
-                w.run_ovf |= (wave_min32(povf ? 0u : 1u) == 0) ? 1u : 0u;
-                add_checked(w.run, task_count, w.run_ovf);
+                task_count = LOCAL ? wave_sum64_checked(part, povf) : 0ull;
+                w.run_ovf |= povf;
+                add_checked(w.run, part, w.run_ovf);
             } else {
                 // SCT rooted at the node (held 1) or the edge (held 2)
                 build_rows<true>(g, list, offs, starts, rows, R, W, w.bytes);
                 task_count = pivot_count<LOCAL>(a, g.psize, k, rows, stk, X, scal, offs, R, W, g.gran ? 2u : 1u,
                                                 w.nodes, w.run_ovf, lacc);
-                add_checked(w.run, task_count, w.run_ovf);
+                run_add(w, task_count);
             }
             __syncthreads();
             publish_local<LOCAL>(a, g, task, list, lacc, R, task_count);
@@ -2072,7 +2206,7 @@ __global__ __launch_bounds__(512) void k_pivot_wide(CountArgs a)
         __syncthreads();
         const uint32_t R = ctl[1], W = (R + 63) / 64;
         if (g.gran && k == 3) {  // an edge task at k=3 adds |T| (no bitmap needed)
-            if (wv == 0) add_checked(w.run, R, w.run_ovf);
+            if (wv == 0) run_add(w, R);
             __syncthreads();
             continue;
         }
@@ -2101,7 +2235,7 @@ __global__ __launch_bounds__(512) void k_pivot_wide(CountArgs a)
                     if (k >= h0 && k - h0 <= p) {
                         const uint64_t idx = (uint64_t)p * a.bstride + (k - h0);
                         if (a.binom_ovf[idx]) w.run_ovf = 1;
-                        add_checked(w.run, a.binom[idx], w.run_ovf);
+                        run_add(w, a.binom[idx]);
                     }
                     break;
                 }
@@ -2129,7 +2263,7 @@ __global__ __launch_bounds__(512) void k_pivot_wide(CountArgs a)
                 const uint64_t tot_s = wave_sum64_checked(sum_s, dummy);
                 const uint32_t max_s = (uint32_t)(key >> 32), pv = INF32 - (uint32_t)(key & 0xFFFFFFFFull);
                 if (j == 0 && h0 + 2 == k) {  // k-cliques of T with the root's h0 held: |E(T)|
-                    add_checked(w.run, tot_s / 2, w.run_ovf);
+                    run_add(w, tot_s / 2);
                     break;
                 }
                 if (h0 + p + max_s + 1 < k) break;
@@ -2174,10 +2308,8 @@ __global__ __launch_bounds__(512) void k_pivot_wide(CountArgs a)
                 }
             }
             const uint32_t h = end ? h0 : h0 + 1;
-            add_checked(w.run,
-                        pivot_count<false, true>(a, g.psize, k, rows, stk, X, scal, cand, R, W, h, w.nodes, w.run_ovf,
-                                                 nullptr, j, false, crows2, crows4),
-                        w.run_ovf);
+            run_add(w, pivot_count<false, true>(a, g.psize, k, rows, stk, X, scal, cand, R, W, h, w.nodes, w.run_ovf,
+                                                nullptr, j, false, crows2, crows4));
         }
         __syncthreads();
         if (wv == 0) {
@@ -2556,8 +2688,7 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     for (uint32_t i = 0; i < nq; ++i) {
         const kc_oriented *o = qs[i].o;
         const kc_query &q = qs[i].q;
-        hq[i] = QDesc{o->rowptr.as<uint32_t>(), o->col.as<uint32_t>(), o->src.as<uint32_t>(), q.k, q.gran,
-                      std::max<uint32_t>(1, qs[i].sample), qs[i].sample > 1 ? qs[i].offset : 0, q.part_size};
+        hq[i] = QDesc{o->rowptr.as<uint32_t>(), o->col.as<uint32_t>(), o->src.as<uint32_t>(), q.k, q.gran, std::max<uint32_t>(1, qs[i].sample), qs[i].sample > 1 ? qs[i].offset : 0, q.part_size};
         halgo[i] = (uint8_t)(q.algo == KC_ALGO_PIVOT);
         hoff[i + 1] = hoff[i] + (q.gran == KC_GRAN_EDGE ? o->m : o->n);
         kmax = std::max(kmax, q.k);

@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import kcgpu_amd as K
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -64,3 +65,47 @@ def test_binning_of_many_queries():
         exp.append(sum(comb(s, k) * t for s, t in parts[j]))
     res, _ = K.batch_count(pairs)
     assert [r.count for r in res] == exp
+
+
+def _oracle_count(G, mode, k, gran):
+    rp, col = G.csr()
+    rp = rp.astype(np.uint64)
+    orp, oc = O.orient(rp, col, O.peel_priority(rp, col)[0] if mode == "degen" else None)
+    return O.count(orp, oc, k, "pivot_tails", gran)["count"]
+
+
+# candidate sets at the edges of the 32- and 64-vertex words, of the matrix blocks and of the register classes
+@pytest.mark.parametrize("n", [5, 6, 31, 32, 33, 34, 63, 64, 65, 66, 96, 97, 128, 129, 130, 160, 200])
+@pytest.mark.parametrize("density", [0.3, 0.7, 0.93])
+def test_dense_random_graphs_vs_oracle(n, density):
+    r = np.random.default_rng(n * 100 + int(density * 100))
+    a, b = np.triu_indices(n, 1)
+    keep = r.random(a.size) < density
+    G = K.Graph.from_edges(a[keep].astype(np.uint32), b[keep].astype(np.uint32), n)
+    o = G.orient("degree")
+    for k in (4, 5) + ((6,) if n <= 130 else ()) + ((7, 8) if n <= 66 else ()):
+        exp = _oracle_count(G, "degree", k, "node")
+        for gran in ("node", "edge"):
+            r = o.count(k, "pivot", gran, part_size=1)
+            assert r.count == exp, (k, gran)
+
+
+# 11 node tasks above 128 vertices a clique: on both sides of the line between one wave and one block a task
+@pytest.mark.parametrize("cliques", [1, 325, 326])
+def test_tasks_above_128_vertices_few_and_many(cliques):
+    src, dst, n = _disjoint_cliques([(140, cliques)])
+    o = K.orient_edges(src, dst, "degree", n=n)
+    for k in (4, 6, 9):
+        assert o.count(k, "pivot", "node", part_size=1).count == cliques * comb(140, k)
+
+
+# out-lists much longer than the tasks (pair by pair) and about as long (entry by entry)
+@pytest.mark.parametrize("n,m,hub", [(3000, 40_000, 900), (20_000, 120_000, 4000), (20_000, 40_000, 50)])
+@pytest.mark.parametrize("mode", ["degree", "degen"])
+def test_bitmaps_of_short_tasks_in_long_rows(n, m, hub, mode):
+    G = K.Graph.generate(K.GEN_CHUNG_LU, seed=n + m, n=n, m=m, gamma=2.1, max_degree=hub)
+    o = G.orient(mode)
+    for k, gran in ((4, "node"), (4, "edge"), (5, "edge")):
+        exp = _oracle_count(G, mode, k, gran)
+        for algo in ("pivot", "orient"):
+            assert o.count(k, algo, gran, part_size=1).count == exp, (k, gran, algo)
