@@ -64,7 +64,7 @@ constexpr uint32_t PIVOT_TOP2 = 256;  // largest pivoting task of the four-word 
 
 // one query of a launch: the oriented graph it runs on and its k
 struct QDesc {
-    const uint32_t *rowptr, *col, *src;
+    const uint32_t *rowptr, *col, *src, *key;
     uint32_t k, gran, sample, offset;  // tasks with id % sample == offset run
     uint32_t psize;                    // lanes per partition of this query
 };
@@ -72,7 +72,7 @@ static_assert(sizeof(QDesc) % 8 == 0, "QDesc is read as 64-bit words");
 
 // the graph and k of the task a wave is working on
 struct Cur {
-    const uint32_t *rowptr, *col, *src;
+    const uint32_t *rowptr, *col, *src, *key;  // key: the orientation's (null: not at hand)
     uint32_t k, gran, psize;
 };
 
@@ -107,8 +107,9 @@ struct CountArgs {
 // the current node and of every stack level, and for both traversals a u64
 // accumulator per task vertex (lacc) and the DFS path of each partition.
 struct Layout {
-    uint64_t misc, list, offs, starts, rows, stk, x, scal, lacc, path, total;
+    uint64_t misc, list, offs, starts, keys, rows, stk, x, scal, lacc, path, total;
 };
+constexpr uint32_t PAIR_ROWS = 64;  // largest class whose bitmaps can be built pair by pair
 
 __host__ __device__ inline Layout make_layout(uint32_t rmax, uint32_t wmax, uint32_t levels, uint32_t nparts,
                                               bool pivot, bool local = false)
@@ -118,7 +119,8 @@ __host__ __device__ inline Layout make_layout(uint32_t rmax, uint32_t wmax, uint
     L.list = L.misc + 8;
     L.starts = L.list + (rmax + 1) / 2;  // list and starts are dead once the rows are built
     L.offs = L.starts + (rmax + 1) / 2;
-    L.rows = L.offs + (rmax + 2) / 2;
+    L.keys = L.offs + (rmax + 2) / 2;
+    L.rows = L.keys + (rmax <= PAIR_ROWS ? (rmax + 1) / 2 : 0);
     L.stk = L.rows + (uint64_t)rmax * wmax;
     const uint64_t sets = local ? 4 : 2;  // per level: candidates, branches (+ held, pivots)
     if (pivot) {
@@ -231,14 +233,28 @@ __device__ inline uint32_t lower_bound_u32(const P *a, uint32_t n, uint32_t x)
 
 // ---- step 2: bitmap rows of the induced subgraph on list[0..R) -------------
 // bit j of row i <=> list[j] in N+(list[i]); FULL also sets bit i of row j.
+// Two ways, the cheaper one a task:
+//   entries: stream the members' out-lists (coalesced) and search each entry
+//     in the staged list (LDS), ceil(sum d+/64) rounds of ~8 instructions per
+//     halving of R;
+//   pairs: search each pair's later vertex in the earlier one's out-list
+//     (global, two searches in flight per lane), ceil(R(R-1)/256) rounds, each
+//     priced 60 + 40 per halving of the longest list (25 and 80 a halving
+//     measured the same and 3 to 10% slower).  The orientation's key tells
+//     which of the two holds the edge.
+// Power-law graphs have out-lists much longer than the part of them inside a
+// task (Chung-Lu n=1.2M, edge tasks of at most 64 vertices: 26 members, 1,530
+// entries, 330 pairs): wave time of those tasks 58 -> 33 s at k=5, 68 -> 39 at
+// k=7, and n=500k at k=7 6.0 -> 5.3 ms.  Above 64 vertices the gathers lose
+// (65..128 at k=5: 32 -> 63 s).  keys = null: entries only.
 template <bool FULL>
 __device__ __attribute__((always_inline)) void build_rows(const Cur &g, uint32_t *list, uint32_t *offs,
-                                                         uint32_t *starts, uint64_t *rows, uint32_t R, uint32_t W,
-                                                         uint64_t &bytes)
+                                                         uint32_t *starts, uint32_t *keys, uint64_t *rows, uint32_t R,
+                                                         uint32_t W, uint64_t &bytes)
 {
     const int lane = lane_id();
     for (uint32_t i = lane; i < R * W; i += 64) rows[i] = 0;
-    uint32_t carry = 0;
+    uint32_t carry = 0, longest = 0;
     for (uint32_t base = 0; base < R; base += 64) {
         uint32_t i = base + lane, d = 0;
         if (i < R) {
@@ -246,25 +262,74 @@ __device__ __attribute__((always_inline)) void build_rows(const Cur &g, uint32_t
             uint32_t s = g.rowptr[w];
             d = g.rowptr[w + 1] - s;
             starts[i] = s;
+            if (keys && g.key) keys[i] = g.key[w];
         }
         uint32_t inc = wave_incl_scan32(d);
         if (i < R) offs[i] = carry + inc - d;
-        carry += __shfl(inc, 63, 64);
+        carry += (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+        longest = max(longest, d);
     }
     if (lane == 0) offs[R] = carry;
     __syncthreads();
-    const uint32_t total = carry;
+    const uint32_t total = uni32(carry);
     bytes += 8ull * R + 4ull * total;
-    const uint32_t lo_v = list[0], hi_v = list[R - 1];
-    uint32_t lo = 0;  // row of entry f: the last i with offs[i] <= f (f only grows)
-    for (uint32_t f = lane; f < total; f += 64) {
-        while (offs[lo + 1] <= f) ++lo;
-        uint32_t x = g.col[starts[lo] + (f - offs[lo])];
-        if (x < lo_v || x > hi_v) continue;
-        uint32_t j = lower_bound_u32(list, R, x);
-        if (j < R && list[j] == x) {
-            atomicOr((unsigned long long *)&rows[(uint64_t)lo * W + (j >> 6)], 1ull << (j & 63));
-            if (FULL) atomicOr((unsigned long long *)&rows[(uint64_t)j * W + (lo >> 6)], 1ull << (lo & 63));
+    auto set = [&](uint32_t i, uint32_t j) {
+        atomicOr((unsigned long long *)&rows[(uint64_t)i * W + (j >> 6)], 1ull << (j & 63));
+        if (FULL) atomicOr((unsigned long long *)&rows[(uint64_t)j * W + (i >> 6)], 1ull << (i & 63));
+    };
+    longest = (uint32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_max_u32(longest));
+    const uint32_t npair = R * (R - 1) / 2, depth = 32u - (uint32_t)__clz(longest | 1u);
+    const uint32_t by_pair = ((npair + 127) / 128) * (60 + 40 * depth);
+    const uint32_t by_entry = ((total + 63) / 64) * (16 + 8 * (32u - (uint32_t)__clz(R)));
+    if (keys && g.key && by_pair < by_entry) {
+        // pair f = (i, i + 1 + c mod R) with f = c R + i: every pair once, lanes side by side
+        uint32_t i = lane, c = 0;
+        auto wrap = [&]() {
+            while (i >= R) {
+                i -= R;
+                ++c;
+            }
+        };
+        wrap();
+        for (uint32_t f = lane; f < npair; f += 128) {
+            uint32_t lo[2], hi[2], x[2], n[2], pos[2] = {0, 0};
+            const uint32_t *l[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                uint32_t j = i + 1 + c;
+                j = j >= R ? j - R : j;
+                const uint32_t ki = keys[i], kj = keys[j], vi = list[i], vj = list[j];
+                const bool first = ki < kj || (ki == kj && vi < vj);
+                lo[e] = first ? i : j;
+                hi[e] = first ? j : i;
+                x[e] = first ? vj : vi;
+                const bool in = f + 64 * e < npair;
+                n[e] = in ? offs[lo[e] + 1] - offs[lo[e]] : 0;
+                l[e] = g.col + starts[lo[e]];
+                if (f + 64 * (e + 1) < npair) {  // (i stays a member past the end)
+                    i += 64;
+                    wrap();
+                }
+            }
+            for (uint32_t step = 1u << (depth - 1); step; step >>= 1)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const uint32_t to = pos[e] + step;
+                    if (to <= n[e] && l[e][to - 1] < x[e]) pos[e] = to;
+                }
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+                if (pos[e] < n[e] && l[e][pos[e]] == x[e]) set(lo[e], hi[e]);
+        }
+    } else {
+        const uint32_t lo_v = list[0], hi_v = list[R - 1];
+        uint32_t lo = 0;  // row of entry f: the last i with offs[i] <= f (f only grows)
+        for (uint32_t f = lane; f < total; f += 64) {
+            while (offs[lo + 1] <= f) ++lo;
+            uint32_t x = g.col[starts[lo] + (f - offs[lo])];
+            if (x < lo_v || x > hi_v) continue;
+            uint32_t j = lower_bound_u32(list, R, x);
+            if (j < R && list[j] == x) set(lo, j);
         }
     }
     __syncthreads();
@@ -1654,7 +1719,7 @@ __device__ __attribute__((always_inline)) Cur select_task(const CountArgs &a, ui
         w.q = q;
     }
     const QDesc d = a.qd[q];
-    return Cur{d.rowptr, d.col, d.src, d.k, d.gran, d.psize};
+    return Cur{d.rowptr, d.col, d.src, d.key, d.k, d.gran, d.psize};
 }
 
 __device__ __attribute__((always_inline)) void finish_wave(const CountArgs &a, WaveAcc &w)
@@ -1739,6 +1804,7 @@ void k_pivot_reg(CountArgs a)
     uint32_t *list = reinterpret_cast<uint32_t *>(lds + L.list);
     uint32_t *offs = reinterpret_cast<uint32_t *>(lds + L.offs);
     uint32_t *starts = reinterpret_cast<uint32_t *>(lds + L.starts);
+    uint32_t *keys = reinterpret_cast<uint32_t *>(lds + L.keys);
     uint64_t *rows = lds + L.rows;
     // (S = 4) the two-word rows of a compacted subtree, 128 x 2 words, over
     // list and starts (256 u32 each, dead once the bitmap is built)
@@ -1768,7 +1834,7 @@ void k_pivot_reg(CountArgs a)
                 continue;
             }
             __syncthreads();
-            build_rows<true>(g, list, offs, starts, rows, R, (R + 63) / 64, bytes);
+            build_rows<true>(g, list, offs, starts, S == 1 ? keys : nullptr, rows, R, (R + 63) / 64, bytes);
             if (lane == 0) st[1] += bytes;
             uint64_t nodes = 0;
             add_checked(w.run, pivot_reg<S>(a, g.k, rows, R, g.gran ? 2u : 1u, offs, nodes, w.run_ovf, 0u, crows),
@@ -1966,7 +2032,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) void k_
             uint64_t *dw = reinterpret_cast<uint64_t *>(&d);
 #pragma unroll
             for (int i = 0; i < (int)(sizeof(OpenSlot) / 8); ++i) dw[i] = uni64(rdlane64(word, (uint32_t)i));
-            g = Cur{d.rowptr, d.col, d.src, d.k, d.gran, 1u};
+            g = Cur{d.rowptr, d.col, d.src, nullptr, d.k, d.gran, 1u};
             total = d.total;
             seq = d.seq;
         }
@@ -1979,7 +2045,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) void k_
                 run_add(w, R);
             } else {
                 __syncthreads();
-                build_rows<true>(g, list, offs, starts, rows, R, (R + 63) / 64, w.bytes);
+                build_rows<true>(g, list, offs, starts, nullptr, rows, R, (R + 63) / 64, w.bytes);
                 add_checked(w.run,
                             pivot_reg<1>(a, g.k, rows, R, g.gran ? 2u : 1u, offs, w.nodes, w.run_ovf, 0u, nullptr),
                             w.run_ovf);
@@ -2023,6 +2089,7 @@ __global__ __launch_bounds__(64) void k_count(CountArgs a)
     uint32_t *list = reinterpret_cast<uint32_t *>(ws + L.list);
     uint32_t *offs = reinterpret_cast<uint32_t *>(ws + L.offs);
     uint32_t *starts = reinterpret_cast<uint32_t *>(ws + L.starts);
+    uint32_t *keys = a.rmax <= PAIR_ROWS ? reinterpret_cast<uint32_t *>(ws + L.keys) : nullptr;
     uint64_t *rows = ws + L.rows;
     uint64_t *stk = ws + L.stk;
     uint64_t *X = ws + L.x;
@@ -2061,7 +2128,7 @@ __global__ __launch_bounds__(64) void k_count(CountArgs a)
             uint64_t task_count;
             if (!PIVOT) {
                 // (k-1)-cliques of the DAG on N+(u) / (k-2)-cliques of the DAG on T
-                build_rows<false>(g, list, offs, starts, rows, R, W, w.bytes);
+                build_rows<false>(g, list, offs, starts, keys, rows, R, W, w.bytes);
                 uint32_t povf = 0;
                 uint64_t part = orient_count<LOCAL>(a, g.psize, rows, stk, misc, R, W, g.gran ? k - 2 : k - 1,
                                                     w.nodes, povf, lacc, path);
@@ -2070,7 +2137,7 @@ __global__ __launch_bounds__(64) void k_count(CountArgs a)
                 add_checked(w.run, part, w.run_ovf);
             } else {
                 // SCT rooted at the node (held 1) or the edge (held 2)
-                build_rows<true>(g, list, offs, starts, rows, R, W, w.bytes);
+                build_rows<true>(g, list, offs, starts, keys, rows, R, W, w.bytes);
                 task_count = pivot_count<LOCAL>(a, g.psize, k, rows, stk, X, scal, offs, R, W, g.gran ? 2u : 1u,
                                                 w.nodes, w.run_ovf, lacc);
                 run_add(w, task_count);
@@ -2688,7 +2755,8 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     for (uint32_t i = 0; i < nq; ++i) {
         const kc_oriented *o = qs[i].o;
         const kc_query &q = qs[i].q;
-        hq[i] = QDesc{o->rowptr.as<uint32_t>(), o->col.as<uint32_t>(), o->src.as<uint32_t>(), q.k, q.gran, std::max<uint32_t>(1, qs[i].sample), qs[i].sample > 1 ? qs[i].offset : 0, q.part_size};
+        hq[i] = QDesc{o->rowptr.as<uint32_t>(), o->col.as<uint32_t>(), o->src.as<uint32_t>(),
+                      o->key.as<uint32_t>(), q.k, q.gran, std::max<uint32_t>(1, qs[i].sample), qs[i].sample > 1 ? qs[i].offset : 0, q.part_size};
         halgo[i] = (uint8_t)(q.algo == KC_ALGO_PIVOT);
         hoff[i + 1] = hoff[i] + (q.gran == KC_GRAN_EDGE ? o->m : o->n);
         kmax = std::max(kmax, q.k);
