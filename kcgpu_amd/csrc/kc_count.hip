@@ -911,7 +911,8 @@ __device__ uint32_t tri_lanes(const uint64_t *rows, uint32_t W, const uint64_t (
 // has the registers for it; the one-wave four-word kernel keeps its budget)
 template <int S, bool CL4 = false>
 __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t R, uint32_t h0,
-                              uint32_t *idx, uint64_t &nodes, uint32_t &ovf, uint32_t p0, uint64_t *crows);
+                              uint32_t *idx, uint64_t &nodes, uint32_t &ovf, uint32_t p0, uint64_t *crows, uint32_t wv = 0,
+                              uint32_t nw = 1);
 
 // triangles of G[X] with X in LDS (W words): the lane walks with the words in registers
 template <int S>
@@ -1462,7 +1463,7 @@ __device__ CliqueCounts k34_complement_rows(const uint64_t *rows, uint32_t W, co
 template <int S>
 __device__ uint64_t compact2_and_count(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t W,
                                        const uint64_t (&X)[S], uint32_t *idx, uint64_t *crows, uint32_t h, uint32_t p,
-                                       uint64_t &nodes, uint32_t &ovf)
+                                       uint64_t &nodes, uint32_t &ovf, uint32_t wv, uint32_t nw)
 {
     const uint32_t lane = (uint32_t)lane_id();
     const uint64_t lt = lanemask_lt();
@@ -1492,12 +1493,17 @@ __device__ uint64_t compact2_and_count(const CountArgs &a, uint32_t k, const uin
         }
     }
     sync_tree<true>();
-    return pivot_reg<2>(a, k, crows, cx, h, idx, nodes, ovf, p, nullptr);
+    return pivot_reg<2>(a, k, crows, cx, h, idx, nodes, ovf, p, nullptr, wv, nw);
 }
 
+// nw > 1: this wave is number wv of nw that walk the same subtree, each with
+// its own idx and crows: all of them walk the root's pivot chain (the nodes
+// with h0 held), each takes every nw-th branch off it, and what a chain node
+// itself adds is wave 0's.
 template <int S, bool CL4>
 __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t R, uint32_t h0,
-                              uint32_t *idx, uint64_t &nodes, uint32_t &ovf, uint32_t p0, uint64_t *crows)
+                              uint32_t *idx, uint64_t &nodes, uint32_t &ovf, uint32_t p0, uint64_t *crows, uint32_t wv,
+                              uint32_t nw)
 {
     const uint32_t lane = (uint32_t)lane_id();
     k = uni32(k);
@@ -1540,21 +1546,24 @@ __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *ro
     }
     int t = -1;
     bool pending = true;
-    uint32_t h = h0, p = p0;
+    uint32_t h = h0, p = p0, turn = wv;  // branches off the chain until the next of this wave's
     uint64_t acc = 0, my_nodes = 0;
     for (;;) {
         if (pending) {
             pending = false;
+            const bool chain = h == h0, solo = !chain || wv == 0;
             uint32_t cx = 0;
 #pragma unroll
             for (int w = 0; w < S; ++w) cx += (uint32_t)__popcll(X[w]);
             if (S == 4 && cx > 64 && cx <= 128 && h + 3 <= k && h + p + cx >= k) {
                 // a subtree of at most 128 candidates: two words per row from here on
-                add_checked(acc, compact2_and_count<S>(a, k, rows, W, X, idx, crows, h, p, nodes, ovf), ovf);
+                add_checked(acc, compact2_and_count<S>(a, k, rows, W, X, idx, crows, h, p, nodes, ovf, chain ? wv : 0u,
+                                                          chain ? nw : 1u),
+                            ovf);
             } else if (cx <= 64 && cx > 0 && h + 3 <= k && h + p + cx >= k) {
                 // a subtree of at most 64 candidates: one word per row from here on
-                add_checked(acc, compact_and_count<S>(a, k, rows, W, X, idx, h, p, nodes, ovf), ovf);
-            } else if (++my_nodes, h + p + cx >= k) {
+                if (solo) add_checked(acc, compact_and_count<S>(a, k, rows, W, X, idx, h, p, nodes, ovf), ovf);
+            } else if (my_nodes += solo, h + p + cx >= k) {
                 // scores |X & row_j| of the lane's member rows; key packs
                 // (score + 1, 0xFFFF - j), so the wave max names the smallest j of
                 // the largest score
@@ -1575,6 +1584,7 @@ __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *ro
                 if (need <= 4) e2 = wave_sum32(lsum);
                 const bool near = (S == 2 || (S == 4 && CL4)) && need == 4 && 4 * (uint64_t)e2 >= 3ull * cx * (cx - 1);
                 if (near || need <= 3 || cx == 0) {
+                    if (!solo) break;  // (a chain node that closes ends the chain: the wave's branches are done)
                     // closed forms: h >= k-3, and h = k-4 over a near-clique (complement
                     // density <= 1/4)
                     const CloseTerm term(a, need, p);
@@ -1622,6 +1632,11 @@ __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *ro
         for (int w = 0; w < S; ++w) X[w] = Cc[w] & lds_row_word(rows, W, b, w);
         h = hh + (b != pv ? 1u : 0u);
         p = pp + (b == pv ? 1u : 0u);
+        bool mine = true;
+        if (nw > 1 && hh == h0 && !last) {
+            mine = turn == 0;
+            turn = mine ? nw - 1 : turn - 1;
+        }
         if (last) {
             --t;  // the pivot branch replaces its level
         } else {
@@ -1635,7 +1650,7 @@ __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *ro
                 stkB[w] = (lane == (uint32_t)t) ? B[w] : stkB[w];
             }
         }
-        if (h <= k) pending = true;
+        if (h <= k) pending = mine;
     }
     if (lane == 0) nodes += my_nodes;
     return acc;
@@ -2230,6 +2245,100 @@ __device__ void build_rows_block(const Cur &g, const uint32_t *list, uint32_t *o
         }
     }
     __syncthreads();
+}
+
+// Tasks of 129..256 vertices, one block of NW waves each: the waves build the
+// bitmap together, share it in LDS and split the SCT by the branches off its
+// root chain (pivot_reg).  For launches that are over with their longest task
+// (at most BLOCK_TASKS_PER_CU tasks per CU, what the one-wave kernel holds at
+// once): 2,825 node tasks of an R-MAT graph at k=5, 3.6 -> 3.2 ms with two
+// waves, 3.5 with four (each walks the chain again).  With many tasks the
+// second walk of the chain only costs (37,889 edge tasks of Chung-Lu n=1.2M
+// at k=5..8: 242 -> 254 ms in all with two waves, 280 with four).
+constexpr uint32_t BLOCK_WAVES = 2, BLOCK_TASKS_PER_CU = 14;
+
+struct BlockLayout {
+    uint64_t st, ctl, list, starts, offs, rows, wave, per_wave, total;
+};
+
+__host__ __device__ inline BlockLayout make_block_layout(uint32_t nw)
+{
+    BlockLayout L;
+    L.st = 0;
+    L.ctl = 8;
+    L.list = L.ctl + 2;
+    L.starts = L.list + 128;
+    L.offs = L.starts + 128;
+    L.rows = L.offs + 129;
+    L.wave = L.rows + 256 * 4;
+    L.per_wave = 128 + 256;  // member list (256 u32), two-word rows of a compacted subtree (128 x 2)
+    L.total = L.wave + L.per_wave * nw;
+    return L;
+}
+
+template <int NW>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) void k_pivot_block(CountArgs a)
+{
+    extern __shared__ uint64_t lds[];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wv = uni32(tid >> 6);
+    const BlockLayout L = make_block_layout(NW);
+    uint64_t *st = lds + L.st;  // launch statistics (as acc, [6] the task's start)
+    uint32_t *ctl = reinterpret_cast<uint32_t *>(lds + L.ctl);
+    uint32_t *list = reinterpret_cast<uint32_t *>(lds + L.list);
+    uint32_t *starts = reinterpret_cast<uint32_t *>(lds + L.starts);
+    uint32_t *offs = reinterpret_cast<uint32_t *>(lds + L.offs);
+    uint64_t *rows = lds + L.rows;
+    uint32_t *idx = reinterpret_cast<uint32_t *>(lds + L.wave + wv * L.per_wave);
+    uint64_t *crows = lds + L.wave + wv * L.per_wave + 128;
+    if (tid < 8) st[tid] = 0;
+    WaveAcc w;
+    TaskQueue tq(blockIdx.x);
+    for (;;) {
+        if (wv == 0) {
+            const uint32_t start = next_tasks(a, tq);
+            if (lane == 0) ctl[0] = start;
+        }
+        __syncthreads();
+        const uint32_t ti = uni32(ctl[0]);
+        if (ti == INF32) break;
+        uint32_t task;
+        const Cur g = select_task(a, a.tasks[ti], w, task);
+        uint64_t bytes = 0;
+        if (wv == 0) {
+            if (lane == 0) st[6] = wall_clock64();
+            const uint32_t r = stage_task(g, task, list, bytes);
+            if (lane == 0) ctl[1] = r;
+        }
+        __syncthreads();
+        const uint32_t R = uni32(ctl[1]);
+        if (g.gran && g.k == 3) {  // an edge task at k=3 adds |T| (no bitmap needed)
+            if (wv == 0) run_add(w, R);
+        } else {
+            build_rows_block(g, list, offs, starts, rows, R, (R + 63) / 64, bytes);
+            uint64_t nodes = 0;
+            add_checked(w.run, pivot_reg<4>(a, g.k, rows, R, g.gran ? 2u : 1u, idx, nodes, w.run_ovf, 0u, crows, wv, NW),
+                        w.run_ovf);
+            if (lane == 0) atomicAdd((unsigned long long *)&st[3], (unsigned long long)nodes);
+        }
+        __syncthreads();
+        if (tid == 0) {
+            st[1] += bytes;
+            ++st[2];
+            if (!(g.gran && g.k == 3)) {
+                const uint64_t dt = wall_clock64() - st[6];
+                st[4] = dt > st[4] ? dt : st[4];
+                st[5] += dt * NW;
+            }
+        }
+    }
+    if (wv == 0) {
+        w.bytes = st[1];
+        w.ntask = st[2];
+        w.nodes = lane == 0 ? st[3] : 0;
+        w.tmax = st[4];
+        w.tsum = st[5];
+    }
+    finish_wave(a, w);
 }
 
 template <bool GLOBAL>
@@ -2914,6 +3023,14 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     const char *fan_env = std::getenv("KC_SIDE_BY_SIDE");
     const bool fan_rule = reg_tasks < FAN_MAX_TASKS_PER_CU * (uint64_t)ctx->cu;
     const bool fan = evs.on && grid_share == 1 && (fan_env && *fan_env ? *fan_env == '1' : fan_rule);
+    // With at most one large task per CU the wide launches are on the device
+    // whole from the start and the small classes take the CUs they leave (R-MAT
+    // scale 17, node tasks at k=5: 187 large tasks, 1.5 ms before the rest, 4.8
+    // -> 4.0 ms).
+    uint64_t wide_tasks = 0;
+    for (int b = 0; b < NB; ++b)
+        if (b % NCLASS > 2) wide_tasks += bcnt[b];
+    const bool few_wide = wide_tasks <= (uint64_t)ctx->cu;
     bool side_waits[DeviceCtx::NSIDE] = {false}, fan_recorded = false;
     hipStream_t bin_stream[NB];
     int nside = 0;
@@ -2968,8 +3085,13 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
             L = make_layout(a.rmax, a.wmax, 0, 0, true);
             variant[b] = 2u;
         }
-        // large tasks of pivoting: blocks of several waves sharing one bitmap
         uint32_t nw = 1;
+        if (pivot && !global && c == 2 && !lc && bcnt[b] <= (uint32_t)ctx->cu * BLOCK_TASKS_PER_CU) {
+            kern = reinterpret_cast<const void *>(&k_pivot_block<BLOCK_WAVES>);
+            nw = BLOCK_WAVES;
+            L.total = make_block_layout(nw).total;
+        }
+        // large tasks of pivoting: blocks of several waves sharing one bitmap
         WideLayout WL{};
         if (pivot && !lc && c >= 3) {
             // chain levels walked by wave 0 before the entries are shared: the
@@ -3031,14 +3153,14 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         }
         hipStream_t st = s;
         if (fan && !global && c <= 2) {
-            if (!fan_recorded) {
+            if (!fan_recorded && !few_wide) {
                 KC_HIP_L(hipEventRecord(evs.fan, s));  // after every launch so far on s
                 fan_recorded = true;
             }
             const int si = nside++ % DeviceCtx::NSIDE;
             st = ctx->side[si];
             if (!side_waits[si]) {
-                KC_HIP_L(hipStreamWaitEvent(st, evs.fan, 0));
+                KC_HIP_L(hipStreamWaitEvent(st, few_wide ? evs.go : evs.fan, 0));
                 side_waits[si] = true;
             }
         }
