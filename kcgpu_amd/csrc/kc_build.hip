@@ -5,8 +5,8 @@
 // plus the reference's optional std::sort (include/FIleReader.cuh:314-320).
 //
 // Steps: degree histogram (both endpoints of every non-loop edge), exclusive
-// scan into row offsets, scatter of both directions through per-row atomic
-// cursors (unordered within a row), a per-row sort that also removes
+// scan into row offsets, scatter of both directions to the places the
+// histogram's atomics gave (unordered within a row), a per-row sort that also removes
 // duplicates, a scan of the unique counts and a compaction into the final
 // CSR.  Rows of at most SMALL_ROW entries are sorted by one wave each with a
 // bitonic network in LDS; longer rows (hubs of power-law graphs, up to
@@ -41,33 +41,46 @@ __global__ __launch_bounds__(BUILD_T) void k_edge_max(const uint32_t *s, const u
         a = 1;
         m = max(m, max(u, v));
     }
+    // one atomic pair per block (one per wave on the two words took 0.38 ms, so 0.10)
+    __shared__ uint32_t bm, ba;
+    if (threadIdx.x == 0) bm = ba = 0;
+    __syncthreads();
     m = build_wave_max(m);
     a = build_wave_max(a);
     if ((threadIdx.x & 63) == 0) {
-        if (a) atomicOr(any, 1u);
-        atomicMax(mx, m);
+        atomicMax(&bm, m);
+        atomicMax(&ba, a);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && ba) {
+        atomicOr(any, 1u);
+        atomicMax(mx, bm);
     }
 }
 
+// The degree histogram's atomics hand every edge end its place in its row,
+// which the scatter then needs no atomic for (2.3 M edges of an R-MAT graph:
+// two passes of atomics, 1.01 ms each -> 1.01 + 0.05).
 __global__ __launch_bounds__(BUILD_T) void k_edge_degree(const uint32_t *s, const uint32_t *d, uint64_t ne,
-                                                         uint32_t *deg)
+                                                         uint32_t *deg, uint2 *rank)
 {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < ne; i += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t u = s[i], v = d[i];
         if (u == v) continue;
-        atomicAdd(&deg[u], 1u);
-        atomicAdd(&deg[v], 1u);
+        const uint32_t ru = atomicAdd(&deg[u], 1u), rv = atomicAdd(&deg[v], 1u);
+        rank[i] = make_uint2(ru, rv);
     }
 }
 
 __global__ __launch_bounds__(BUILD_T) void k_edge_scatter(const uint32_t *s, const uint32_t *d, uint64_t ne,
-                                                          uint32_t *cursor, uint32_t *tmp)
+                                                          const uint32_t *off, const uint2 *rank, uint32_t *tmp)
 {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < ne; i += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t u = s[i], v = d[i];
         if (u == v) continue;
-        tmp[atomicAdd(&cursor[u], 1u)] = v;
-        tmp[atomicAdd(&cursor[v], 1u)] = u;
+        const uint2 r = rank[i];
+        tmp[off[u] + r.x] = v;
+        tmp[off[v] + r.y] = u;
     }
 }
 
@@ -82,8 +95,14 @@ __global__ __launch_bounds__(BUILD_T) void k_row_sort_small(const uint32_t *off,
     const uint32_t lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     const uint64_t lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
     uint32_t *a = buf[wv];
-    const uint32_t nwave = gridDim.x * (BUILD_T / 64);
-    for (uint32_t r = blockIdx.x * (BUILD_T / 64) + wv; r < n; r += nwave) {
+    // a wave's rows are a step of nwave apart, turned a little further each time:
+    // the long rows of an R-MAT graph have ids with few bits set, and without
+    // the turn one wave sorted all those at multiples of nwave (1.9 ms -> 0.7)
+    const uint32_t nwave = gridDim.x * (BUILD_T / 64), me = blockIdx.x * (BUILD_T / 64) + wv;
+    for (uint64_t r0 = 0, turn = 0; r0 < n; r0 += nwave, turn += 977) {
+        const uint64_t rr = r0 + (me + turn) % nwave;
+        if (rr >= n) continue;
+        const uint32_t r = (uint32_t)rr;
         const uint32_t b = off[r], dn = off[r + 1] - b;
         if (dn > SMALL_ROW) {
             if (lane == 0) big[atomicAdd(nbig, 1u)] = r;
@@ -189,16 +208,28 @@ __global__ __launch_bounds__(BUILD_T) void k_row_compact(const uint32_t *off, co
     const uint32_t nwave = gridDim.x * (BUILD_T / 64);
     for (uint32_t r = blockIdx.x * (BUILD_T / 64) + (threadIdx.x >> 6); r < n; r += nwave) {
         const uint32_t b = off[r], o = rowptr[r], c = rowptr[r + 1] - o;
-        for (uint32_t i = lane; i < c; i += 64) col[o + i] = tmp[b + i];
+        for (uint32_t i = lane; i < c; i += 64 * 8) {  // (eight steps in flight, for the hubs)
+            uint32_t v[8];
+#pragma unroll
+            for (int t = 0; t < 8; ++t) v[t] = i + 64 * t < c ? tmp[b + i + 64 * t] : 0u;
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+                if (i + 64 * t < c) col[o + i + 64 * t] = v[t];
+        }
     }
 }
 
 __global__ __launch_bounds__(BUILD_T) void k_build_max(const uint32_t *a, uint32_t n, uint32_t *out)
 {
+    __shared__ uint32_t bm;
+    if (threadIdx.x == 0) bm = 0;
+    __syncthreads();
     uint32_t m = 0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) m = max(m, a[i]);
+    for (uint64_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) m = max(m, a[i]);
     m = build_wave_max(m);
-    if ((threadIdx.x & 63) == 0) atomicMax(out, m);
+    if ((threadIdx.x & 63) == 0) atomicMax(&bm, m);
+    __syncthreads();
+    if (threadIdx.x == 0) atomicMax(out, bm);
 }
 
 __global__ void k_build_fill(uint32_t *a, uint64_t n, uint32_t v)
@@ -234,20 +265,20 @@ int build_csr_device(DeviceCtx *ctx, hipStream_t s, uint32_t n_in, size_t ne, co
     if (h[1] && h[0] >= nn) return fail(KC_ERR_ARG, "vertex id %u >= n=%llu", h[0], (unsigned long long)nn);
     if (nn >= 0xFFFFFFFFull) return fail(KC_ERR_LIMIT, "n=%llu does not fit 32-bit ids", (unsigned long long)nn);
     const uint32_t n = (uint32_t)nn;
-    DevBuf deg, off, cur, tmp, ucnt, big, scan_tmp;
+    DevBuf deg, off, rank, tmp, ucnt, big, scan_tmp;
     if ((rc = deg.ensure(4 * ((size_t)n + 1))) || (rc = off.ensure(4 * ((size_t)n + 1))) ||
-        (rc = cur.ensure(4 * ((size_t)n + 1))) || (rc = tmp.ensure(8 * ne + 4)) ||
+        (rc = rank.ensure(8 * ne + 8)) || (rc = tmp.ensure(8 * ne + 4)) ||
         (rc = ucnt.ensure(4 * ((size_t)n + 1))) || (rc = big.ensure(4 * ((size_t)n + 1))) ||
         (rc = rowptr.ensure(4 * ((size_t)n + 1))))
         return rc;
     const int gn = (int)std::max<uint64_t>(1, std::min<uint64_t>(((uint64_t)n + BUILD_T - 1) / BUILD_T, (uint64_t)ctx->cu * 16));
     hipLaunchKernelGGL(k_build_fill, dim3(gn), dim3(BUILD_T), 0, s, deg.as<uint32_t>(), (uint64_t)n + 1, 0u);
-    if (ne) hipLaunchKernelGGL(k_edge_degree, dim3(ge), dim3(BUILD_T), 0, s, S, D, (uint64_t)ne, deg.as<uint32_t>());
+    if (ne) hipLaunchKernelGGL(k_edge_degree, dim3(ge), dim3(BUILD_T), 0, s, S, D, (uint64_t)ne, deg.as<uint32_t>(),
+                               rank.as<uint2>());
     KC_HIP(hipGetLastError());
     if ((rc = scan_exclusive_u32(deg.as<uint32_t>(), off.as<uint32_t>(), n, scan_tmp, s))) return rc;
-    KC_HIP(hipMemcpyAsync(cur.p, off.p, 4 * (size_t)n, hipMemcpyDeviceToDevice, s));
-    if (ne) hipLaunchKernelGGL(k_edge_scatter, dim3(ge), dim3(BUILD_T), 0, s, S, D, (uint64_t)ne, cur.as<uint32_t>(),
-                               tmp.as<uint32_t>());
+    if (ne) hipLaunchKernelGGL(k_edge_scatter, dim3(ge), dim3(BUILD_T), 0, s, S, D, (uint64_t)ne, off.as<uint32_t>(),
+                               rank.as<uint2>(), tmp.as<uint32_t>());
     // rows: distinct sorted values at each row's start, counts in ucnt
     const int gw = (int)std::max<uint64_t>(1, std::min<uint64_t>(((uint64_t)n + 3) / 4, (uint64_t)ctx->cu * 8));
     if (n) hipLaunchKernelGGL(k_row_sort_small, dim3(gw), dim3(BUILD_T), 0, s, off.as<uint32_t>(), n,

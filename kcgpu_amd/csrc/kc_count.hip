@@ -2686,8 +2686,10 @@ __device__ inline void binom_rows(const BinArgs &b, uint32_t nmax)
             ovf[(uint64_t)n * b.bstride + r] = (uint8_t)o;
         }
         if (n == nmax) break;
-        const uint64_t w = __shfl_up(v, 1u, 64);
-        const uint32_t ow = __shfl_up(o, 1u, 64);
+        // (the lane below's values: a wave shift in the ALU, not a trip through LDS, a row)
+        auto below = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x138, 0xf, 0xf, false); };
+        const uint64_t w = ((uint64_t)below((uint32_t)(v >> 32)) << 32) | below((uint32_t)v);
+        const uint32_t ow = below(o);
         if (r > 0) {
             const uint64_t sum = v + w;
             o |= ow | (sum < v ? 1u : 0u);

@@ -238,7 +238,13 @@ __device__ inline uint32_t vkey(const uint32_t *rowptr, const uint32_t *key, uin
     return rowptr[v + 1] - rowptr[v];
 }
 
-// one wave per row: out-degree after orientation; also records the key
+// One wave per row, eight steps of 64 entries in flight: a step is a load of
+// the neighbours and one of their keys, and a hub's row of 25,000 entries, one
+// step at a time, was the whole time of both kernels (R-MAT scale 17: 0.36 and
+// 0.38 ms -> 0.23 and 0.24).
+constexpr int ROW_U = 8;
+
+// out-degree after orientation; also records the key
 template <bool DEGEN>
 __global__ __launch_bounds__(256) void k_orient_count(uint32_t n, const uint32_t *rowptr, const uint32_t *col,
                                                        uint32_t *key, uint32_t *outdeg)
@@ -247,16 +253,18 @@ __global__ __launch_bounds__(256) void k_orient_count(uint32_t n, const uint32_t
     uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) >> 6;
     for (uint64_t u = wave; u < n; u += nw) {
-        uint32_t b = rowptr[u], e = rowptr[u + 1];
-        uint32_t ku = DEGEN ? key[u] : e - b;
+        const uint32_t b = rowptr[u], e = rowptr[u + 1];
+        const uint32_t ku = DEGEN ? key[u] : e - b;
         uint32_t cnt = 0;
-        for (uint32_t i = b; i < e; i += 64) {
-            bool k = false;
-            if (i + lane < e) {
-                uint32_t v = col[i + lane];
-                k = keep_edge(ku, (uint32_t)u, vkey<DEGEN>(rowptr, key, v), v);
-            }
-            cnt += (uint32_t)__popcll(__ballot(k));
+        for (uint64_t i = b; i < e; i += 64 * ROW_U) {
+            uint32_t v[ROW_U], kv[ROW_U];
+#pragma unroll
+            for (int t = 0; t < ROW_U; ++t) v[t] = i + 64 * t + lane < e ? col[i + 64 * t + lane] : 0u;
+#pragma unroll
+            for (int t = 0; t < ROW_U; ++t) kv[t] = i + 64 * t + lane < e ? vkey<DEGEN>(rowptr, key, v[t]) : 0u;
+#pragma unroll
+            for (int t = 0; t < ROW_U; ++t)
+                cnt += (uint32_t)__popcll(__ballot(i + 64 * t + lane < e && keep_edge(ku, (uint32_t)u, kv[t], v[t])));
         }
         if (lane == 0) {
             outdeg[u] = cnt;
@@ -265,7 +273,7 @@ __global__ __launch_bounds__(256) void k_orient_count(uint32_t n, const uint32_t
     }
 }
 
-// one wave per row: stable write of kept entries at ballot-prefix ranks
+// stable write of kept entries at ballot-prefix ranks
 template <bool DEGEN>
 __global__ __launch_bounds__(256) void k_orient_write(uint32_t n, const uint32_t *rowptr, const uint32_t *col,
                                                        const uint32_t *key, const uint32_t *orowptr,
@@ -276,34 +284,43 @@ __global__ __launch_bounds__(256) void k_orient_write(uint32_t n, const uint32_t
     uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) >> 6;
     for (uint64_t u = wave; u < n; u += nw) {
-        uint32_t b = rowptr[u], e = rowptr[u + 1];
-        uint32_t ku = DEGEN ? key[u] : e - b;
+        const uint32_t b = rowptr[u], e = rowptr[u + 1];
+        const uint32_t ku = DEGEN ? key[u] : e - b;
         uint32_t w = orowptr[u];
-        for (uint32_t i = b; i < e; i += 64) {
-            bool k = false;
-            uint32_t v = 0;
-            if (i + lane < e) {
-                v = col[i + lane];
-                k = keep_edge(ku, (uint32_t)u, vkey<DEGEN>(rowptr, key, v), v);
+        for (uint64_t i = b; i < e; i += 64 * ROW_U) {
+            uint32_t v[ROW_U], kv[ROW_U];
+#pragma unroll
+            for (int t = 0; t < ROW_U; ++t) v[t] = i + 64 * t + lane < e ? col[i + 64 * t + lane] : 0u;
+#pragma unroll
+            for (int t = 0; t < ROW_U; ++t) kv[t] = i + 64 * t + lane < e ? vkey<DEGEN>(rowptr, key, v[t]) : 0u;
+#pragma unroll
+            for (int t = 0; t < ROW_U; ++t) {
+                const bool k = i + 64 * t + lane < e && keep_edge(ku, (uint32_t)u, kv[t], v[t]);
+                const uint64_t bal = __ballot(k);
+                if (k) {
+                    const uint32_t r = w + (uint32_t)__popcll(bal & lt);
+                    ocol[r] = v[t];
+                    osrc[r] = (uint32_t)u;
+                }
+                w += (uint32_t)__popcll(bal);
             }
-            uint64_t bal = __ballot(k);
-            if (k) {
-                uint32_t r = w + (uint32_t)__popcll(bal & lt);
-                ocol[r] = v;
-                osrc[r] = (uint32_t)u;
-            }
-            w += (uint32_t)__popcll(bal);
         }
     }
 }
 
-__global__ void k_max_u32(const uint32_t *a, uint32_t n, uint32_t *out)
+// one atomic per block (one per wave of 1,024 blocks on the one word took 47 us, this 4)
+__global__ __launch_bounds__(256) void k_max_u32(const uint32_t *a, uint32_t n, uint32_t *out)
 {
+    __shared__ uint32_t best;
+    if (threadIdx.x == 0) best = 0;
+    __syncthreads();
     uint32_t m = 0;
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
         m = max(m, a[i]);
     for (int d = 32; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor(m, d, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax(out, m);
+    if ((threadIdx.x & 63) == 0) atomicMax(&best, m);
+    __syncthreads();
+    if (threadIdx.x == 0) atomicMax(out, best);
 }
 
 // ---------------------------------------------------------------------------
@@ -526,8 +543,8 @@ __global__ __launch_bounds__(256) void k_peel(PeelArgs a)
 }
 
 // ---------------------------------------------------------------------------
-// The same peel as ordinary launches (the default path; it also serves
-// processes that cannot get a cooperative launch).  A one-thread control
+// The same peel as ordinary launches (on request, and when the blocks of
+// k_peel_run below found no room on the device together).  A one-thread control
 // kernel keeps the state machine that k_peel keeps in registers; the host
 // enqueues steps of five kernels in batches and reads the phase once per
 // batch.  Kernels of a step that has nothing to do return at once, so a
@@ -651,13 +668,227 @@ __global__ void k_peel_ctl_round(PeelCtl *ctl, uint32_t *cnt, uint32_t maxdeg)
     ctl->phase = 0;
 }
 
+// ---------------------------------------------------------------------------
+// The same peel in one launch of a few resident blocks with a barrier of
+// their own (the default).  A round is a handful of dependent memory accesses
+// over a small frontier, a level adds a pass over the live vertices, and both
+// are shorter than the five launches of a step (Chung-Lu n=700,000, 913 rounds:
+// the orientation 17.2 -> 10.3 ms): what bounds it is the latency of a round, so each phase ends in one
+// barrier and nothing else.
+//   * A vertex is live exactly while deg > level, and a frontier vertex has
+//     deg <= level, so no state array is needed: a decrement of a dead or
+//     frontier vertex changes nothing that is read again (every neighbour
+//     decrements once, so no degree goes below 0).  Looking first, to spare
+//     those atomics, costs one more trip to memory a round (13.0 against 10.5
+//     ms), more blocks cost longer barriers (128: 10.5, 64: 10.3, 32: no gain).
+//   * Short rows go eight lanes each, rows up to HUB a wave each, longer ones
+//     to all waves together.
+//   * The gather of a level reads a list of the vertices live when it was last
+//     rebuilt (at a quarter of its size), and finds the lowest live degree, so
+//     empty levels are skipped.
+// Every cross-block value is accessed with device-scope atomics (loads and
+// stores past the L1 and the XCD's L2), so a barrier only waits for this
+// thread's own accesses.  Counters that all blocks read after a barrier sit in
+// three slots taken in turn; a slot is cleared one phase before it is filled.
+// A wait is bounded: when the other blocks do not arrive (the device holds
+// no room for them) every block leaves and the host steps the peel.
+// ---------------------------------------------------------------------------
+struct PeelShared {
+    unsigned long long arrive;
+    uint32_t abort, max_core, done, pad;
+    uint32_t cnt[3][4];   // frontier: short rows, middle rows, hubs
+    uint32_t live[3][2];  // vertices of the rebuilt list; ~(lowest live degree above the level)
+};
+
+struct PeelRunArgs {
+    uint32_t n;
+    const uint32_t *rowptr, *col;
+    uint32_t *deg, *prio;
+    uint32_t *q[2];     // n each: short rows from the front, middle rows from the back
+    uint32_t *hubs[2];
+    uint32_t *list[2];  // n/4, n/16
+    PeelShared *s;
+    uint64_t wait_ticks;
+};
+
+constexpr uint32_t PEEL_SHORT = 64, PEEL_HUB = 4096;
+constexpr int PEEL_BLOCKS = 64, PEEL_T = 256;
+
+__device__ inline uint32_t ld_dev(const uint32_t *p)
+{
+    return __hip_atomic_load(const_cast<uint32_t *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void st_dev(uint32_t *p, uint32_t v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// add the lanes' vertices to a list (device-scope stores); from: 0 front, else entries go down from it
+__device__ inline void peel_append(bool take, uint32_t v, uint32_t *q, uint32_t *cnt, uint32_t from)
+{
+    const int lane = threadIdx.x & 63;
+    const uint64_t bal = __ballot(take);
+    if (!bal) return;
+    const int leader = __ffsll((unsigned long long)bal) - 1;
+    uint32_t base = 0;
+    if (lane == leader) base = atomicAdd(cnt, (uint32_t)__popcll(bal));
+    base = __shfl(base, leader, 64);
+    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+    const uint32_t at = base + (uint32_t)__popcll(bal & lt);
+    if (take) st_dev(q + (from ? from - 1 - at : at), v);
+}
+
+__device__ inline void peel_push(const PeelRunArgs &a, bool take, uint32_t v, int buf, uint32_t *cnt)
+{
+    if (!__ballot(take)) return;
+    const uint32_t len = take ? a.rowptr[v + 1] - a.rowptr[v] : 0;
+    peel_append(take && len <= PEEL_SHORT, v, a.q[buf], cnt, 0);
+    peel_append(take && len > PEEL_SHORT && len <= PEEL_HUB, v, a.q[buf], cnt + 1, a.n);
+    peel_append(take && len > PEEL_HUB, v, a.hubs[buf], cnt + 2, 0);
+}
+
+// the neighbours at col[j], j from b on by step below e, U at a time: decrement them, push those that
+// join the level
+template <int U>
+__device__ inline void peel_row(const PeelRunArgs &a, uint32_t level, uint32_t b, uint32_t e, uint32_t step, int buf,
+                                uint32_t *cnt)
+{
+    for (uint64_t j = b; __ballot(j < e); j += (uint64_t)U * step) {
+        uint32_t x[U], old[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint64_t at = j + (uint64_t)u * step;
+            x[u] = at < e ? a.col[at] : 0xFFFFFFFFu;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) old[u] = x[u] != 0xFFFFFFFFu ? atomicSub(a.deg + x[u], 1u) : 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) peel_push(a, old[u] == level + 1, x[u], buf, cnt);
+    }
+}
+
+__global__ __launch_bounds__(PEEL_T) void k_peel_run(PeelRunArgs a)
+{
+    __shared__ uint32_t ok, low;
+    const uint32_t lane = threadIdx.x & 63, tid = blockIdx.x * PEEL_T + threadIdx.x, nthr = gridDim.x * PEEL_T;
+    const uint32_t wave = tid >> 6, nwave = nthr >> 6;
+    PeelShared *s = a.s;
+    unsigned long long target = 0;
+    auto barrier = [&]() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_s_waitcnt(0);  // this thread's stores and atomics are done
+        __syncthreads();
+        target += gridDim.x;
+        if (threadIdx.x == 0) {
+            __hip_atomic_fetch_add(&s->arrive, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const uint64_t t0 = wall_clock64();
+            uint32_t fine = 1;
+            while (__hip_atomic_load(&s->arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
+                if (wall_clock64() - t0 > a.wait_ticks || ld_dev(&s->abort)) {
+                    st_dev(&s->abort, 1u);
+                    fine = 0;
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+            ok = fine;
+        }
+        __syncthreads();
+        const bool r = ok != 0;
+        __syncthreads();  // (ok is written again by the next barrier)
+        return r;
+    };
+    uint32_t level = 0, round = 0, todo = a.n, m = a.n;
+    const uint32_t *list = nullptr;  // null: every vertex
+    int nlist = 0;
+    for (uint32_t r = 0, g = 0;; ++r, ++g) {
+        // gather the live vertices of degree `level` into slot r; slot r + 1 is the next round's
+        uint32_t *cnt = s->cnt[r % 3];
+        if (tid < 4) st_dev(&s->cnt[(r + 1) % 3][tid], 0u);
+        if (tid < 2) st_dev(&s->live[(g + 1) % 3][tid], 0u);
+        const bool rebuild = todo <= m / 4 && m >= 1024;
+        uint32_t *to = a.list[nlist & 1];
+        uint32_t lowest = 0xFFFFFFFFu;
+        if (threadIdx.x == 0) low = 0xFFFFFFFFu;
+        __syncthreads();
+        for (uint64_t i = tid; __ballot(i < m); i += nthr) {
+            const uint32_t v = i >= m ? 0u : list ? ld_dev(list + i) : (uint32_t)i;
+            const uint32_t d = i < m ? ld_dev(a.deg + v) : 0;
+            const bool in = i < m && d >= level;
+            peel_push(a, in && d == level, v, (int)(r & 1), cnt);
+            if (in && d > level) lowest = min(lowest, d);
+            if (rebuild) peel_append(in, v, to, &s->live[g % 3][0], 0);
+        }
+        for (int d = 32; d >= 1; d >>= 1) lowest = min(lowest, (uint32_t)__shfl_xor(lowest, d, 64));
+        if (lane == 0 && lowest != 0xFFFFFFFFu) atomicMin(&low, lowest);
+        __syncthreads();
+        if (threadIdx.x == 0 && low != 0xFFFFFFFFu) atomicMax(&s->live[g % 3][1], ~low);
+        if (!barrier()) return;
+        if (rebuild) {
+            m = ld_dev(&s->live[g % 3][0]);
+            list = to;
+            ++nlist;
+        }
+        uint32_t ns = ld_dev(cnt), nm = ld_dev(cnt + 1), nh = ld_dev(cnt + 2);
+        if (ns + nm + nh == 0) {  // an empty level: on to the lowest live degree
+            const uint32_t lo = ld_dev(&s->live[g % 3][1]);
+            if (lo == 0) return;  // (live vertices left, none seen: cannot be; done stays 0)
+            level = ~lo;
+            continue;
+        }
+        for (;;) {
+            todo -= ns + nm + nh;
+            if (todo == 0) {  // the round that empties the graph assigns nothing
+                if (tid == 0) {
+                    st_dev(&s->max_core, level);
+                    st_dev(&s->done, 1u);
+                }
+                return;
+            }
+            const int cur = (int)(r & 1), nxt = cur ^ 1;
+            uint32_t *ncnt = s->cnt[(r + 1) % 3];
+            if (tid < 4) st_dev(&s->cnt[(r + 2) % 3][tid], 0u);
+            for (uint32_t i = wave * 8; i < ns; i += nwave * 8) {
+                const uint32_t k = i + (lane >> 3);
+                uint32_t b = 0, e = 0;
+                if (k < ns) {
+                    const uint32_t v = ld_dev(a.q[cur] + k);
+                    b = a.rowptr[v];
+                    e = a.rowptr[v + 1];
+                    if ((lane & 7) == 0) a.prio[v] = round;
+                }
+                peel_row<2>(a, level, b + (lane & 7), e, 8, nxt, ncnt);
+            }
+            for (uint32_t i = wave; i < nm; i += nwave) {
+                const uint32_t v = ld_dev(a.q[cur] + (a.n - 1 - i)), b = a.rowptr[v], e = a.rowptr[v + 1];
+                if (lane == 0) a.prio[v] = round;
+                peel_row<4>(a, level, b + lane, e, 64, nxt, ncnt);
+            }
+            for (uint32_t i = 0; i < nh; ++i) {
+                const uint32_t v = ld_dev(a.hubs[cur] + i), b = a.rowptr[v], e = a.rowptr[v + 1];
+                if (tid == 0) a.prio[v] = round;
+                peel_row<1>(a, level, b + wave * 64 + lane, e, nwave * 64, nxt, ncnt);
+            }
+            if (!barrier()) return;
+            ++r;
+            ++round;
+            cnt = s->cnt[r % 3];
+            ns = ld_dev(cnt);
+            nm = ld_dev(cnt + 1);
+            nh = ld_dev(cnt + 2);
+            if (ns + nm + nh == 0) break;
+        }
+        ++level;
+    }
+}
+
 __global__ void k_peel_init(uint32_t n, const uint32_t *rowptr, int *deg, uint32_t *prio, uint8_t *state,
                             uint32_t nnz)
 {
     for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (uint64_t)gridDim.x * blockDim.x) {
         deg[v] = (int)(rowptr[v + 1] - rowptr[v]);
         prio[v] = nnz;
-        state[v] = 0;
+        if (state) state[v] = 0;
     }
 }
 
@@ -696,10 +927,48 @@ static int run_peel(DeviceCtx *ctx, hipStream_t s, uint32_t n, uint32_t nnz, uin
 {
     DevBuf deg, st, q0, q1, cnt;
     int rc;
-    if ((rc = deg.ensure(sizeof(int) * (size_t)n + 4)) || (rc = st.ensure((size_t)n + 4)) ||
-        (rc = q0.ensure(sizeof(uint32_t) * (size_t)n + 4)) || (rc = q1.ensure(sizeof(uint32_t) * (size_t)n + 4)) ||
-        (rc = cnt.ensure(sizeof(uint32_t) * 4)))
+    if ((rc = deg.ensure(sizeof(int) * (size_t)n + 4)) || (rc = q0.ensure(sizeof(uint32_t) * (size_t)n + 4)) ||
+        (rc = q1.ensure(sizeof(uint32_t) * (size_t)n + 4)) || (rc = cnt.ensure(sizeof(uint32_t) * 4)))
         return rc;
+    // KC_PEEL_MODE=coop selects the cooperative kernel, =step the stepped launches
+    const char *mode = std::getenv("KC_PEEL_MODE");
+    bool coop = mode && std::strcmp(mode, "coop") == 0;
+    if (!coop && !(mode && std::strcmp(mode, "step") == 0)) {
+        const size_t nhub = (size_t)nnz / PEEL_HUB + 1, nl = (size_t)n / 4 + n / 16 + 2;
+        DevBuf more;  // hub queues, live lists, counters
+        const size_t at_list = 2 * nhub, at_shared = (at_list + nl + 1) & ~(size_t)1;
+        if ((rc = more.ensure(4 * at_shared + sizeof(PeelShared)))) return rc;
+        PeelRunArgs pa{};
+        pa.n = n;
+        pa.rowptr = rowptr;
+        pa.col = col;
+        pa.deg = deg.as<uint32_t>();
+        pa.prio = prio;
+        pa.q[0] = q0.as<uint32_t>();
+        pa.q[1] = q1.as<uint32_t>();
+        pa.hubs[0] = more.as<uint32_t>();
+        pa.hubs[1] = pa.hubs[0] + nhub;
+        pa.list[0] = pa.hubs[0] + at_list;
+        pa.list[1] = pa.list[0] + n / 4 + 1;
+        pa.s = reinterpret_cast<PeelShared *>(more.as<uint32_t>() + at_shared);
+        pa.wait_ticks = 2000000000ull;  // 20 s at 100 MHz
+        const int gb = (int)std::max<uint64_t>(1, std::min<uint64_t>(((uint64_t)n + PEEL_T - 1) / PEEL_T, PEEL_BLOCKS));
+        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, reinterpret_cast<uint32_t *>(pa.s),
+                           (uint32_t)(sizeof(PeelShared) / 4), 0u);
+        hipLaunchKernelGGL(k_peel_init, dim3(std::min(1024, (int)((n + 255) / 256))), dim3(256), 0, s, n, rowptr,
+                           deg.as<int>(), prio, (uint8_t *)nullptr, nnz);
+        hipLaunchKernelGGL(k_peel_run, dim3(std::min(gb, ctx->cu)), dim3(PEEL_T), 0, s, pa);
+        KC_HIP(hipGetLastError());
+        PeelShared h;
+        KC_HIP(hipMemcpyAsync(&h, pa.s, sizeof h, hipMemcpyDeviceToHost, s));
+        KC_HIP(hipStreamSynchronize(s));
+        if (h.done) {
+            *max_core = h.max_core;
+            return KC_OK;
+        }
+        if (!h.abort) return fail(KC_ERR_DEVICE, "peel did not converge (internal error)");
+    }
+    if ((rc = st.ensure((size_t)n + 4))) return rc;
     int gi = (int)std::min<uint64_t>(((uint64_t)n + 255) / 256, (uint64_t)ctx->cu * 8);
     if (gi < 1) gi = 1;
     hipLaunchKernelGGL(k_peel_init, dim3(gi), dim3(256), 0, s, n, rowptr, deg.as<int>(), prio, st.as<uint8_t>(), nnz);
@@ -721,12 +990,6 @@ static int run_peel(DeviceCtx *ctx, hipStream_t s, uint32_t n, uint32_t nnz, uin
     a.q1 = q1.as<uint32_t>();
     a.cnt = cnt.as<uint32_t>();
     void *args[] = {&a};
-    // The stepped peel is the default: on the 1.7M-vertex power-law graph it
-    // takes 93 ms against 384 ms for the cooperative kernel, whose three grid
-    // barriers per round (1312 rounds there) dominate.  KC_PEEL_MODE=coop
-    // selects the cooperative kernel (falling back when it is refused).
-    const char *mode = std::getenv("KC_PEEL_MODE");
-    bool coop = mode && std::strcmp(mode, "coop") == 0;
     if (coop && hipLaunchCooperativeKernel((const void *)k_peel, dim3(grid), dim3(256), args, 0, s) != hipSuccess) {
         (void)hipGetLastError();  // the launch was refused, nothing ran: step the peel from the host
         coop = false;
@@ -933,7 +1196,7 @@ int kc::orient_device_csr(DeviceCtx *ctx, uint32_t n, uint32_t nnz, uint32_t max
         }
         hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, mx.as<uint32_t>(), 1u, 0u);
         if (n > 0)
-            hipLaunchKernelGGL(k_max_u32, dim3(std::max(1, std::min(grid, 1024))), dim3(256), 0, s, od, n,
+            hipLaunchKernelGGL(k_max_u32, dim3(std::max(1, std::min(grid, 256))), dim3(256), 0, s, od, n,
                                mx.as<uint32_t>());
     };
     Captured orient_graph;
