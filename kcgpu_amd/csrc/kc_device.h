@@ -37,12 +37,14 @@ struct DeviceCtx {
 // Select and check the device (gfx950).  Returns KC_OK or KC_ERR_DEVICE.
 int device_ctx(DeviceCtx **out);
 
-// Grow-only device buffer, or a view into memory owned elsewhere (owned =
+// Grow-only device buffer (blocks come from and go back to a bounded pool, see
+// kc_prep.hip), or a view into memory owned elsewhere (owned =
 // false; ensure() on a view checks its size and never allocates).
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
     bool owned = true;
+    int dev = 0;  // device of an owned block
     int ensure(size_t want);
     void release();
     void view(void *q, size_t b)

@@ -22,6 +22,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <memory>
 #include <mutex>
 #include <thread>
@@ -86,6 +87,55 @@ int device_ctx(DeviceCtx **out)
     return KC_OK;
 }
 
+// Device blocks that released buffers leave for the next ones, at most
+// POOL_BYTES of them over all devices: an orientation takes and gives a dozen
+// buffers, and the runtime's own allocation and free (which waits for the
+// device) took 2 to 3 ms of a 10 ms call.  Every call of the library has
+// waited for its work on a buffer before it releases it, or (on an error)
+// releases it with that work still in the library's stream, on which the next
+// owner's first use is queued too.  Blocks are given back by kc_shutdown and
+// when the device has no memory left.
+namespace {
+constexpr size_t POOL_BYTES = (size_t)512 << 20;
+struct BlockPool {
+    std::mutex mu;
+    std::multimap<std::pair<int, size_t>, void *> blocks;  // by (device, bytes)
+    size_t held = 0;
+    // a block of want..1.25 want bytes, or null
+    void *take(int dev, size_t want, size_t &got)
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        auto it = blocks.lower_bound({dev, want});
+        if (it == blocks.end() || it->first.first != dev || it->first.second > want + want / 4) return nullptr;
+        void *p = it->second;
+        got = it->first.second;
+        held -= got;
+        blocks.erase(it);
+        return p;
+    }
+    bool give(int dev, void *p, size_t bytes)
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        if (bytes > POOL_BYTES / 4 || held + bytes > POOL_BYTES) return false;
+        blocks.emplace(std::make_pair(dev, bytes), p);
+        held += bytes;
+        return true;
+    }
+    void clear()
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        for (auto &b : blocks) hipFree(b.second);
+        blocks.clear();
+        held = 0;
+    }
+};
+BlockPool &pool()
+{
+    static BlockPool *p = new BlockPool;  // (never destroyed: buffers may be released late)
+    return *p;
+}
+}  // namespace
+
 int DevBuf::ensure(size_t want)
 {
     if (!owned && p) {
@@ -95,8 +145,27 @@ int DevBuf::ensure(size_t want)
     if (want <= bytes && p && owned) return KC_OK;
     release();
     owned = true;
+    // sizes up to the pool's limit go up to the next eighth of a power of two, so
+    // that graphs of about one size fit each other's blocks
     size_t b = want ? want : 256;
+    if (b <= POOL_BYTES / 4) {
+        size_t step = 256;
+        while (step * 16 <= b) step <<= 1;
+        b = (b + step - 1) / step * step;
+    }
+    dev = 0;
+    hipGetDevice(&dev);
+    size_t got = b;
+    if ((p = pool().take(dev, b, got))) {
+        bytes = got;
+        return KC_OK;
+    }
     hipError_t e = hipMalloc(&p, b);
+    if (e != hipSuccess) {
+        pool().clear();
+        (void)hipGetLastError();
+        e = hipMalloc(&p, b);
+    }
     if (e != hipSuccess) {
         p = nullptr;
         bytes = 0;
@@ -108,7 +177,7 @@ int DevBuf::ensure(size_t want)
 
 void DevBuf::release()
 {
-    if (p && owned) hipFree(p);
+    if (p && owned && !pool().give(dev, p, bytes)) hipFree(p);
     p = nullptr;
     bytes = 0;
     owned = true;
@@ -1100,6 +1169,7 @@ int kc_shutdown(void)
                 st = nullptr;
             }
     }
+    if (g_state != 0) pool().clear();
     g_state = 0;
     return KC_OK;
 }
@@ -1143,8 +1213,7 @@ int kc::orient_device_csr(DeviceCtx *ctx, uint32_t n, uint32_t nnz, uint32_t max
     o->mode = mode;
     o->stream = ctx->stream;
     hipStream_t s = o->stream;
-    // every buffer is sized up front, so the launches need no host read in
-    // between and run as captured graphs
+    // every buffer is sized up front, so the launches need no host read in between
     DevBuf frow, fcol, outdeg, tmp, mx;
     frow.view(const_cast<uint32_t *>(frow_p), sizeof(uint32_t) * ((size_t)n + 1));
     fcol.view(const_cast<uint32_t *>(fcol_p), sizeof(uint32_t) * (size_t)nnz + 4);
@@ -1171,12 +1240,13 @@ int kc::orient_device_csr(DeviceCtx *ctx, uint32_t n, uint32_t nnz, uint32_t max
         (rc = run_peel(ctx, s, n, nnz, maxdeg, frow.as<uint32_t>(), fcol.as<uint32_t>(), o->key.as<uint32_t>(),
                        &max_core)))
         return rc;
-    // keep flags, per-row counts, scan, stable compaction, max out-degree:
-    // one captured graph
+    // keep flags, per-row counts, scan, stable compaction, max out-degree
+    // (plain launches: instantiating, launching and destroying a graph of these
+    // seven kernels, used once, took 0.45 ms of a call)
     int grid = (int)std::min<uint64_t>(((uint64_t)n + 3) / 4, (uint64_t)ctx->cu * 16);
     if (grid < 1) grid = 1;
     int scan_rc = KC_OK;
-    auto enqueue = [&]() {
+    {
         const uint32_t *fr = frow.as<uint32_t>(), *fc = fcol.as<uint32_t>();
         uint32_t *key = o->key.as<uint32_t>(), *od = outdeg.as<uint32_t>(), *orow = o->rowptr.as<uint32_t>();
         if (n > 0) {
@@ -1198,12 +1268,9 @@ int kc::orient_device_csr(DeviceCtx *ctx, uint32_t n, uint32_t nnz, uint32_t max
         if (n > 0)
             hipLaunchKernelGGL(k_max_u32, dim3(std::max(1, std::min(grid, 256))), dim3(256), 0, s, od, n,
                                mx.as<uint32_t>());
-    };
-    Captured orient_graph;
-    orient_graph.capture(s, enqueue);
+    }
     if (scan_rc) return scan_rc;
-    KC_HIP(orient_graph.launch(s, enqueue));
-    if (scan_rc) return scan_rc;
+    KC_HIP(hipGetLastError());
     KC_HIP(hipEventRecord(ev.e1, s));
     uint32_t res[2] = {0, 0};  // m, max out-degree
     KC_HIP(hipMemcpyAsync(&res[0], o->rowptr.as<uint32_t>() + n, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
