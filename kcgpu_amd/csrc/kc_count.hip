@@ -2541,6 +2541,118 @@ __device__ inline int class_of(uint32_t s, uint32_t top2)
     return s <= 64 ? 0 : s <= 128 ? 1 : s <= top2 ? 2 : s <= 512 ? 3 : s <= 1024 ? 4 : 5;
 }
 
+// Sizes |T| = |N+(u) & N+(v)| of every edge task of one graph, and, with sum,
+// what a count at k = 3 adds for them: triangles, tasks and bytes by size class.
+// A wave takes 64 consecutive edges; the edges of one u share a hash of N+(u)
+// in LDS (at most half full), and four lists N+(v) at a time are streamed
+// against it by 16 lanes each, two loads in flight, the hits counted by ballot.
+// The merge of both lists by one lane an edge, and at k = 3 staging every task
+// once more to add its size, were bound by uncoalesced loads and divergence
+// (R-MAT scale 18, 3.8 M edges: sizes 4.3 -> 1.1 ms, a call at k = 3 4.1 -> 1.3
+// ms).  Rows above HASH_ROW are searched in place.
+constexpr uint32_t HASH_SLOTS = 1024, HASH_ROW = 512;
+
+struct EdgeArgs {
+    const uint32_t *rowptr, *col, *src;
+    uint32_t m, sample, offset, top2, sum;
+    uint32_t *size;
+    uint64_t *acc;  // the algorithm's first bin (copies as in CountArgs)
+};
+
+__global__ __launch_bounds__(256) void k_edge_sizes(EdgeArgs a)
+{
+    __shared__ uint32_t tables[4][HASH_SLOTS];
+    __shared__ unsigned long long sums[NCLASS][3];
+    if (threadIdx.x < NCLASS * 3) (&sums[0][0])[threadIdx.x] = 0;
+    __syncthreads();
+    const uint32_t lane = (uint32_t)lane_id(), wv = uni32(threadIdx.x >> 6), grp = lane >> 4, sub = lane & 15;
+    uint32_t *tab = tables[wv];
+    const uint32_t nwave = gridDim.x * 4;
+    for (uint64_t e0 = (uint64_t)(blockIdx.x * 4 + wv) * 64; e0 < a.m; e0 += (uint64_t)nwave * 64) {
+        const uint32_t cnt = (uint32_t)min((uint64_t)64, a.m - e0);
+        uint32_t u = INF32, vb = 0, dv = 0, du = 0, mine = 0;
+        if (lane < cnt) {
+            u = a.src[e0 + lane];
+            const uint32_t v = a.col[e0 + lane];
+            vb = a.rowptr[v];
+            dv = a.rowptr[v + 1] - vb;
+        }
+        for (uint32_t pos = 0; pos < cnt;) {
+            const uint32_t uu = (uint32_t)__builtin_amdgcn_readlane((int)u, (int)pos);
+            const uint32_t nseg = (uint32_t)__popcll(__ballot(u == uu));  // (side by side: edges are sorted by u)
+            const uint32_t ub = a.rowptr[uu], d = a.rowptr[uu + 1] - ub;
+            const uint32_t *row = a.col + ub;
+            if (u == uu) du = d;
+            uint32_t bits = 6;
+            while (bits < 10 && (1u << bits) < 4 * d) ++bits;
+            const uint32_t mask = (1u << bits) - 1;
+            const bool hashed = d <= HASH_ROW;
+            auto slot_of = [&](uint32_t x) { return (x * 2654435761u) >> (32 - bits); };
+            if (hashed) {
+                for (uint32_t i = lane; i <= mask; i += 64) tab[i] = INF32;
+                sync_tree<true>();
+                for (uint32_t i = lane; i < d; i += 64) {
+                    const uint32_t x = row[i];
+                    uint32_t s = slot_of(x);
+                    while (atomicCAS(&tab[s], INF32, x) != INF32) s = (s + 1) & mask;
+                }
+                sync_tree<true>();
+            }
+            auto found = [&](uint32_t x) {
+                if (!hashed) {
+                    const uint32_t i = lower_bound_u32(row, d, x);
+                    return i < d && row[i] == x;
+                }
+                uint32_t s = slot_of(x), t = tab[s];
+                while (t != x && t != INF32) {
+                    s = (s + 1) & mask;
+                    t = tab[s];
+                }
+                return t == x;
+            };
+            for (uint32_t q = 0; q < nseg; q += 4) {
+                const int from = (int)((pos + q + grp) & 63);
+                const uint32_t b = __shfl(vb, from, 64), l0 = __shfl(dv, from, 64), len = q + grp < nseg ? l0 : 0;
+                uint32_t hits = 0;
+                for (uint32_t j = sub; __ballot(j < len); j += 32) {
+                    const bool in0 = j < len, in1 = j + 16 < len;
+                    const uint32_t x0 = in0 ? a.col[b + j] : INF32, x1 = in1 ? a.col[b + j + 16] : INF32;
+                    const uint64_t h0 = __ballot(in0 && found(x0)), h1 = __ballot(in1 && found(x1));
+                    hits += (uint32_t)__popc((uint32_t)(h0 >> (16 * grp)) & 0xFFFFu) +
+                            (uint32_t)__popc((uint32_t)(h1 >> (16 * grp)) & 0xFFFFu);
+                }
+                const uint32_t mq = lane - (pos + q), h = __shfl(hits, (int)((mq & 3) * 16), 64);
+                if (mq < 4 && q + mq < nseg) mine = h;
+            }
+            if (hashed) sync_tree<true>();  // the table is cleared next
+            pos += nseg;
+        }
+        if (lane < cnt) {
+            const uint32_t e = (uint32_t)e0 + lane;
+            a.size[e] = mine;
+            if (a.sum && mine && (a.sample <= 1 || e % a.sample == a.offset)) {
+                const int c = class_of(mine, a.top2);
+                atomicAdd(&sums[c][0], (unsigned long long)mine);
+                atomicAdd(&sums[c][1], 24ull + 4ull * ((uint64_t)du + dv));
+                atomicAdd(&sums[c][2], 1ull);
+            }
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < NCLASS * 3) {
+        const uint32_t c = threadIdx.x / 3, i = threadIdx.x % 3;
+        const unsigned long long v = sums[c][i];
+        unsigned long long *acc = reinterpret_cast<unsigned long long *>(
+            a.acc + ((uint64_t)c * NSTRIPE + blockIdx.x % NSTRIPE) * ACC);
+        if (i != 0) {
+            if (v) atomicAdd(&acc[i], v);
+        } else if (v) {  // a count: its low and high half (flush_query)
+            atomicAdd(&acc[0], v & 0xFFFFFFFFull);
+            atomicAdd(&acc[6], v >> 32);
+        }
+    }
+}
+
 // Bin tasks by (algorithm, size class, size slice); a task smaller than the
 // clique part still to find (k-1 for a node, k-2 for an edge) is dropped.
 // Each class from 65 to 1024 vertices is cut into NSUB slices of its size
@@ -2939,11 +3051,25 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     // that the host waits for the device once, for the result.  Otherwise it
     // reads the bins' sizes first: they choose the launches.
     const bool one_bin = one_algo && max_out <= CLASS_ROWS[0] && total < 0xFFFFFFFFull;
+    // edge tasks at k = 3 add their sizes: nothing to bin, nothing to launch after
+    // (lists of at most MERGE_OUT are sooner merged by a lane an edge, and binned:
+    // 23,936 edges with lists of at most 8, 47 us a call against 59)
+    constexpr uint32_t MERGE_OUT = 32;
+    const bool lists = nq == 1 && any_edge && max_out > MERGE_OUT;
+    const bool triangles = lists && kmax == 3 && !local && total > 0;
     BinArgs ba{dq, dalgo, doff, nq, pivot_top2, total, any_edge ? scr.size.as<uint32_t>() : nullptr, sub_cnt, bin_max,
                sub_pos, sub_off, scr.tasks.as<uint64_t>(), any_pivot ? scr.binom.as<uint64_t>() : nullptr, brows, bstride};
     if (total > 0) {
-        if (any_edge && !sizes_cached)
+        if (lists && (triangles || !sizes_cached)) {
+            EdgeArgs ea{hq[0].rowptr, hq[0].col, hq[0].src, (uint32_t)total, hq[0].sample, hq[0].offset,
+                        halgo[0] ? pivot_top2 : CLASS_ROWS[2], triangles ? 1u : 0u, scr.size.as<uint32_t>(),
+                        dacc + (halgo[0] ? NCLASS * NSTRIPE * ACC : 0)};
+            const unsigned eb = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((total + 255) / 256, (uint64_t)ctx->cu * 8));
+            if (triangles) evs.record(evs.go, s);
+            hipLaunchKernelGGL(k_edge_sizes, dim3(eb), dim3(256), 0, s, ea);
+        } else if (any_edge && !sizes_cached) {
             hipLaunchKernelGGL(k_task_size, dim3(gs), dim3(256), 0, s, dq, doff, nq, total, scr.size.as<uint32_t>());
+        }
         const bool few = total < (uint64_t)BIN_T * BIN_I * ctx->cu;  // (less than a full tile per CU)
         const int per = BIN_T * (few ? BIN_I_FEW : BIN_I);
         const unsigned tiles = (unsigned)((total + per - 1) / per);
@@ -2951,7 +3077,8 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         auto go = [&](const void *kern, unsigned blocks, unsigned threads) {
             return hipLaunchKernel(kern, dim3(blocks), dim3(threads), args, 0, s);
         };
-        if (one_bin) {
+        if (triangles) {
+        } else if (one_bin) {
             KC_HIP(go(few ? (const void *)&k_bin_scatter<true, BIN_I_FEW> : (const void *)&k_bin_scatter<true, BIN_I>,
                       tiles + 1, BIN_T));
         } else {
@@ -2968,7 +3095,8 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         scr.size_total = total;
     }
     uint32_t bcnt[NB] = {0}, bmax[NB] = {0}, boff[NB] = {0};
-    if (one_bin) {
+    if (triangles) {
+    } else if (one_bin) {
         bcnt[halgo[0] ? NCLASS : 0] = (uint32_t)total;  // (at most)
     } else {
         uint32_t h[NS + 16] = {0};
@@ -2985,7 +3113,7 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         }
         if (tot >= 0xFFFFFFFFull) return fail(KC_ERR_LIMIT, "more than 2^32 tasks in one launch");
     }
-    evs.record(evs.cls, s);
+    if (!triangles) evs.record(evs.cls, s);
 
     // --- one persistent launch per non-empty bin, largest tasks first ---
     // The bins of tasks of at most 256 vertices can run side by side on the
@@ -3010,7 +3138,7 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
             return kc::fail(KC_ERR_DEVICE, "%s failed: %s", #call, hipGetErrorString(e_));         \
         }                                                                                          \
     } while (0)
-    evs.record(evs.go, s);
+    if (!triangles) evs.record(evs.go, s);
     // Side by side only when the register classes hold few tasks per CU: then
     // a class's last long tasks are a large part of its launch (Chung-Lu
     // n=1.7M m=11.1M, edge tasks at k=8: 8,600 per CU, one 125 ms task in a
@@ -3190,14 +3318,19 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
                 uint64_t &h = hacc[b * ACC + i];
                 h = i == 4 ? std::max(h, v) : h + v;  // [4] is the longest task
             }
-    for (int b = 0; b < NB; ++b)
+    for (int b = 0; b < NB; ++b) {
+        if (triangles && hacc[ACC * b + 2]) {
+            launched[b] = true;
+            variant[b] = 6u;
+        }
         if (one_bin && hacc[ACC * b + 2] == 0) launched[b] = false;  // the bin was empty
+    }
     const uint64_t *hq_sum = back.data() + NB * NSTRIPE * ACC;
     const uint32_t *hq_flag = reinterpret_cast<const uint32_t *>(hq_sum + 2 * (size_t)nq);
     float bin_ms[NB] = {0};
-    const float prep_ms = evs.ms(evs.start, evs.cls), total_ms = evs.ms(evs.go, evs.end);
+    const float prep_ms = evs.ms(evs.start, triangles ? evs.go : evs.cls), total_ms = evs.ms(evs.go, evs.end);
     for (int b = 0; b < NB; ++b)
-        if (launched[b]) bin_ms[b] = evs.ms(evs.b0[b], evs.b1[b]);
+        if (launched[b]) bin_ms[b] = triangles ? total_ms : evs.ms(evs.b0[b], evs.b1[b]);
     int wall_khz = 100000;
     hipDeviceGetAttribute(&wall_khz, hipDeviceAttributeWallClockRate, ctx->dev);
     if (wall_khz <= 0) wall_khz = 100000;

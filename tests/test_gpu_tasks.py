@@ -3,6 +3,7 @@ from math import comb
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
 
 import kcgpu_amd as K
 from oracle import oracle as O
@@ -109,3 +110,58 @@ def test_bitmaps_of_short_tasks_in_long_rows(n, m, hub, mode):
         exp = _oracle_count(G, mode, k, gran)
         for algo in ("pivot", "orient"):
             assert o.count(k, algo, gran, part_size=1).count == exp, (k, gran, algo)
+
+
+def test_device_blocks_are_reused():
+    """graphs of several sizes oriented, counted and freed in turn, twice over the same device blocks"""
+    for i in range(20):
+        t = 50 + 400 * (i % 5)
+        src, dst, n = _disjoint_cliques([(7, t), (3, i + 1)])
+        G = K.Graph.from_edges(src, dst, n)
+        for mode in ("degree", "degen"):
+            o = G.orient(mode)
+            assert o.count(5, "pivot", "edge", part_size=1).count == t * 21
+            rp, col, key = o.export()
+            assert int(rp[-1]) == col.size == 21 * t + 3 * (i + 1) and key.size == n
+            o.close()
+
+
+def _edge_list_graphs():
+    """out-lists around the hash's sizes (512, 256), 16-lane groups and 64-edge chunks"""
+    yield "cliques", [(s, 1) for s in (3, 16, 17, 18, 33, 64, 65, 66, 128, 257, 258, 512, 513, 514, 515, 600)]
+    yield "chunk63", [(2, 63), (3, 1)]
+    yield "chunk64", [(2, 64), (4, 1)]
+    yield "many", [(3, 5001), (5, 700), (2, 31)]
+
+
+@pytest.mark.parametrize("name,sizes", list(_edge_list_graphs()))
+def test_triangles_over_edge_tasks(name, sizes):
+    src, dst, n = _disjoint_cliques(sizes)
+    o = K.orient_edges(src, dst, "degree", n=n)
+    exp = sum(comb(s, 3) * t for s, t in sizes)
+    tasks = sum(comb(s - 1, 2) * t for s, t in sizes)  # edges whose list has a member
+    for algo in ("pivot", "orient"):
+        r = o.count(3, algo, "edge", part_size=1)
+        assert r.count == exp and r.raw["tasks"] == tasks
+        assert sum(o.count_sampled(3, 5, f, algo, "edge").count for f in range(5)) == exp
+    assert o.count_noalloc(3, "pivot", "edge").count == exp
+    assert o.count(4, "pivot", "edge", part_size=1).count == sum(comb(s, 4) * t for s, t in sizes)
+
+
+@pytest.mark.parametrize("mode", ["degree", "degen"])
+def test_triangles_over_edge_tasks_vs_oracle(mode):
+    for kind, kw in ((K.GEN_RMAT, dict(scale=12, edge_factor=12, a=0.57, b=0.19, c=0.19)),
+                     (K.GEN_CHUNG_LU, dict(n=30_000, m=200_000, gamma=2.1, max_degree=3000)),
+                     (K.GEN_ER, dict(n=5000, m=60_000))):
+        G = K.Graph.generate(kind, seed=11, **kw)
+        rp, col = G.csr()
+        rp = rp.astype(np.uint64)
+        orp, oc = O.orient(rp, col, O.peel_priority(rp, col)[0] if mode == "degen" else None)
+        exp = O.count(orp, oc, 3, "pivot", "edge")
+        r = G.orient(mode).count(3, "pivot", "edge", part_size=1)
+        assert (r.count, r.raw["tasks"]) == (exp["count"], exp["tasks"])
+        # bytes: the two list heads and both lists of every edge whose lists meet (no bitmap is built at k = 3)
+        d = np.diff(orp.astype(np.int64))
+        A = sp.csr_matrix((np.ones(oc.size, np.int64), oc, orp.astype(np.int64)), shape=(d.size, d.size))
+        met = A.multiply(A @ A.T).tocoo()
+        assert r.raw["alg_bytes"] == int((24 + 4 * (d[met.row] + d[met.col])).sum())
