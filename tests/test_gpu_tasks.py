@@ -165,3 +165,22 @@ def test_triangles_over_edge_tasks_vs_oracle(mode):
         A = sp.csr_matrix((np.ones(oc.size, np.int64), oc, orp.astype(np.int64)), shape=(d.size, d.size))
         met = A.multiply(A @ A.T).tocoo()
         assert r.raw["alg_bytes"] == int((24 + 4 * (d[met.row] + d[met.col])).sum())
+
+
+# per-vertex counts of tasks at the edges of one word, where one count goes through both kernels
+@pytest.mark.parametrize("n", [4, 5, 33, 64, 65, 66, 90])
+@pytest.mark.parametrize("density", [0.3, 0.8, 1.0])
+def test_local_counts_at_word_edges_vs_oracle(n, density):
+    r = np.random.default_rng(n)
+    a, b = np.triu_indices(n, 1)
+    keep = r.random(a.size) < density
+    G = K.Graph.from_edges(a[keep].astype(np.uint32), b[keep].astype(np.uint32), n)
+    rp, col = G.csr()
+    orp, oc = O.orient(rp.astype(np.uint64), col)
+    o = G.orient("degree")
+    for k in (3, 4, 5, 6, 9):
+        exp, ovf = O.count_local(orp, oc, k, "pivot_tails", "node")
+        assert not ovf
+        for gran in ("node", "edge"):
+            loc, tot = o.count_local(k, "pivot", gran)
+            assert (loc == exp).all() and tot.count * k == int(exp.sum(dtype=np.uint64)), (k, gran)
