@@ -29,7 +29,8 @@
 //        maxDeg levels in HBM).  Subtrees are re-encoded into one-, two- or
 //        four-word rows held in registers once their candidate sets shrink,
 //        and the last levels close in form (edges; triangles by lane walks;
-//        3- and 4-cliques of near-cliques from the complement).
+//        3- and 4-cliques from the complement, by MFMA where a set is dense
+//        enough).
 // Sizes: tasks are binned by their exact list size (64, 128, 256 vertices in
 // registers, 512, 1024 in LDS, larger in an HBM slice), each class cut into
 // slices drained largest first.
@@ -852,24 +853,48 @@ __device__ inline uint64_t sct64(const CountArgs &a, uint32_t k, uint64_t row, u
     return sct_word<MM, uint64_t>(a, k, row, X0, h0, p0, nodes, ovf);
 }
 
-// The SCT of a task of at most 64 vertices with per-vertex credits: lane l
-// holds row l and the credit of vertex l, the sets X (candidates), H (held) and
-// P (pivots) of a node are uniform words, kept with every open level as in
-// sct_word.  A subtree with t = k - h vertices to find and no 4-clique wanted
-// inside X (h >= k-3, or at most three candidates) closes with
+// A set of task vertices as S uniform words.
+template <int S>
+struct Words {
+    uint64_t w[S];
+};
+
+// word o of the row of vertex v (uniform), from the lanes that hold the rows
+template <int S>
+__device__ __forceinline__ uint64_t row_word(const uint64_t (&row)[S][S], uint32_t v, int o)
+{
+    if (S == 1) return rdlane64(row[0][0], v);
+    return v < 64 ? rdlane64(row[0][o], v) : rdlane64(row[S - 1][o], v & 63);
+}
+
+// The SCT of a task of at most 64 * S vertices with per-vertex credits: lane l
+// holds the rows and credits of vertices l, l + 64, ..; the sets X (candidates),
+// H (held) and P (pivots) of a node are uniform words, kept with every open
+// level as in sct_word (a level stays open only while a vertex of its branches
+// is held, so there are at most k - 3 of them).  A subtree
+// with t = k - h vertices to find and no 4-clique wanted inside X (t <= 3, or at
+// most three candidates) closes with
 //     in all      sum_j C(p, t-j) c_j(X)            (every held vertex)
 //     a pivot     sum_j C(p-1, t-1-j) c_j(X)
 //     x in X      sum_j C(p, t-j) c_{j-1}(X & row_x)
 // j <= 3, the triangles through x counted by a uniform walk of X; the eight
 // binomials are one load.  No credit can wrap unless the count does.
 // Returns the count of the subtree (every lane).
-__device__ uint64_t sct_local(const CountArgs &a, uint32_t k, uint64_t row, uint64_t X0, uint32_t h0, uint64_t &credit,
-                              uint64_t &nodes, uint32_t &ovf)
+template <int S>
+__device__ uint64_t sct_local(const CountArgs &a, uint32_t k, const uint64_t (&row)[S][S], uint32_t R, uint32_t h0,
+                              uint64_t (&credit)[S], uint64_t &nodes, uint32_t &ovf)
 {
+    static_assert(KC_MAX_K <= 64, "a level per lane");
     const uint32_t lane = (uint32_t)lane_id();
     k = uni32(k);
-    uint64_t X = uni64(X0), H = 0, P = 0;
-    uint64_t tC = 0, tB = 0, tH = 0, tP = 0, stkC = 0, stkB = 0, stkH = 0, stkP = 0;
+    Words<S> X, H, P, tC, tB, tH, tP, stkC, stkB, stkH, stkP;
+#pragma unroll
+    for (int o = 0; o < S; ++o) {
+        const uint32_t r = R > 64u * o ? R - 64u * o : 0u;
+        X.w[o] = uni64(r >= 64 ? ~0ull : (1ull << r) - 1);
+        H.w[o] = P.w[o] = tC.w[o] = tB.w[o] = tH.w[o] = tP.w[o] = 0;
+        stkC.w[o] = stkB.w[o] = stkH.w[o] = stkP.w[o] = 0;
+    }
     uint32_t tM = 0, stkM = 0;  // h | p << 8 | pivot << 20
     bool open = false;
     int t = -1;
@@ -877,40 +902,74 @@ __device__ uint64_t sct_local(const CountArgs &a, uint32_t k, uint64_t row, uint
     uint64_t acc = 0, my_nodes = 0;
     for (;;) {
         ++my_nodes;
-        uint32_t cx = (uint32_t)__popcll(X);
+        uint32_t cx = 0;
+#pragma unroll
+        for (int o = 0; o < S; ++o) cx += (uint32_t)__popcll(X.w[o]);
         const uint32_t need = k - h;
         if (p + cx >= need) {
-            uint32_t sc = (uint32_t)__popcll(X & row);
+            uint32_t sc[S];
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                sc[s] = 0;
+#pragma unroll
+                for (int o = 0; o < S; ++o) sc[s] += (uint32_t)__popcll(X.w[o] & row[s][o]);
+            }
             bool close = need <= 3;
             if (!close) {
-                const uint64_t all = __ballot(in_mask(X) && sc + 1 == cx);  // adjacent to every other candidate
-                const uint32_t na = (uint32_t)__popcll(all);
-                X &= ~all;
-                P |= all;
+                uint32_t na = 0;
+#pragma unroll
+                for (int s = 0; s < S; ++s) {
+                    const uint64_t all = __ballot(in_mask(X.w[s]) && sc[s] + 1 == cx);  // adjacent to every other candidate
+                    na += (uint32_t)__popcll(all);
+                    X.w[s] &= ~all;
+                    P.w[s] |= all;
+                }
                 p += na;
                 cx -= na;
-                sc -= na;  // (members of X: each is adjacent to all of them)
+#pragma unroll
+                for (int s = 0; s < S; ++s) sc[s] -= na;  // (members of X: each is adjacent to all of them)
                 close = cx <= 3;
             }
             if (close) {
                 uint64_t b = 0;
-                uint32_t o = 0;
+                uint32_t o8 = 0;
                 const int up = lane < 4 ? 0 : 1, r = (int)need - up - (int)(lane & 3);
                 if (lane < 8 && r >= 0 && (up == 0 || p > 0)) {
                     const uint64_t at = (uint64_t)(p - up) * a.bstride + (uint32_t)r;
                     b = a.binom[at];
-                    o = a.binom_ovf[at];
+                    o8 = a.binom_ovf[at];
                 }
-                uint32_t e = 0, tri = 0, t2 = 0;
-                const bool mem = in_mask(X);
-                if (cx >= 2 && need >= 2) e = wave_sum32(mem ? sc : 0u) / 2;
+                uint32_t e = 0, tri = 0, t2[S];
+#pragma unroll
+                for (int s = 0; s < S; ++s) {
+                    t2[s] = 0;
+                    e += in_mask(X.w[s]) ? sc[s] : 0u;
+                }
+                e = cx >= 2 && need >= 2 ? wave_sum32(e) / 2 : 0u;
                 if (cx >= 3 && need >= 3) {
-                    const uint64_t g = mem ? (X & row) : 0ull;
-                    for (uint64_t bits = X; bits; bits &= bits - 1) {
-                        const uint64_t gu = rdlane64(g, (uint32_t)__builtin_ctzll(bits));
-                        t2 += in_mask(gu) ? (uint32_t)__popcll(g & gu) : 0u;
-                    }
-                    tri = wave_sum32(t2) / 6;
+                    uint64_t g[S][S];
+#pragma unroll
+                    for (int s = 0; s < S; ++s)
+#pragma unroll
+                        for (int o = 0; o < S; ++o) g[s][o] = in_mask(X.w[s]) ? (X.w[o] & row[s][o]) : 0ull;
+#pragma unroll
+                    for (int q = 0; q < S; ++q)
+                        for (uint64_t bits = X.w[q]; bits; bits &= bits - 1) {
+                            const uint32_t u = (uint32_t)__builtin_ctzll(bits);
+                            uint64_t gu[S];
+#pragma unroll
+                            for (int o = 0; o < S; ++o) gu[o] = rdlane64(g[q][o], u);
+#pragma unroll
+                            for (int s = 0; s < S; ++s) {
+                                uint32_t c = 0;
+#pragma unroll
+                                for (int o = 0; o < S; ++o) c += (uint32_t)__popcll(g[s][o] & gu[o]);
+                                t2[s] += in_mask(gu[s]) ? c : 0u;
+                            }
+                        }
+#pragma unroll
+                    for (int s = 0; s < S; ++s) tri += t2[s];
+                    tri = wave_sum32(tri) / 6;
                 }
                 const uint64_t B0 = rdlane64(b, 0), B1 = rdlane64(b, 1), B2 = rdlane64(b, 2), B3 = rdlane64(b, 3);
                 uint64_t all = 0;
@@ -919,30 +978,43 @@ __device__ uint64_t sct_local(const CountArgs &a, uint32_t k, uint64_t row, uint
                 add_checked(all, mul_chk(B2, e, ovf), ovf);
                 add_checked(all, mul_chk(B3, tri, ovf), ovf);
                 const uint32_t oc = lane == 0 ? 1u : lane == 1 ? cx : lane == 2 ? e : lane == 3 ? tri : 0u;
-                if (__ballot(o && oc)) ovf = 1;
+                if (__ballot(o8 && oc)) ovf = 1;
                 add_checked(acc, all, ovf);
                 const uint64_t piv = rdlane64(b, 4) + rdlane64(b, 5) * cx + rdlane64(b, 6) * e + rdlane64(b, 7) * tri;
-                const uint64_t own = B1 + B2 * sc + B3 * (t2 / 2);
-                credit += mem ? own : in_mask(H) ? all : in_mask(P) ? piv : 0ull;
+#pragma unroll
+                for (int s = 0; s < S; ++s) {
+                    const uint64_t own = B1 + B2 * sc[s] + B3 * (t2[s] / 2);
+                    credit[s] += in_mask(X.w[s]) ? own : in_mask(H.w[s]) ? all : in_mask(P.w[s]) ? piv : 0ull;
+                }
+                // (B1, B2 and B3 are 0 where need has no room for them)
             } else {
-                uint32_t key = in_mask(X) ? ((sc + 1) << 8) | (63u - lane) : 0u;
+                uint32_t key = 0;
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+                    key = in_mask(X.w[s]) ? max(key, ((sc[s] + 1) << 8) | (64u * S - 1 - 64u * s - lane)) : key;
                 key = (uint32_t)__builtin_amdgcn_readfirstlane((int)__ockl_wfred_max_u32(key));
                 if ((key >> 8) + p >= need) {
-                    const uint32_t pv = 63u - (key & 0xFFu);
+                    const uint32_t pv = 64u * S - 1 - (key & 0xFFu);
                     if (open) {
                         ++t;
                         const bool here = lane == (uint32_t)t;
-                        stkC = here ? tC : stkC;
-                        stkB = here ? tB : stkB;
-                        stkH = here ? tH : stkH;
-                        stkP = here ? tP : stkP;
+#pragma unroll
+                        for (int o = 0; o < S; ++o) {
+                            stkC.w[o] = here ? tC.w[o] : stkC.w[o];
+                            stkB.w[o] = here ? tB.w[o] : stkB.w[o];
+                            stkH.w[o] = here ? tH.w[o] : stkH.w[o];
+                            stkP.w[o] = here ? tP.w[o] : stkP.w[o];
+                        }
                         stkM = here ? tM : stkM;
                     }
                     open = true;
-                    tC = X;
-                    tB = X & ~rdlane64(row, pv) & ~(1ull << pv);
-                    tH = H;
-                    tP = P;
+#pragma unroll
+                    for (int o = 0; o < S; ++o) {
+                        tC.w[o] = X.w[o];
+                        tB.w[o] = X.w[o] & ~row_word<S>(row, pv, o) & ~((pv >> 6) == (uint32_t)o ? 1ull << (pv & 63) : 0ull);
+                        tH.w[o] = H.w[o];
+                        tP.w[o] = P.w[o];
+                    }
                     tM = h | (p << 8) | (pv << 20);
                 }
             }
@@ -950,10 +1022,13 @@ __device__ uint64_t sct_local(const CountArgs &a, uint32_t k, uint64_t row, uint
         // next branch of the open level: non-pivot vertices first, the pivot last
         if (!open) {
             if (t < 0) break;
-            tC = rdlane64(stkC, (uint32_t)t);
-            tB = rdlane64(stkB, (uint32_t)t);
-            tH = rdlane64(stkH, (uint32_t)t);
-            tP = rdlane64(stkP, (uint32_t)t);
+#pragma unroll
+            for (int o = 0; o < S; ++o) {
+                tC.w[o] = rdlane64(stkC.w[o], (uint32_t)t);
+                tB.w[o] = rdlane64(stkB.w[o], (uint32_t)t);
+                tH.w[o] = rdlane64(stkH.w[o], (uint32_t)t);
+                tP.w[o] = rdlane64(stkP.w[o], (uint32_t)t);
+            }
             tM = (uint32_t)__builtin_amdgcn_readlane((int)stkM, t);
             --t;
             open = true;
@@ -962,20 +1037,25 @@ __device__ uint64_t sct_local(const CountArgs &a, uint32_t k, uint64_t row, uint
         p = (tM >> 8) & 0xFFF;
         H = tH;
         P = tP;
-        if (tB) {
-            const uint32_t v = (uint32_t)__builtin_ctzll(tB);
-            X = tC & rdlane64(row, v);
-            tC &= ~(1ull << v);
-            tB &= tB - 1;
-            H |= 1ull << v;
-            ++h;
-        } else {  // the pivot branch replaces its level
-            const uint32_t v = tM >> 20;
-            X = tC & rdlane64(row, v);
-            P |= 1ull << v;
-            ++p;
-            open = false;
+        uint64_t left = tB.w[0];
+        if (S > 1) left |= tB.w[S - 1];
+        const bool held = left != 0;
+        uint32_t v = tM >> 20;
+        if (held) v = tB.w[0] ? (uint32_t)__builtin_ctzll(tB.w[0]) : 64u + (uint32_t)__builtin_ctzll(tB.w[S - 1]);
+#pragma unroll
+        for (int o = 0; o < S; ++o) {
+            const uint64_t bit = (v >> 6) == (uint32_t)o ? 1ull << (v & 63) : 0ull;
+            X.w[o] = tC.w[o] & row_word<S>(row, v, o);
+            H.w[o] |= held ? bit : 0ull;
+            P.w[o] |= held ? 0ull : bit;
+            if (held) {
+                tC.w[o] &= ~bit;
+                tB.w[o] &= ~bit;
+            }
         }
+        h += held ? 1u : 0u;
+        p += held ? 0u : 1u;
+        open = held;  // the pivot branch replaces its level
     }
     if (lane == 0) nodes += my_nodes;
     return acc;
@@ -1937,9 +2017,9 @@ __device__ __attribute__((always_inline)) uint32_t next_tasks(const CountArgs &a
 }
 
 // register-bitmap pivoting kernel for tasks of at most 64*S vertices
-// waves per SIMD the register budget is held to: 4 for S = 4 (<= 128 VGPRs), 6 for S = 2, 8 for S = 1
+// waves per SIMD the register budget is held to: 4 for S = 4 and 2 (<= 128 VGPRs), 8 for S = 1
 template <int S>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S == 4 ? 4 : S == 2 ? 4 : 8)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S == 1 ? 8 : 4)))
 void k_pivot_reg(CountArgs a)
 {
     extern __shared__ uint64_t lds[];
@@ -2224,7 +2304,7 @@ __device__ __attribute__((always_inline)) void publish_local(const CountArgs &a,
 
 constexpr uint32_t LOCAL_CACHE_LOG = 8, LOCAL_CACHE = 1u << LOCAL_CACHE_LOG;  // per wave: sum, vertex, owner lane
 
-// Per-vertex counts of pivoting tasks of at most 64 vertices, one wave a task,
+// Per-vertex counts of pivoting tasks of at most 64 * S vertices, one wave a task,
 // the credits in registers.  The generic kernel kept X, the held and pivot sets,
 // every level's copies and the credits in LDS behind block barriers.
 // The credits of a task go to a direct-mapped table of sums per wave in LDS, and
@@ -2234,7 +2314,10 @@ constexpr uint32_t LOCAL_CACHE_LOG = 8, LOCAL_CACHE = 1u << LOCAL_CACHE_LOG;  //
 // Chung-Lu n=300,000, m=1.96M, k=6, edge tasks: generic kernel 9.1 ms, credits
 // straight to HBM 5.5, through tables of 128 / 256 / 512 entries 3.75 / 3.35 /
 // 3.9 (512 cost resident waves); without the atomics at all it took 2.9.
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_local_reg(CountArgs a)
+// Two words (S = 2) against the generic kernel: node tasks of the same graph,
+// 2,055 of them above 64 vertices, 28.1 -> 8.0 ms for the launch.
+template <int S>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S == 1 ? 6 : 4))) void k_local_reg(CountArgs a)
 {
     extern __shared__ uint64_t lds[];
     const int lane = lane_id();
@@ -2264,50 +2347,57 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6))) void k_
             const Cur g = select_task(a, a.tasks[ti], w, task);
             ++w.ntask;
             const uint32_t R = stage_task(g, task, list, w.bytes);
-            uint64_t credit = 0, count = 0;
+            uint64_t credit[S] = {}, count = 0;
             __syncthreads();
             if (g.gran && g.k == 3) {  // an edge task at k=3 adds |T| (no bitmap needed)
                 count = R;
-                credit = lane < (int)R ? 1 : 0;
+#pragma unroll
+                for (int s = 0; s < S; ++s) credit[s] = 1;
             } else {
-                build_rows<true>(g, list, offs, starts, keys, rows, R, 1, w.bytes);
-                const uint64_t row = lane < (int)R ? rows[lane] : 0ull;
-                count = sct_local(a, g.k, row, R >= 64 ? ~0ull : ((1ull << R) - 1), g.gran ? 2u : 1u, credit, w.nodes,
-                                  w.run_ovf);
+                build_rows<true>(g, list, offs, starts, S == 1 ? keys : nullptr, rows, R, S, w.bytes);
+                uint64_t row[S][S];
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+#pragma unroll
+                    for (int o = 0; o < S; ++o)
+                        row[s][o] = (uint32_t)lane + 64u * s < R ? rows[((uint32_t)lane + 64u * s) * S + o] : 0ull;
+                count = sct_local<S>(a, g.k, row, R, g.gran ? 2u : 1u, credit, w.nodes, w.run_ovf);
             }
             run_add(w, count);
-            // one sum per lane: the vertices of the task, then its root vertices (or
-            // those by themselves when the task leaves no lane free)
-            const uint32_t roots = g.gran ? 2u : 1u;
-            uint32_t v = lane < (int)R ? list[lane] : INF32;
-            const uint32_t rt = (uint32_t)lane - (R + roots <= 64 ? R : 0u);
+            // a sum per lane: the vertices of the task, then its root vertices (those
+            // by themselves when the task leaves no lane free)
+            const uint32_t roots = g.gran ? 2u : 1u, last = R - min(R, 64u * (S - 1));
+            const uint32_t rt = (uint32_t)lane - (last + roots <= 64 ? last : 0u);
             const uint32_t root = rt == 0 ? (g.gran ? g.src[task] : task) : rt == 1 && g.gran ? g.col[task] : INF32;
-            if (R + roots <= 64) {
-                if (lane >= (int)R && root != INF32) {
-                    v = root;
-                    credit = count;
-                }
-            } else if (root != INF32 && count) {
+            if (last + roots > 64 && root != INF32 && count)
                 atomicAdd((unsigned long long *)&a.local[root], (unsigned long long)count);
-            }
-            const bool has = v != INF32 && credit;
-            const uint32_t slot = (v * 0x9E3779B1u) >> (32 - LOCAL_CACHE_LOG);
-            if (has) cown[slot] = (uint8_t)lane;
-            __syncthreads();
-            if (has) {
-                uint32_t ov = v;
-                uint64_t oc = credit;
-                if (cown[slot] == (uint8_t)lane) {
-                    const uint32_t kv = ckey[slot];
-                    const uint64_t kc = csum[slot];
-                    csum[slot] = kv == v ? kc + credit : credit;
-                    ckey[slot] = v;
-                    ov = kv == v ? INF32 : kv;
-                    oc = kc;
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                uint32_t v = (uint32_t)lane + 64u * s < R ? list[lane + 64 * s] : INF32;
+                uint64_t c = credit[s];
+                if (s == S - 1 && last + roots <= 64 && (uint32_t)lane >= last && root != INF32) {
+                    v = root;
+                    c = count;
                 }
-                if (ov != INF32) atomicAdd((unsigned long long *)&a.local[ov], (unsigned long long)oc);
+                const bool has = v != INF32 && c;
+                const uint32_t slot = (v * 0x9E3779B1u) >> (32 - LOCAL_CACHE_LOG);
+                if (has) cown[slot] = (uint8_t)lane;
+                __syncthreads();
+                if (has) {
+                    uint32_t ov = v;
+                    uint64_t oc = c;
+                    if (cown[slot] == (uint8_t)lane) {
+                        const uint32_t kv = ckey[slot];
+                        const uint64_t kc = csum[slot];
+                        csum[slot] = kv == v ? kc + c : c;
+                        ckey[slot] = v;
+                        ov = kv == v ? INF32 : kv;
+                        oc = kc;
+                    }
+                    if (ov != INF32) atomicAdd((unsigned long long *)&a.local[ov], (unsigned long long)oc);
+                }
+                __syncthreads();
             }
-            __syncthreads();
             const uint64_t dt = wall_clock64() - t0;
             w.tmax = dt > w.tmax ? dt : w.tmax;
             w.tsum += dt;
@@ -3440,8 +3530,9 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
             L = make_layout(a.rmax, a.wmax, 0, 0, true);
             variant[b] = 2u;
         }
-        if (pivot && !global && c == 0 && lc) {
-            kern = reinterpret_cast<const void *>(&k_local_reg);
+        if (pivot && !global && lc && c <= 1) {
+            kern = c == 0 ? reinterpret_cast<const void *>(&k_local_reg<1>)
+                          : reinterpret_cast<const void *>(&k_local_reg<2>);
             L = make_layout(a.rmax, a.wmax, 0, 0, true);
             L.total += LOCAL_CACHE * (sizeof(uint64_t) + sizeof(uint32_t) + 1) / sizeof(uint64_t);
             variant[b] = 2u;

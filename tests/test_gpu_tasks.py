@@ -168,7 +168,7 @@ def test_triangles_over_edge_tasks_vs_oracle(mode):
 
 
 # per-vertex counts of tasks at the edges of one word, where one count goes through both kernels
-@pytest.mark.parametrize("n", [4, 5, 33, 64, 65, 66, 90])
+@pytest.mark.parametrize("n", [4, 5, 33, 64, 65, 66, 90, 128, 129, 130, 140])
 @pytest.mark.parametrize("density", [0.3, 0.8, 1.0])
 def test_local_counts_at_word_edges_vs_oracle(n, density):
     r = np.random.default_rng(n)
