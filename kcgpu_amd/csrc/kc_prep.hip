@@ -5,10 +5,10 @@
 // Reference path replaced (src/main.cu:164-235):
 //   getNodeDegree_kernel            kcore/kcore.cuh:50-59
 //   findKcoreIncremental_async      kcore/kcore.cuh:442-584 (host loop, a D->H
-//                                   count read per round) -> steps of five
-//                                   kernels queued 32 at a time, one D->H
-//                                   read per 32 steps (or, on request, one
-//                                   cooperative kernel with grid barriers)
+//                                   count read per round) -> one launch of
+//                                   64 blocks with a barrier of their own
+//                                   (k_peel_run); steps of five kernels where
+//                                   those find no room, or on request
 //   init (keep flags)               include/main_support.cuh:54-128
 //   CUBSelect x2                    include/cub_wrappers.cuh:121-179
 //   warp_detect_deleted_edges       include/main_support.cuh:133-167
@@ -26,6 +26,7 @@
 #include <memory>
 #include <mutex>
 #include <thread>
+#include <vector>
 
 #include "kc_device.h"
 
@@ -93,21 +94,28 @@ int device_ctx(DeviceCtx **out)
 // device) took 2 to 3 ms of a 10 ms call.  Every call of the library has
 // waited for its work on a buffer before it releases it, or (on an error)
 // releases it with that work still in the library's stream, on which the next
-// owner's first use is queued too.  Blocks are given back by kc_shutdown and
-// when the device has no memory left.
+// owner's first use is queued too.  Blocks are given back by kc_shutdown, when
+// the device has no memory left, and, oldest first, when newer ones need their
+// place (a pool full of sizes that nobody asks for any more cost every call its
+// allocations again: an edge list to a count 5.1 -> 7.1 ms).
 namespace {
 constexpr size_t POOL_BYTES = (size_t)512 << 20;
 struct BlockPool {
     std::mutex mu;
-    std::multimap<std::pair<int, size_t>, void *> blocks;  // by (device, bytes)
+    struct Block {
+        void *p;
+        uint64_t seq;
+    };
+    std::multimap<std::pair<int, size_t>, Block> blocks;  // by (device, bytes)
     size_t held = 0;
+    uint64_t seq = 0;
     // a block of want..1.25 want bytes, or null
     void *take(int dev, size_t want, size_t &got)
     {
         std::lock_guard<std::mutex> lk(mu);
         auto it = blocks.lower_bound({dev, want});
         if (it == blocks.end() || it->first.first != dev || it->first.second > want + want / 4) return nullptr;
-        void *p = it->second;
+        void *p = it->second.p;
         got = it->first.second;
         held -= got;
         blocks.erase(it);
@@ -115,16 +123,27 @@ struct BlockPool {
     }
     bool give(int dev, void *p, size_t bytes)
     {
-        std::lock_guard<std::mutex> lk(mu);
-        if (bytes > POOL_BYTES / 4 || held + bytes > POOL_BYTES) return false;
-        blocks.emplace(std::make_pair(dev, bytes), p);
-        held += bytes;
+        if (bytes > POOL_BYTES / 4) return false;
+        std::vector<void *> old;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            while (held + bytes > POOL_BYTES) {
+                auto it = std::min_element(blocks.begin(), blocks.end(),
+                                           [](const auto &a, const auto &b) { return a.second.seq < b.second.seq; });
+                old.push_back(it->second.p);
+                held -= it->first.second;
+                blocks.erase(it);
+            }
+            blocks.emplace(std::make_pair(dev, bytes), Block{p, seq++});
+            held += bytes;
+        }
+        for (void *o : old) hipFree(o);  // (waits for the device: not under the lock)
         return true;
     }
     void clear()
     {
         std::lock_guard<std::mutex> lk(mu);
-        for (auto &b : blocks) hipFree(b.second);
+        for (auto &b : blocks) hipFree(b.second.p);
         blocks.clear();
         held = 0;
     }
