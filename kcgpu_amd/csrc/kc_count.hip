@@ -101,6 +101,8 @@ struct CountArgs {
     uint64_t gscr_words;
     uint64_t *local;        // per-vertex counts of the (single) query, or null
     uint32_t chain;         // wide kernel: pivot-chain levels walked before the entries
+    const uint64_t *bits;   // per edge (u, v), N+(v) among N+(u): word o of edge e at o * bits_m + e (or null)
+    uint64_t bits_m;
 };
 
 // ---- workspace layout (u64 units) -----------------------------------------
@@ -184,6 +186,20 @@ __device__ inline uint64_t wave_max64(uint64_t x)
         x = y > x ? y : x;
     }
     return x;
+}
+
+// Barrier for the state of one traversal: the whole block when a block is
+// one wave, only the wave when the waves of a block run separate subtrees.
+template <bool WIDE>
+__device__ inline void sync_tree()
+{
+    if (WIDE) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+        __syncthreads();
+    }
 }
 
 // checked sum over the wave; *ovf set on carry-out
@@ -1096,20 +1112,6 @@ __device__ inline uint64_t binom_at(const CountArgs &a, int64_t n, int64_t r)
     return (r < 0 || n < 0 || r > n) ? 0ull : a.binom[(uint64_t)n * a.bstride + (uint64_t)r];
 }
 
-// Barrier for the state of one traversal: the whole block when a block is
-// one wave, only the wave when the waves of a block run separate subtrees.
-template <bool WIDE>
-__device__ inline void sync_tree()
-{
-    if (WIDE) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    } else {
-        __syncthreads();
-    }
-}
-
 // The SCT from the root candidate set (all R task vertices, held h0, no
 // pivots), or -- with init_x false -- from the candidate set already in X
 // with h0 held and p0 pivot vertices (a subtree handed to one wave of a block).
@@ -1902,6 +1904,117 @@ __device__ __attribute__((always_inline)) uint32_t stage_task(const Cur &g, uint
     return cnt;
 }
 
+// Steps 1 and 2 from the words of a.bits, for d+(u) <= BITS_ROW.  An edge task
+// (u, v) reads T, as places in N+(u), in the word of (u, v); a node task takes
+// all places.  The words of (u, w), w in T, hold every edge inside T, and one
+// pass over T's places turns them into rows of the task: place j's bit of every
+// member is one ballot, the in-neighbours of j, and a bit of each member's own
+// out-neighbours.  IDS: list[] ends with the vertices.  Returns |T|; touches a
+// wave's own LDS only.
+// About 6 S instructions a member, where streaming the members' out-lists and
+// searching the staged list took ~100 per 64 entries of them, for every edge
+// task of u anew: without the tree walk, the launches of edge tasks of Chung-Lu
+// n=1.2M at k=5 took 14.7 ms, with it 16.2, and from the words 4.3.
+constexpr uint32_t BITS_ROW = 256;
+
+template <int S, bool IDS>
+__device__ __attribute__((always_inline)) uint32_t rows_from_bits(const CountArgs &a, const Cur &g, uint32_t task,
+                                                                  uint32_t *list, uint64_t *rows, uint64_t &bytes)
+{
+    const uint32_t lane = (uint32_t)lane_id();
+    const uint32_t u = g.gran ? uni32(g.src[task]) : task;
+    const uint32_t ub = uni32(g.rowptr[u]), du = uni32(g.rowptr[u + 1]) - ub;
+    uint64_t T[4], t0 = 0;
+    if (lane * 64 < du) {
+        const uint32_t left = du - lane * 64;
+        t0 = g.gran ? a.bits[lane * a.bits_m + task] : left >= 64 ? ~0ull : (1ull << left) - 1;
+    }
+    uint32_t R = 0;
+    if (g.gran) {
+        const uint32_t v = uni32(g.col[task]);
+        bytes += 24 + 4ull * (du + uni32(g.rowptr[v + 1]) - uni32(g.rowptr[v]));
+    } else {
+        bytes += 8 + 4ull * du;
+    }
+#pragma unroll
+    for (int o = 0; o < 4; ++o) {
+        T[o] = rdlane64(t0, o);
+        if (in_mask(T[o])) list[R + (uint32_t)__popcll(T[o] & lanemask_lt())] = 64u * o + lane;
+        R += (uint32_t)__popcll(T[o]);
+    }
+    sync_tree<true>();
+    uint32_t r[S][8], id[S], d = 0;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const uint32_t i = lane + 64u * s;
+        const uint64_t at = (uint64_t)ub + (i < R ? list[i] : 0u);
+#pragma unroll
+        for (int o = 0; o < 4; ++o) {
+            const uint64_t x = i < R && 64u * o < du ? a.bits[o * a.bits_m + at] : 0ull;
+            r[s][2 * o] = (uint32_t)x;
+            r[s][2 * o + 1] = (uint32_t)(x >> 32);
+        }
+        id[s] = g.col[at];
+        d += i < R ? g.rowptr[id[s] + 1] - g.rowptr[id[s]] : 0u;
+    }
+    bytes += 8ull * R + 4ull * wave_sum32(d);
+    const uint32_t W = (R + 63) / 64;
+    for (uint32_t i = lane; i < R * W; i += 64) rows[i] = 0;
+    if (IDS) {
+        sync_tree<true>();
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+            if (lane + 64u * s < R) list[lane + 64u * s] = id[s];
+    }
+    sync_tree<true>();
+    uint32_t jj = 0, out[S], inl[S], inh[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) out[s] = inl[s] = inh[s] = 0;
+    uint32_t *half = reinterpret_cast<uint32_t *>(rows);
+#pragma unroll
+    for (int h = 0; h < 8; ++h) {
+        for (uint32_t b = (uint32_t)(T[h >> 1] >> (32 * (h & 1))); b; b &= b - 1) {
+            const uint32_t sh = (uint32_t)__builtin_ctz(b);
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                const uint32_t bit = (r[s][h] >> sh) & 1u;
+                const uint64_t in = __ballot(bit != 0);
+                out[s] |= bit << (jj & 31);
+                inl[s] = lane == (jj & 63) ? (uint32_t)in : inl[s];
+                inh[s] = lane == (jj & 63) ? (uint32_t)(in >> 32) : inh[s];
+            }
+            ++jj;
+            if ((jj & 31) == 0 || jj == R) {  // 32 columns: into the members' rows
+                const uint32_t q = (jj - 1) >> 5;
+#pragma unroll
+                for (int s = 0; s < S; ++s) {
+                    if (lane + 64u * s < R) half[(lane + 64u * s) * 2 * W + q] |= out[s];
+                    out[s] = 0;
+                }
+                sync_tree<true>();
+                if ((jj & 63) == 0 || jj == R) {  // 64 members' in-neighbours: into their rows
+                    const uint32_t j = (q >> 1) * 64 + lane;
+#pragma unroll
+                    for (int s = 0; s < S; ++s) {
+                        if (j < R && (uint32_t)s < W) rows[(uint64_t)j * W + s] |= ((uint64_t)inh[s] << 32) | inl[s];
+                        inl[s] = inh[s] = 0;
+                    }
+                    sync_tree<true>();
+                }
+            }
+        }
+    }
+    return R;
+}
+
+// true if the task's rows come from a.bits
+__device__ inline bool has_bits(const CountArgs &a, const Cur &g, uint32_t task)
+{
+    if (!a.bits || (g.gran && g.k == 3)) return false;
+    const uint32_t u = g.gran ? uni32(g.src[task]) : task;
+    return uni32(g.rowptr[u + 1]) - uni32(g.rowptr[u]) <= BITS_ROW;
+}
+
 // Per-wave bookkeeping shared by the kernels: the graph of the current task,
 // the running count of the current query (flushed to qcount[] when the query
 // changes and at the end), and the launch statistics.
@@ -2049,7 +2162,9 @@ void k_pivot_reg(CountArgs a)
             uint32_t task;
             const Cur g = select_task(a, a.tasks[ti], w, task);
             uint64_t bytes = 0;
-            const uint32_t R = stage_task(g, task, list, bytes);
+            const bool made = has_bits(a, g, task);
+            const uint32_t R = made ? rows_from_bits<S, false>(a, g, task, list, rows, bytes)
+                                    : stage_task(g, task, list, bytes);
             if (lane == 0) ++st[2];
             if (g.gran && g.k == 3) {  // an edge task at k=3 adds |T| (no bitmap needed)
                 run_add(w, R);
@@ -2058,7 +2173,7 @@ void k_pivot_reg(CountArgs a)
                 continue;
             }
             __syncthreads();
-            build_rows<true>(g, list, offs, starts, S == 1 ? keys : nullptr, rows, R, (R + 63) / 64, bytes);
+            if (!made) build_rows<true>(g, list, offs, starts, S == 1 ? keys : nullptr, rows, R, (R + 63) / 64, bytes);
             if (lane == 0) st[1] += bytes;
             uint64_t nodes = 0;
             add_checked(w.run, pivot_reg<S>(a, g.k, rows, R, g.gran ? 2u : 1u, offs, nodes, w.run_ovf, 0u, crows),
@@ -2346,7 +2461,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S == 1 ? 6 :
             uint32_t task;
             const Cur g = select_task(a, a.tasks[ti], w, task);
             ++w.ntask;
-            const uint32_t R = stage_task(g, task, list, w.bytes);
+            const bool made = has_bits(a, g, task);
+            const uint32_t R = made ? rows_from_bits<S, true>(a, g, task, list, rows, w.bytes)
+                                    : stage_task(g, task, list, w.bytes);
             uint64_t credit[S] = {}, count = 0;
             __syncthreads();
             if (g.gran && g.k == 3) {  // an edge task at k=3 adds |T| (no bitmap needed)
@@ -2354,7 +2471,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S == 1 ? 6 :
 #pragma unroll
                 for (int s = 0; s < S; ++s) credit[s] = 1;
             } else {
-                build_rows<true>(g, list, offs, starts, S == 1 ? keys : nullptr, rows, R, S, w.bytes);
+                if (!made) build_rows<true>(g, list, offs, starts, S == 1 ? keys : nullptr, rows, R, S, w.bytes);
                 uint64_t row[S][S];
 #pragma unroll
                 for (int s = 0; s < S; ++s)
@@ -2621,15 +2738,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
         uint64_t bytes = 0;
         if (wv == 0) {
             if (lane == 0) st[6] = wall_clock64();
-            const uint32_t r = stage_task(g, task, list, bytes);
-            if (lane == 0) ctl[1] = r;
+            const bool made = has_bits(a, g, task);
+            const uint32_t r = made ? rows_from_bits<4, false>(a, g, task, list, rows, bytes)
+                                    : stage_task(g, task, list, bytes);
+            if (lane == 0) {
+                ctl[1] = r;
+                ctl[2] = made ? 1u : 0u;
+            }
         }
         __syncthreads();
         const uint32_t R = uni32(ctl[1]);
         if (g.gran && g.k == 3) {  // an edge task at k=3 adds |T| (no bitmap needed)
             if (wv == 0) run_add(w, R);
         } else {
-            build_rows_block(g, list, offs, starts, rows, R, (R + 63) / 64, bytes);
+            if (!uni32(ctl[2])) build_rows_block(g, list, offs, starts, rows, R, (R + 63) / 64, bytes);
             uint64_t nodes = 0;
             add_checked(w.run, pivot_reg<4>(a, g.k, rows, R, g.gran ? 2u : 1u, idx, nodes, w.run_ovf, 0u, crows, wv, NW),
                         w.run_ovf);
@@ -2856,8 +2978,9 @@ __device__ inline int class_of(uint32_t s, uint32_t top2)
     return s <= 64 ? 0 : s <= 128 ? 1 : s <= top2 ? 2 : s <= 512 ? 3 : s <= 1024 ? 4 : 5;
 }
 
-// Sizes |T| = |N+(u) & N+(v)| of every edge task of one graph, and, with sum,
-// what a count at k = 3 adds for them: triangles, tasks and bytes by size class.
+// Sizes |T| = |N+(u) & N+(v)| of every edge task of one graph, with sum
+// what a count at k = 3 adds for them (triangles, tasks and bytes by size
+// class), and with bits the adjacency words that rows_from_bits reads.
 // A wave takes 64 consecutive edges; the edges of one u share a hash of N+(u)
 // in LDS (at most half full), and four lists N+(v) at a time are streamed
 // against it by 16 lanes each, two loads in flight, the hits counted by ballot.
@@ -2872,11 +2995,16 @@ struct EdgeArgs {
     uint32_t m, sample, offset, top2, sum;
     uint32_t *size;
     uint64_t *acc;  // the algorithm's first bin (copies as in CountArgs)
+    uint64_t *bits;  // as CountArgs::bits, written (or null)
 };
 
+template <bool BITS>
 __global__ __launch_bounds__(256) void k_edge_sizes(EdgeArgs a)
 {
     __shared__ uint32_t tables[4][HASH_SLOTS];
+    __shared__ uint8_t places[BITS ? 4 : 1][BITS ? HASH_SLOTS : 1];  // of the table's vertices in N+(u)
+    __shared__ unsigned long long words[BITS ? 4 : 1][4][BITS_ROW / 64];
+    if (BITS && threadIdx.x < 4 * 4 * (BITS_ROW / 64)) (&words[0][0][0])[threadIdx.x] = 0;
     __shared__ unsigned long long sums[NCLASS][3];
     if (threadIdx.x < NCLASS * 3) (&sums[0][0])[threadIdx.x] = 0;
     __syncthreads();
@@ -2898,10 +3026,14 @@ __global__ __launch_bounds__(256) void k_edge_sizes(EdgeArgs a)
             const uint32_t ub = a.rowptr[uu], d = a.rowptr[uu + 1] - ub;
             const uint32_t *row = a.col + ub;
             if (u == uu) du = d;
+            if (BITS && !a.size && (d < 2 || d > BITS_ROW)) {  // (node tasks want the words alone)
+                pos += nseg;
+                continue;
+            }
             uint32_t bits = 6;
             while (bits < 10 && (1u << bits) < 4 * d) ++bits;
             const uint32_t mask = (1u << bits) - 1;
-            const bool hashed = d <= HASH_ROW;
+            const bool hashed = d <= HASH_ROW, bits_on = BITS && d <= BITS_ROW;
             auto slot_of = [&](uint32_t x) { return (x * 2654435761u) >> (32 - bits); };
             if (hashed) {
                 for (uint32_t i = lane; i <= mask; i += 64) tab[i] = INF32;
@@ -2910,10 +3042,11 @@ __global__ __launch_bounds__(256) void k_edge_sizes(EdgeArgs a)
                     const uint32_t x = row[i];
                     uint32_t s = slot_of(x);
                     while (atomicCAS(&tab[s], INF32, x) != INF32) s = (s + 1) & mask;
+                    if (bits_on) places[wv][s] = (uint8_t)i;
                 }
                 sync_tree<true>();
             }
-            auto found = [&](uint32_t x) {
+            auto found = [&](uint32_t x) {  // (and the bit of the group's list)
                 if (!hashed) {
                     const uint32_t i = lower_bound_u32(row, d, x);
                     return i < d && row[i] == x;
@@ -2922,6 +3055,10 @@ __global__ __launch_bounds__(256) void k_edge_sizes(EdgeArgs a)
                 while (t != x && t != INF32) {
                     s = (s + 1) & mask;
                     t = tab[s];
+                }
+                if (bits_on && t == x) {
+                    const uint32_t at = places[wv][s];
+                    atomicOr(&words[wv][grp][at >> 6], 1ull << (at & 63));
                 }
                 return t == x;
             };
@@ -2938,14 +3075,22 @@ __global__ __launch_bounds__(256) void k_edge_sizes(EdgeArgs a)
                 }
                 const uint32_t mq = lane - (pos + q), h = __shfl(hits, (int)((mq & 3) * 16), 64);
                 if (mq < 4 && q + mq < nseg) mine = h;
+                if (bits_on) {
+                    sync_tree<true>();
+                    if (sub * 64 < d && q + grp < nseg) {
+                        a.bits[(uint64_t)sub * a.m + e0 + pos + q + grp] = words[wv][grp][sub];
+                        words[wv][grp][sub] = 0;
+                    }
+                    sync_tree<true>();
+                }
             }
             if (hashed) sync_tree<true>();  // the table is cleared next
             pos += nseg;
         }
         if (lane < cnt) {
             const uint32_t e = (uint32_t)e0 + lane;
-            a.size[e] = mine;
-            if (a.sum && mine && (a.sample <= 1 || e % a.sample == a.offset)) {
+            if (!BITS || a.size) a.size[e] = mine;
+            if (!BITS && a.sum && mine && (a.sample <= 1 || e % a.sample == a.offset)) {
                 const int c = class_of(mine, a.top2);
                 atomicAdd(&sums[c][0], (unsigned long long)mine);
                 atomicAdd(&sums[c][1], 24ull + 4ull * ((uint64_t)du + dv));
@@ -3370,18 +3515,32 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     // (lists of at most MERGE_OUT are sooner merged by a lane an edge, and binned:
     // 23,936 edges with lists of at most 8, 47 us a call against 59)
     constexpr uint32_t MERGE_OUT = 32;
+    constexpr uint64_t BITS_BYTES = 2ull << 30;
     const bool lists = nq == 1 && any_edge && max_out > MERGE_OUT;
     const bool triangles = lists && kmax == 3 && !local && total > 0;
+    // The adjacency words (rows_from_bits) of a pivoting query on a graph with
+    // long lists: they belong to the handle's scratch like the sizes, and are
+    // made by the pass that makes those, of a whole count and within BITS_BYTES.
+    // A sample of the tasks would not earn the pass; the fixed scratch and the
+    // server's workers keep to the memory they declared.
+    const uint64_t nedge = qs[0].o->m;
+    const uint64_t bits_bytes = nedge * sizeof(uint64_t) * std::min<uint64_t>(BITS_ROW / 64, ((uint64_t)max_out + 63) / 64);
+    const bool with_bits = nq == 1 && max_out > MERGE_OUT && !triangles && halgo[0] && !(any_edge && kmax == 3) && nedge > 0 &&
+                           !scr.fixed && grid_share <= 1 && scr.may_grow && hq[0].sample <= 1 &&
+                           bits_bytes <= BITS_BYTES && scr.bits.ensure(bits_bytes) == KC_OK;
+    const bool bits_cached = with_bits && scr.bits_uid == qs[0].o->uid;
+    if (with_bits && !bits_cached) scr.bits_uid = 0;
     BinArgs ba{dq, dalgo, doff, nq, pivot_top2, total, any_edge ? scr.size.as<uint32_t>() : nullptr, sub_cnt, bin_max,
                sub_pos, sub_off, scr.tasks.as<uint64_t>(), any_pivot ? scr.binom.as<uint64_t>() : nullptr, brows, bstride};
     if (total > 0) {
-        if (lists && (triangles || !sizes_cached)) {
-            EdgeArgs ea{hq[0].rowptr, hq[0].col, hq[0].src, (uint32_t)total, hq[0].sample, hq[0].offset,
-                        halgo[0] ? pivot_top2 : CLASS_ROWS[2], triangles ? 1u : 0u, scr.size.as<uint32_t>(),
-                        dacc + (halgo[0] ? NCLASS * NSTRIPE * ACC : 0)};
-            const unsigned eb = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((total + 255) / 256, (uint64_t)ctx->cu * 8));
+        if ((lists && (triangles || !sizes_cached)) || (with_bits && !bits_cached)) {
+            EdgeArgs ea{hq[0].rowptr, hq[0].col, hq[0].src, (uint32_t)nedge, hq[0].sample, hq[0].offset,
+                        halgo[0] ? pivot_top2 : CLASS_ROWS[2], triangles ? 1u : 0u, any_edge ? scr.size.as<uint32_t>() : nullptr,
+                        dacc + (halgo[0] ? NCLASS * NSTRIPE * ACC : 0), with_bits && !bits_cached ? scr.bits.as<uint64_t>() : nullptr};
+            const unsigned eb = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((nedge + 255) / 256, (uint64_t)ctx->cu * 8));
             if (triangles) evs.record(evs.go, s);
-            hipLaunchKernelGGL(k_edge_sizes, dim3(eb), dim3(256), 0, s, ea);
+            if (ea.bits) hipLaunchKernelGGL(k_edge_sizes<true>, dim3(eb), dim3(256), 0, s, ea);
+            else hipLaunchKernelGGL(k_edge_sizes<false>, dim3(eb), dim3(256), 0, s, ea);
         } else if (any_edge && !sizes_cached) {
             hipLaunchKernelGGL(k_task_size, dim3(gs), dim3(256), 0, s, dq, doff, nq, total, scr.size.as<uint32_t>());
         }
@@ -3409,6 +3568,7 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         scr.size_uid = qs[0].o->uid;
         scr.size_total = total;
     }
+    if (with_bits) scr.bits_uid = qs[0].o->uid;
     uint32_t bcnt[NB] = {0}, bmax[NB] = {0}, boff[NB] = {0};
     if (triangles) {
     } else if (one_bin) {
@@ -3503,6 +3663,8 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         a.qhead = qhead + (size_t)b * NQUEUE * QSTRIDE;
         a.acc = dacc + (size_t)b * NSTRIPE * ACC;
         a.acc_mask = NSTRIPE - 1;
+        a.bits = with_bits ? scr.bits.as<uint64_t>() : nullptr;
+        a.bits_m = nedge;
         a.qcount = qcount;
         a.single = nq == 1;
         a.qovf = qovf;
@@ -4043,6 +4205,7 @@ static int count_tasks(const kc_oriented *o, const kc_query *q, uint32_t stride,
     std::vector<QueryRun> qs{run};
     std::vector<kc_result> res;
     LaunchStats ls;
+    om->scr.may_grow = true;
     rc = run_queries(om->scr, om->stream, qs, res, &ls);
     if (rc) return rc;
     fill_result(r, res[0], ls);
@@ -4089,6 +4252,7 @@ extern "C" int kc_count_local(const kc_oriented *o, const kc_query *q, uint64_t 
     std::vector<QueryRun> qs{QueryRun{o, qq}};
     std::vector<kc_result> res;
     LaunchStats ls;
+    om->scr.may_grow = true;
     rc = run_queries(om->scr, om->stream, qs, res, &ls, om->scr.local.as<uint64_t>());
     if (rc) return rc;
     if (n) {

@@ -65,14 +65,16 @@ int scan_exclusive_u32(const uint32_t *in, uint32_t *out, uint32_t n, DevBuf &tm
 // scratch of one launch sequence (grow-only), or views into a fixed region
 // (fixed = true: ensure() never allocates, run_queries creates no events)
 struct Scratch {
-    DevBuf tasks, meta, binom, gscr, size, qdesc, local;
+    DevBuf tasks, meta, binom, gscr, size, qdesc, local, bits;
     bool fixed = false;
+    bool may_grow = false;  // a handle's own: pivoting may keep the adjacency words of the tasks in `bits`
     // what `size` holds when it was filled for one query of edge tasks: the
     // oriented graph (its uid) and the task count; an edge task's size
     // |N+(u) & N+(v)| does not depend on k, so the next query on that graph
     // reuses it
     uint64_t size_uid = 0;
     uint64_t size_total = 0;
+    uint64_t bits_uid = 0;  // likewise the oriented graph of `bits`
 };
 
 // a number no other oriented graph of the process carries

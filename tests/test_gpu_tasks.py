@@ -184,3 +184,38 @@ def test_local_counts_at_word_edges_vs_oracle(n, density):
         for gran in ("node", "edge"):
             loc, tot = o.count_local(k, "pivot", gran)
             assert (loc == exp).all() and tot.count * k == int(exp.sum(dtype=np.uint64)), (k, gran)
+
+
+# tasks whose rows come from the adjacency words of the size pass, on both sides of the list lengths that
+# decide it (32, 256) and of the words and half words of T; a batch of two queries takes the lists
+@pytest.mark.parametrize("sizes", [(31, 32, 33, 34, 35), (64, 65, 66, 67), (96, 97, 98), (128, 129, 130, 131),
+                                   (192, 193, 194, 195), (255, 256, 257, 258, 259), (400,)])
+@pytest.mark.parametrize("density", [0.15, 0.9])
+def test_tasks_from_adjacency_words_equal_lists(sizes, density):
+    r = np.random.default_rng(sum(sizes))
+    src, dst, at = [], [], 0
+    for n in sizes:
+        a, b = np.triu_indices(n, 1)
+        keep = r.random(a.size) < density
+        keep |= (a == 0) | (a == n // 2)  # two vertices with long lists either way
+        p = at + r.permutation(n)
+        src.append(p[a[keep]])
+        dst.append(p[b[keep]])
+        at += n
+    s, d = np.concatenate(src).astype(np.uint32), np.concatenate(dst).astype(np.uint32)
+    G = K.Graph.from_edges(s, d, at)
+    for mode in ("degree", "degen"):
+        o = G.orient(mode)
+        for k in (4, 5, 6):
+            both, _ = K.batch_count([(o, dict(k=k, algo="pivot", gran="edge"))] * 2)
+            one = [o.count(k, "pivot", "edge") for _ in range(2)]
+            for x in one:
+                assert x.count == both[0].count == both[1].count == o.count(k, "pivot", "node").count
+            loc, tot = o.count_local(k, "pivot", "edge")
+            ref, _ = o.count_local(k, "pivot", "node")
+            assert (loc == ref).all() and tot.count == one[0].count
+            for gran in ("edge", "node"):
+                parts = [o.count_sampled(k, 3, i, "pivot", gran) for i in range(3)]  # (lists too)
+                one = o.count(k, "pivot", gran)
+                for what in ("count", "tasks", "alg_bytes"):
+                    assert sum(x.raw[what] for x in parts) == one.raw[what], (k, gran, what)
