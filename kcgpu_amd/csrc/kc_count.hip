@@ -263,7 +263,8 @@ __device__ inline uint32_t lower_bound_u32(const P *a, uint32_t n, uint32_t x)
 // task (Chung-Lu n=1.2M, edge tasks of at most 64 vertices: 26 members, 1,530
 // entries, 330 pairs): wave time of those tasks 58 -> 33 s at k=5, 68 -> 39 at
 // k=7, and n=500k at k=7 6.0 -> 5.3 ms.  Above 64 vertices the gathers lose
-// (65..128 at k=5: 32 -> 63 s).  keys = null: entries only.
+// (65..128 at k=5: 32 -> 63 s).  keys = null: entries only.  Tasks whose rows
+// come from the adjacency words (rows_from_bits) need neither.
 template <bool FULL>
 __device__ __attribute__((always_inline)) void build_rows(const Cur &g, uint32_t *list, uint32_t *offs,
                                                          uint32_t *starts, uint32_t *keys, uint64_t *rows, uint32_t R,
@@ -1909,15 +1910,15 @@ __device__ __attribute__((always_inline)) uint32_t stage_task(const Cur &g, uint
 // all places.  The words of (u, w), w in T, hold every edge inside T, and one
 // pass over T's places turns them into rows of the task: place j's bit of every
 // member is one ballot, the in-neighbours of j, and a bit of each member's own
-// out-neighbours.  IDS: list[] ends with the vertices.  Returns |T|; touches a
-// wave's own LDS only.
+// out-neighbours (all that is wanted without FULL, as in build_rows).  IDS: list[]
+// ends with the vertices.  Returns |T|; touches a wave's own LDS only.
 // About 6 S instructions a member, where streaming the members' out-lists and
 // searching the staged list took ~100 per 64 entries of them, for every edge
 // task of u anew: without the tree walk, the launches of edge tasks of Chung-Lu
 // n=1.2M at k=5 took 14.7 ms, with it 16.2, and from the words 4.3.
 constexpr uint32_t BITS_ROW = 256;
 
-template <int S, bool IDS>
+template <int S, bool IDS, bool FULL = true>
 __device__ __attribute__((always_inline)) uint32_t rows_from_bits(const CountArgs &a, const Cur &g, uint32_t task,
                                                                   uint32_t *list, uint64_t *rows, uint64_t &bytes)
 {
@@ -1978,8 +1979,9 @@ __device__ __attribute__((always_inline)) uint32_t rows_from_bits(const CountArg
 #pragma unroll
             for (int s = 0; s < S; ++s) {
                 const uint32_t bit = (r[s][h] >> sh) & 1u;
-                const uint64_t in = __ballot(bit != 0);
                 out[s] |= bit << (jj & 31);
+                if (!FULL) continue;
+                const uint64_t in = __ballot(bit != 0);
                 inl[s] = lane == (jj & 63) ? (uint32_t)in : inl[s];
                 inh[s] = lane == (jj & 63) ? (uint32_t)(in >> 32) : inh[s];
             }
@@ -1992,7 +1994,7 @@ __device__ __attribute__((always_inline)) uint32_t rows_from_bits(const CountArg
                     out[s] = 0;
                 }
                 sync_tree<true>();
-                if ((jj & 63) == 0 || jj == R) {  // 64 members' in-neighbours: into their rows
+                if (FULL && ((jj & 63) == 0 || jj == R)) {  // 64 members' in-neighbours: into their rows
                     const uint32_t j = (q >> 1) * 64 + lane;
 #pragma unroll
                     for (int s = 0; s < S; ++s) {
@@ -2556,7 +2558,13 @@ __global__ __launch_bounds__(64) void k_count(CountArgs a)
             const Cur g = select_task(a, a.tasks[ti], w, task);
             const uint32_t k = g.k;
             ++w.ntask;
-            const uint32_t R = stage_task(g, task, list, w.bytes);
+            // (the orientation's tasks up to 128 vertices: Chung-Lu n=200,000, k=5, edge
+            // tasks 0.95 -> 0.71 ms a call, n=300,000, k=4 1.27 -> 0.61; with the four words
+            // of larger tasks too the registers cost waves: 0.75, 0.64)
+            const bool made = !PIVOT && !GLOBAL && a.rmax <= 128 && has_bits(a, g, task);
+            const uint32_t R = !made          ? stage_task(g, task, list, w.bytes)
+                               : a.rmax <= 64 ? rows_from_bits<1, LOCAL, false>(a, g, task, list, rows, w.bytes)
+                                              : rows_from_bits<2, LOCAL, false>(a, g, task, list, rows, w.bytes);
             if (LOCAL)
                 for (uint32_t i = lane; i < R; i += 64) lacc[i] = 0;
             if (g.gran && k == 3) {  // an edge task at k=3 adds |T| (no bitmap needed)
@@ -2575,7 +2583,7 @@ __global__ __launch_bounds__(64) void k_count(CountArgs a)
             uint64_t task_count;
             if (!PIVOT) {
                 // (k-1)-cliques of the DAG on N+(u) / (k-2)-cliques of the DAG on T
-                build_rows<false>(g, list, offs, starts, keys, rows, R, W, w.bytes);
+                if (!made) build_rows<false>(g, list, offs, starts, keys, rows, R, W, w.bytes);
                 uint32_t povf = 0;
                 uint64_t part = orient_count<LOCAL>(a, g.psize, rows, stk, misc, R, W, g.gran ? k - 2 : k - 1,
                                                     w.nodes, povf, lacc, path);
@@ -3518,14 +3526,14 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     constexpr uint64_t BITS_BYTES = 2ull << 30;
     const bool lists = nq == 1 && any_edge && max_out > MERGE_OUT;
     const bool triangles = lists && kmax == 3 && !local && total > 0;
-    // The adjacency words (rows_from_bits) of a pivoting query on a graph with
+    // The adjacency words (rows_from_bits) of one query on a graph with
     // long lists: they belong to the handle's scratch like the sizes, and are
     // made by the pass that makes those, of a whole count and within BITS_BYTES.
     // A sample of the tasks would not earn the pass; the fixed scratch and the
     // server's workers keep to the memory they declared.
     const uint64_t nedge = qs[0].o->m;
     const uint64_t bits_bytes = nedge * sizeof(uint64_t) * std::min<uint64_t>(BITS_ROW / 64, ((uint64_t)max_out + 63) / 64);
-    const bool with_bits = nq == 1 && max_out > MERGE_OUT && !triangles && halgo[0] && !(any_edge && kmax == 3) && nedge > 0 &&
+    const bool with_bits = nq == 1 && max_out > MERGE_OUT && !triangles && !(any_edge && kmax == 3) && nedge > 0 &&
                            !scr.fixed && grid_share <= 1 && scr.may_grow && hq[0].sample <= 1 &&
                            bits_bytes <= BITS_BYTES && scr.bits.ensure(bits_bytes) == KC_OK;
     const bool bits_cached = with_bits && scr.bits_uid == qs[0].o->uid;

@@ -219,3 +219,8 @@ def test_tasks_from_adjacency_words_equal_lists(sizes, density):
                 one = o.count(k, "pivot", gran)
                 for what in ("count", "tasks", "alg_bytes"):
                     assert sum(x.raw[what] for x in parts) == one.raw[what], (k, gran, what)
+                if k == 4 and sizes[-1] < 300:  # the orientation's search over the same rows
+                    for P in (1, 8, 64):
+                        assert o.count(k, "orient", gran, part_size=P).count == one.count
+                    if sizes[-1] < 100:
+                        assert (o.count_local(k, "orient", gran)[0] == ref).all()
