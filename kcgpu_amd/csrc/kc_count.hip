@@ -3529,6 +3529,10 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     // The adjacency words (rows_from_bits) of one query on a graph with
     // long lists: they belong to the handle's scratch like the sizes, and are
     // made by the pass that makes those, of a whole count and within BITS_BYTES.
+    // With lists of at most MERGE_OUT the pass costs the first call more than a
+    // later one gains (BA n=200,000: 0.63 -> 0.84 and 0.52 -> 0.41 ms); with longer
+    // ones both gain (Chung-Lu n=300,000, 2 M edges: pass 0.36 ms, the launches of a
+    // count at k=6 1.39 -> 0.90 ms).
     // A sample of the tasks would not earn the pass; the fixed scratch and the
     // server's workers keep to the memory they declared.
     const uint64_t nedge = qs[0].o->m;
