@@ -3648,6 +3648,22 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     for (int b = 0; b < NB; ++b)
         if (b % NCLASS > 2) wide_tasks += bcnt[b];
     const bool few_wide = wide_tasks <= (uint64_t)ctx->cu;
+    // Every launch is planned before the first one starts: the HBM slices of the
+    // classes that need them are one block, sized here for the largest need.  A
+    // block that grew between two launches would be released while the launch
+    // before still keeps its bitmaps, chains and entry lists in it (the class
+    // above 1024 vertices goes first, with few tasks; the 513..1024 class behind
+    // it has smaller slices and usually more of them).
+    struct Launch {
+        CountArgs a;
+        const void *kern;
+        int b;
+        uint32_t blocks, nw;
+        size_t lds;
+        bool global;
+    };
+    std::vector<Launch> plan;
+    size_t slice_bytes = 0;
     bool side_waits[DeviceCtx::NSIDE] = {false}, fan_recorded = false;
     hipStream_t bin_stream[NB];
     int nside = 0;
@@ -3723,10 +3739,8 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
             // chain levels walked by wave 0 before the entries are shared: the
             // whole chain for the HBM classes (a chain left whole is one entry,
             // which one wave would walk alone), 32 levels when LDS holds them
-            if (a.rmax >= 0xFFFFu) {
-                drain();
+            if (a.rmax >= 0xFFFFu)
                 return fail(KC_ERR_LIMIT, "a task of %u vertices exceeds the wide kernel's 65534", a.rmax);
-            }
             a.chain = c == 3 ? 32u : std::min<uint32_t>(1024u, std::max<uint32_t>(64u, a.rmax));
             bool fits = false;
             if (c < NCLASS - 1)
@@ -3748,9 +3762,9 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
             variant[b] = global ? 5u : 4u;
         }
         const size_t lds = global ? 0 : L.total * 8;
-        if (!global) KC_HIP_L(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        if (!global) KC_HIP(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         int per_cu = 0;
-        KC_HIP_L(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, (int)(64 * nw), lds));
+        KC_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, (int)(64 * nw), lds));
         if (per_cu < 1) per_cu = 1;
         uint64_t blocks = std::max<uint64_t>(1, (uint64_t)per_cu * ctx->cu / std::max<uint32_t>(1, grid_share));
         // one block per task while the tasks are few, else the persistent grid
@@ -3765,20 +3779,21 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
             a.gscr_words = L.total;
             // a fixed scratch holds as many slices as fit in what it has left
             const uint64_t cap = (scr.fixed ? scr.gscr.bytes : (2ull << 30)) / (L.total * 8 + 1);
-            if (scr.fixed && cap == 0) {
-                drain();
+            if (scr.fixed && cap == 0)
                 return fail(KC_ERR_LIMIT, "a task of %u vertices needs %llu bytes of HBM workspace, more than the "
                             "%zu left in the fixed scratch", a.rmax, (unsigned long long)(L.total * 8), scr.gscr.bytes);
-            }
             blocks = std::max<uint64_t>(1, std::min<uint64_t>(blocks, cap));
-            if ((rc = scr.gscr.ensure(blocks * L.total * 8))) {
-                drain();
-                return rc;
-            }
-            a.gscr = scr.gscr.as<uint64_t>();
+            slice_bytes = std::max<size_t>(slice_bytes, blocks * L.total * 8);
         }
+        plan.push_back(Launch{a, kern, b, (uint32_t)blocks, nw, lds, global});
+    }
+    if (slice_bytes && (rc = scr.gscr.ensure(slice_bytes))) return rc;
+    DevBuf::InUse in_use;  // from here to the wait below no buffer of this thread may move
+    for (Launch &l : plan) {
+        const int b = l.b;
+        if (l.global) l.a.gscr = scr.gscr.as<uint64_t>();
         hipStream_t st = s;
-        if (fan && !global && c <= 2) {
+        if (fan && !l.global && b % NCLASS <= 2) {
             if (!fan_recorded && !few_wide) {
                 KC_HIP_L(hipEventRecord(evs.fan, s));  // after every launch so far on s
                 fan_recorded = true;
@@ -3791,9 +3806,11 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
             }
         }
         bin_stream[b] = st;
-        void *args[] = {&a};
+        if (plan.size() > 1 && !l.global)  // (two classes may share a kernel: the last plan's limit stands)
+            KC_HIP_L(hipFuncSetAttribute(l.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.lds));
+        void *args[] = {&l.a};
         evs.record(evs.b0[b], st);
-        KC_HIP_L(hipLaunchKernel(kern, dim3((unsigned)blocks), dim3(64 * nw), args, lds, st));
+        KC_HIP_L(hipLaunchKernel(l.kern, dim3(l.blocks), dim3(64 * l.nw), args, l.lds, st));
         evs.record(evs.b1[b], st);
         launched[b] = true;
     }

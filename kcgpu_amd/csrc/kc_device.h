@@ -56,6 +56,12 @@ struct DevBuf {
     }
     ~DevBuf() { release(); }
     template <class T> T *as() const { return static_cast<T *>(p); }
+    // While one lives, this thread has launches running on its buffers: ensure()
+    // refuses to move a block, which would hand it on (or free it) under them.
+    struct InUse {
+        InUse();
+        ~InUse();
+    };
 };
 
 // Exclusive scan of n uint32 counts into out[0..n] (out[n] = total); total

@@ -155,6 +155,10 @@ BlockPool &pool()
 }
 }  // namespace
 
+static thread_local int t_in_use = 0;  // DevBuf::InUse of this thread
+DevBuf::InUse::InUse() { ++t_in_use; }
+DevBuf::InUse::~InUse() { --t_in_use; }
+
 int DevBuf::ensure(size_t want)
 {
     if (!owned && p) {
@@ -162,6 +166,7 @@ int DevBuf::ensure(size_t want)
         return fail(KC_ERR_LIMIT, "%zu bytes of scratch needed, the fixed region holds %zu", want, bytes);
     }
     if (want <= bytes && p && owned) return KC_OK;
+    if (p && t_in_use) return fail(KC_ERR_DEVICE, "a buffer in use by a launch would move (internal error)");
     release();
     owned = true;
     // sizes up to the pool's limit go up to the next eighth of a power of two, so
