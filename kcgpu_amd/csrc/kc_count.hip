@@ -504,6 +504,18 @@ struct CliqueCounts {
     uint32_t e, c3, c4;
 };
 
+// How the tree walk below a task closes its nodes, by the kernel around it:
+//   MFMA      register kernels: sets of 33..128 vertices go through the matrix cores
+//   LEAN      such sets by a uniform walk (no operand registers)
+//   WIDE_SCT  the block-wide kernel: as LEAN, its one-word walk a function of its
+//         own, the binomials of a closing node computed: two waves per SIMD do not
+//         hide the trip to the table, and its registers are full.  With the matrix
+//         cores and pivot_count as a function it spilled 736 bytes a lane and saved
+//         registers at every call (R-MAT scale 22: edge tasks of 257..512 vertices
+//         at k=5 2.16 s, 1.69 s now, node tasks above 512 0.84 -> 0.73 s; 1/1024 of
+//         the edge tasks at k=8, both classes, 1.51 + 1.92 -> 1.22 + 1.58 s)
+enum Kind { MFMA, LEAN, WIDE_SCT };
+
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
@@ -705,13 +717,19 @@ __device__ inline uint64_t close_k3(const CountArgs &a, uint32_t p, uint32_t cx,
 // over the lanes until the task ends).  The five binomials are one load,
 // issued before the counts are made: term by term they were five dependent
 // trips to memory, which a closing node waited for longer than it computed.
+// With COMPUTED they are worked out for need <= 4 (p < 2^16: p^4 fits 64 bits).
+template <bool COMPUTED>
 struct CloseTerm {
     uint64_t b = 0;
     uint32_t o = 0;
     __device__ CloseTerm(const CountArgs &a, uint32_t need, uint32_t p)
     {
         const uint32_t j = (uint32_t)lane_id();
-        if (j <= 4 && j <= need) {
+        if (COMPUTED && need <= 4) {
+            const uint32_t r = need - j;  // (j > need: no term)
+            const uint64_t q = p, p2 = p ? q * (q - 1) : 0ull, p3 = p > 1 ? p2 * (q - 2) : 0ull;
+            b = r == 0 ? 1ull : r == 1 ? q : r == 2 ? p2 / 2 : r == 3 ? p3 / 6 : r == 4 && p > 2 ? p3 * (q - 3) / 24 : 0ull;
+        } else if (j <= 4 && j <= need) {
             const uint64_t idx = (uint64_t)p * a.bstride + (need - j);
             b = a.binom[idx];
             o = a.binom_ovf[idx];
@@ -747,11 +765,12 @@ __device__ inline uint64_t wave_total(uint64_t x, uint32_t lane_ovf, uint32_t &o
 // adjacent to all others lie in every maximal clique of X: they become pivots
 // together instead of one node each.  A 64-vertex subtree whose candidates
 // are at most 32 is re-encoded as a 32-vertex one.
-template <bool MM, class U>
+template <Kind KIND, class U>
 __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32_t h0, uint32_t p0, uint64_t &nodes,
                              uint32_t &ovf)
 {
     constexpr uint32_t BITS = 8 * sizeof(U);
+    constexpr bool MM = KIND == MFMA;
     const uint32_t lane = (uint32_t)lane_id(), v = lane & (BITS - 1);
     k = uni32(k);
     U X = BITS == 64 ? (U)uni64(X0) : (U)uni32((uint32_t)X0);
@@ -790,7 +809,7 @@ __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32
                         }
                         X1 = cx >= 32 ? ~0u : (1u << cx) - 1;
                     }
-                    add_checked(acc, sct_word<MM, uint32_t>(a, k, row1, X1, h, p, nodes, ovf), ovf);
+                    add_checked(acc, sct_word<KIND, uint32_t>(a, k, row1, X1, h, p, nodes, ovf), ovf);
                     --my_nodes;  // counted again as the subtree's root
                 }
             } else {
@@ -823,7 +842,7 @@ __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32
                     }
                 }
                 if (close) {
-                    const CloseTerm term(a, need, p);
+                    const CloseTerm<KIND == WIDE_SCT> term(a, need, p);
                     CliqueCounts c{0, 0, 0};
                     if (cx >= 2 && need >= 3) {
                         c = close_word<MM>(X, row, cx, need > 3);
@@ -863,11 +882,16 @@ __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32
 }
 
 // SCT of a one-word subproblem (row = the lane's row, 0 beyond the subproblem)
-template <bool MM>
+template <Kind KIND>
 __device__ inline uint64_t sct64(const CountArgs &a, uint32_t k, uint64_t row, uint64_t X0, uint32_t h0, uint32_t p0,
                                  uint64_t &nodes, uint32_t &ovf)
 {
-    return sct_word<MM, uint64_t>(a, k, row, X0, h0, p0, nodes, ovf);
+    return sct_word<KIND, uint64_t>(a, k, row, X0, h0, p0, nodes, ovf);
+}
+__device__ __attribute__((noinline)) uint64_t sct64_wide(const CountArgs &a, uint32_t k, uint64_t row, uint64_t X0,
+                                                         uint32_t h0, uint32_t p0, uint64_t &nodes, uint32_t &ovf)
+{
+    return sct64<WIDE_SCT>(a, k, row, X0, h0, p0, nodes, ovf);
 }
 
 // A set of task vertices as S uniform words.
@@ -1119,9 +1143,9 @@ __device__ inline uint64_t binom_at(const CountArgs &a, int64_t n, int64_t r)
 template <int S>
 __device__ uint32_t tri_lanes(const uint64_t *rows, uint32_t W, const uint64_t (&X)[S], uint32_t cx, uint32_t e2,
                               uint32_t *idx);
-// CL4: the four-word kernel also closes h = k-4 near-cliques (the wide kernel
-// has the registers for it; the one-wave four-word kernel keeps its budget)
-template <int S, bool CL4 = false>
+// (WIDE_SCT: four words close h = k-4 near-cliques too; the wide kernel has the
+// registers for it, the one-wave four-word kernel keeps its budget)
+template <int S, Kind KIND>
 __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t R, uint32_t h0,
                               uint32_t *idx, uint64_t &nodes, uint32_t &ovf, uint32_t p0, uint64_t *crows, uint32_t wv = 0,
                               uint32_t nw = 1);
@@ -1137,8 +1161,10 @@ __device__ uint32_t tri_lds(const uint64_t *rows, uint32_t W, const uint64_t *X,
     return tri_lanes<S>(rows, W, Xr, cx, e2, idx);
 }
 
+// (inline always: as a function of its own it saved and restored its registers for
+// every entry of the wide kernel)
 template <bool LOCAL, bool WIDE = false>
-__device__ uint64_t pivot_count(const CountArgs &a, uint32_t P, uint32_t k, const uint64_t *rows, uint64_t *stk,
+__device__ __attribute__((always_inline)) uint64_t pivot_count(const CountArgs &a, uint32_t P, uint32_t k, const uint64_t *rows, uint64_t *stk,
                                 uint64_t *X, Scal *scal, uint32_t *cand, uint32_t R, uint32_t W, uint32_t h0,
                                 uint64_t &nodes, uint32_t &ovf, uint64_t *lacc, uint32_t p0 = 0, bool init_x = true,
                                 uint64_t *crows2 = nullptr, uint64_t *crows4 = nullptr)
@@ -1213,7 +1239,7 @@ __device__ uint64_t pivot_count(const CountArgs &a, uint32_t P, uint32_t k, cons
                     row1 = (lane == j) ? col : row1;
                 }
                 uint32_t lo = 0;
-                const uint64_t part = sct64<true>(a, k, row1, cx >= 64 ? ~0ull : ((1ull << cx) - 1), h, p, nodes, lo);
+                const uint64_t part = sct64_wide(a, k, row1, cx >= 64 ? ~0ull : ((1ull << cx) - 1), h, p, nodes, lo);
                 add_checked(acc, wave_total(part, lo, ovf), ovf);
                 --my_nodes;  // counted again as the subtree's root
             } else if (!LOCAL && crows4 && cx > 128 && cx <= 256 && h + 3 <= k && h + p + cx >= k) {
@@ -1237,7 +1263,7 @@ __device__ uint64_t pivot_count(const CountArgs &a, uint32_t P, uint32_t k, cons
                 }
                 sync_tree<WIDE>();
                 uint32_t lo = 0;
-                const uint64_t part = pivot_reg<4, true>(a, k, crows4, cx, h, cand, nodes, lo, p, crows2);
+                const uint64_t part = pivot_reg<4, WIDE_SCT>(a, k, crows4, cx, h, cand, nodes, lo, p, crows2);
                 add_checked(acc, wave_total(part, lo, ovf), ovf);
                 --my_nodes;
             } else if (!LOCAL && crows2 && cx <= 128 && h + 3 <= k && h + p + cx >= k) {
@@ -1254,7 +1280,7 @@ __device__ uint64_t pivot_count(const CountArgs &a, uint32_t P, uint32_t k, cons
                 }
                 sync_tree<WIDE>();
                 uint32_t lo = 0;
-                const uint64_t part = pivot_reg<2>(a, k, crows2, cx, h, cand, nodes, lo, p, nullptr);
+                const uint64_t part = pivot_reg<2, WIDE_SCT>(a, k, crows2, cx, h, cand, nodes, lo, p, nullptr);
                 add_checked(acc, wave_total(part, lo, ovf), ovf);
                 --my_nodes;
             } else if (h + p + cx >= k) {
@@ -1407,7 +1433,7 @@ __device__ inline uint64_t lds_row_word(const uint64_t *rows, uint32_t W, uint32
 // of X) and finished by sct64.  Lane i loads the full row of the i-th member
 // from the LDS copy; new row j is the ballot over lanes of bit x_j of those
 // rows (the bitmap is symmetric).  Cost ~ 6 instructions per member.
-template <int S>
+template <int S, Kind KIND>
 __device__ uint64_t compact_and_count(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t W,
                                       const uint64_t (&X)[S], uint32_t *idx, uint32_t h, uint32_t p,
                                       uint64_t &nodes, uint32_t &ovf)
@@ -1438,7 +1464,7 @@ __device__ uint64_t compact_and_count(const CountArgs &a, uint32_t k, const uint
         }
     }
     const uint64_t X1 = cx >= 64 ? ~0ull : ((1ull << cx) - 1);
-    return sct64<true>(a, k, row1, X1, h, p, nodes, ovf);
+    return KIND == WIDE_SCT ? sct64_wide(a, k, row1, X1, h, p, nodes, ovf) : sct64<KIND>(a, k, row1, X1, h, p, nodes, ovf);
 }
 
 // Triangles of G[X] for X of up to 64*S vertices (rows of stride W in LDS) by
@@ -1518,13 +1544,13 @@ __device__ uint32_t tri_lanes(const uint64_t *rows, uint32_t W, const uint64_t (
 
 // The counts of close_word for X of up to 64*S vertices (rows of stride W in
 // LDS): lane l takes the vertices l + 64s, s < S, with their complement rows in
-// S words each.  Two words go through the matrix cores like one; over four
-// (the wide kernel) the operands would not fit the registers, and a uniform
-// walk over u in X keeps the four running sums of each vertex, summed over
-// the lanes in 64 bits (C(256,4) * 24 does not fit 32).  Used at h = k-4 when X
+// S words each.  With MM two words go through the matrix cores like one; else
+// (over four words the operands would not fit the registers) a uniform walk
+// over u in X keeps the four running sums of each vertex, summed over the
+// lanes in 64 bits (C(256,4) * 24 does not fit 32).  Used at h = k-4 when X
 // is a near-clique (the K4 walk, over the vertices in three or more complement
 // triangles, stays short).
-template <int S>
+template <int S, bool MM>
 __device__ CliqueCounts k34_complement_rows(const uint64_t *rows, uint32_t W, const uint64_t (&X)[S], uint32_t cx)
 {
     const uint32_t lane = (uint32_t)lane_id();
@@ -1544,9 +1570,9 @@ __device__ CliqueCounts k34_complement_rows(const uint64_t *rows, uint32_t W, co
         }
     }
     uint64_t T3[S];
-    uint32_t s4 = 0, s3 = 0, s2 = 0;  // (S = 2)
+    uint32_t s4 = 0, s3 = 0, s2 = 0;  // (MM)
     uint32_t q[S], qE[S], t2[S], sd[S];
-    if constexpr (S == 2) {
+    if constexpr (S == 2 && MM) {
         uint32_t H[4][4], t3[4], live = 0;
 #pragma unroll
         for (int s = 0; s < 2; ++s)
@@ -1637,7 +1663,7 @@ __device__ CliqueCounts k34_complement_rows(const uint64_t *rows, uint32_t W, co
             }
         }
     }
-    if constexpr (S == 2) {
+    if constexpr (S == 2 && MM) {
         s4 += 24 * (uint32_t)(k4acc[0] + k4acc[1]);
         return complement_counts(cx, wave_sum32(s2) / 2, wave_sum32(s3), wave_sum32(s4));
     }
@@ -1672,7 +1698,7 @@ __device__ CliqueCounts k34_complement_rows(const uint64_t *rows, uint32_t W, co
 // quarter of the four-word ones.  Lanes l and l+64 load the full rows of
 // members l and l+64; word t of new row j is the ballot over lanes of bit x_j
 // of the rows of members 64t + lane (the bitmap is symmetric).
-template <int S>
+template <int S, Kind KIND>
 __device__ uint64_t compact2_and_count(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t W,
                                        const uint64_t (&X)[S], uint32_t *idx, uint64_t *crows, uint32_t h, uint32_t p,
                                        uint64_t &nodes, uint32_t &ovf, uint32_t wv, uint32_t nw)
@@ -1705,14 +1731,14 @@ __device__ uint64_t compact2_and_count(const CountArgs &a, uint32_t k, const uin
         }
     }
     sync_tree<true>();
-    return pivot_reg<2>(a, k, crows, cx, h, idx, nodes, ovf, p, nullptr, wv, nw);
+    return pivot_reg<2, KIND>(a, k, crows, cx, h, idx, nodes, ovf, p, nullptr, wv, nw);
 }
 
 // nw > 1: this wave is number wv of nw that walk the same subtree, each with
 // its own idx and crows: all of them walk the root's pivot chain (the nodes
 // with h0 held), each takes every nw-th branch off it, and what a chain node
 // itself adds is wave 0's.
-template <int S, bool CL4>
+template <int S, Kind KIND>
 __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t R, uint32_t h0,
                               uint32_t *idx, uint64_t &nodes, uint32_t &ovf, uint32_t p0, uint64_t *crows, uint32_t wv,
                               uint32_t nw)
@@ -1725,7 +1751,7 @@ __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *ro
     const uint32_t W = (R + 63) / 64;
     if (S == 1) {
         const uint64_t r1 = lane < R ? rows[lane] : 0ull;
-        return sct64<false>(a, k, r1, R >= 64 ? ~0ull : ((1ull << R) - 1), h0, p0, nodes, ovf);
+        return sct64<LEAN>(a, k, r1, R >= 64 ? ~0ull : ((1ull << R) - 1), h0, p0, nodes, ovf);
     }
     // rows of the lane in VGPRs for the two-word kernel; the four-word level
     // (a small share of the work once subtrees of <= 128 candidates are
@@ -1769,12 +1795,12 @@ __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *ro
             for (int w = 0; w < S; ++w) cx += (uint32_t)__popcll(X[w]);
             if (S == 4 && cx > 64 && cx <= 128 && h + 3 <= k && h + p + cx >= k) {
                 // a subtree of at most 128 candidates: two words per row from here on
-                add_checked(acc, compact2_and_count<S>(a, k, rows, W, X, idx, crows, h, p, nodes, ovf, chain ? wv : 0u,
+                add_checked(acc, compact2_and_count<S, KIND>(a, k, rows, W, X, idx, crows, h, p, nodes, ovf, chain ? wv : 0u,
                                                           chain ? nw : 1u),
                             ovf);
             } else if (cx <= 64 && cx > 0 && h + 3 <= k && h + p + cx >= k) {
                 // a subtree of at most 64 candidates: one word per row from here on
-                if (solo) add_checked(acc, compact_and_count<S>(a, k, rows, W, X, idx, h, p, nodes, ovf), ovf);
+                if (solo) add_checked(acc, compact_and_count<S, KIND>(a, k, rows, W, X, idx, h, p, nodes, ovf), ovf);
             } else if (my_nodes += solo, h + p + cx >= k) {
                 // scores |X & row_j| of the lane's member rows; key packs
                 // (score + 1, 0xFFFF - j), so the wave max names the smallest j of
@@ -1794,14 +1820,14 @@ __device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *ro
                 }
                 uint32_t e2 = 0;  // twice the edges of G[X]
                 if (need <= 4) e2 = wave_sum32(lsum);
-                const bool near = (S == 2 || (S == 4 && CL4)) && need == 4 && 4 * (uint64_t)e2 >= 3ull * cx * (cx - 1);
+                const bool near = (S == 2 || (S == 4 && KIND == WIDE_SCT)) && need == 4 && 4 * (uint64_t)e2 >= 3ull * cx * (cx - 1);
                 if (near || need <= 3 || cx == 0) {
                     if (!solo) break;  // (a chain node that closes ends the chain: the wave's branches are done)
                     // closed forms: h >= k-3, and h = k-4 over a near-clique (complement
                     // density <= 1/4)
-                    const CloseTerm term(a, need, p);
+                    const CloseTerm<KIND == WIDE_SCT> term(a, need, p);
                     CliqueCounts c{0, 0, 0};
-                    if (near && cx) c = k34_complement_rows<S>(rows, W, X, cx);
+                    if (near && cx) c = k34_complement_rows<S, KIND == MFMA>(rows, W, X, cx);
                     else if (need >= 2) c.e = e2 / 2;
                     if (need == 3 && cx) c.c3 = tri_lanes<S>(rows, W, X, cx, e2, idx);
                     term.add(acc, ovf, cx, c);
@@ -2178,7 +2204,7 @@ void k_pivot_reg(CountArgs a)
             if (!made) build_rows<true>(g, list, offs, starts, S == 1 ? keys : nullptr, rows, R, (R + 63) / 64, bytes);
             if (lane == 0) st[1] += bytes;
             uint64_t nodes = 0;
-            add_checked(w.run, pivot_reg<S>(a, g.k, rows, R, g.gran ? 2u : 1u, offs, nodes, w.run_ovf, 0u, crows),
+            add_checked(w.run, pivot_reg<S, MFMA>(a, g.k, rows, R, g.gran ? 2u : 1u, offs, nodes, w.run_ovf, 0u, crows),
                         w.run_ovf);
             __syncthreads();
             if (lane == 0) {
@@ -2388,7 +2414,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) void k_
                 __syncthreads();
                 build_rows<true>(g, list, offs, starts, nullptr, rows, R, (R + 63) / 64, w.bytes);
                 add_checked(w.run,
-                            pivot_reg<1>(a, g.k, rows, R, g.gran ? 2u : 1u, offs, w.nodes, w.run_ovf, 0u, nullptr),
+                            pivot_reg<1, LEAN>(a, g.k, rows, R, g.gran ? 2u : 1u, offs, w.nodes, w.run_ovf, 0u, nullptr),
                             w.run_ovf);
             }
         }
@@ -2761,7 +2787,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
         } else {
             if (!uni32(ctl[2])) build_rows_block(g, list, offs, starts, rows, R, (R + 63) / 64, bytes);
             uint64_t nodes = 0;
-            add_checked(w.run, pivot_reg<4>(a, g.k, rows, R, g.gran ? 2u : 1u, idx, nodes, w.run_ovf, 0u, crows, wv, NW),
+            add_checked(w.run, pivot_reg<4, MFMA>(a, g.k, rows, R, g.gran ? 2u : 1u, idx, nodes, w.run_ovf, 0u, crows, wv, NW),
                         w.run_ovf);
             if (lane == 0) atomicAdd((unsigned long long *)&st[3], (unsigned long long)nodes);
         }
