@@ -2158,9 +2158,9 @@ __device__ __attribute__((always_inline)) uint32_t next_tasks(const CountArgs &a
 }
 
 // register-bitmap pivoting kernel for tasks of at most 64*S vertices
-// waves per SIMD the register budget is held to: 4 for S = 4 and 2 (<= 128 VGPRs), 8 for S = 1
-template <int S>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S == 1 ? 8 : 4)))
+// waves per SIMD the register budget is held to: 4 (<= 128 VGPRs), 8 for S = 1, 6 for S = 2 LEAN
+template <int S, Kind KIND>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S == 1 ? 8 : S == 2 && KIND == LEAN ? 6 : 4)))
 void k_pivot_reg(CountArgs a)
 {
     extern __shared__ uint64_t lds[];
@@ -2204,7 +2204,7 @@ void k_pivot_reg(CountArgs a)
             if (!made) build_rows<true>(g, list, offs, starts, S == 1 ? keys : nullptr, rows, R, (R + 63) / 64, bytes);
             if (lane == 0) st[1] += bytes;
             uint64_t nodes = 0;
-            add_checked(w.run, pivot_reg<S, MFMA>(a, g.k, rows, R, g.gran ? 2u : 1u, offs, nodes, w.run_ovf, 0u, crows),
+            add_checked(w.run, pivot_reg<S, KIND>(a, g.k, rows, R, g.gran ? 2u : 1u, offs, nodes, w.run_ovf, 0u, crows),
                         w.run_ovf);
             __syncthreads();
             if (lane == 0) {
@@ -3379,12 +3379,14 @@ static const void *generic_kernel(bool pivot, bool global, bool local)
     return k[(local ? 4 : 0) + (pivot ? 2 : 0) + (global ? 1 : 0)];
 }
 
-static const void *register_kernel(int c)
+static const void *register_kernel(int c, bool deep)
 {
-    static const void *const reg[3] = {reinterpret_cast<const void *>(&k_pivot_reg<1>),
-                                       reinterpret_cast<const void *>(&k_pivot_reg<2>),
-                                       reinterpret_cast<const void *>(&k_pivot_reg<4>)};
-    return reg[c];
+    static const void *const reg[5] = {reinterpret_cast<const void *>(&k_pivot_reg<1, LEAN>),
+                                       reinterpret_cast<const void *>(&k_pivot_reg<2, LEAN>),
+                                       reinterpret_cast<const void *>(&k_pivot_reg<4, LEAN>),
+                                       reinterpret_cast<const void *>(&k_pivot_reg<2, MFMA>),
+                                       reinterpret_cast<const void *>(&k_pivot_reg<4, MFMA>)};
+    return reg[deep && c > 0 ? c + 2 : c];
 }
 
 // exact C(n, r) for n <= nmax, r <= rmax; ovf[i] = 1 when it exceeds 2^64-1
@@ -3491,11 +3493,20 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     // per query: two sums, then a flag (the sums of a single query are in the accumulators)
     const size_t q_bytes = sizeof(uint64_t) * 2 * nq + sizeof(uint32_t) * nq;
     bool any_pivot = false, any_edge = false, one_algo = true;
+    // Five or more vertices below the root of some pivoting task: its tree is walked,
+    // and most of the time goes to closing its nodes, for which the two- and
+    // four-word kernels have the matrix cores.  With fewer, most roots close by
+    // themselves; the operands' registers then only cost waves and spills.  Edge
+    // tasks, ms, without / with matrix cores: Chung-Lu n=1.7M k=5 17.5 / 19.9, k=6
+    // 26.6 / 30.7, k=7 79 / 73, k=8 434 / 357; R-MAT scale 22 k=5, 65..128 vertices 341
+    // / 476, 129..256 982 / 1196; k=8, 1 of 1024, both 165 / 138.
+    bool deep = false;
     uint32_t max_out = 0;  // bounds every task's size
     for (uint32_t i = 0; i < nq; ++i) {
         any_pivot |= halgo[i] != 0;
         any_edge |= hq[i].gran == KC_GRAN_EDGE;
         one_algo &= halgo[i] == halgo[0];
+        deep |= halgo[i] && hq[i].k >= (hq[i].gran == KC_GRAN_EDGE ? 7u : 6u);
         max_out = std::max(max_out, qs[i].o->max_out);
     }
     const uint32_t bstride = kmax + 1, brows = max_out + 2;
@@ -3742,7 +3753,7 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         const void *kern = generic_kernel(pivot, global, lc);
         variant[b] = global ? 3u : 1u;
         if (pivot && !global && c <= 2 && !lc) {
-            kern = register_kernel(c);
+            kern = register_kernel(c, deep);
             L = make_layout(a.rmax, a.wmax, 0, 0, true);
             variant[b] = 2u;
         }

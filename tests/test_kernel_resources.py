@@ -62,3 +62,10 @@ def test_wide_kernel_keeps_its_registers(kernels):
     for name, m in _named(kernels, "k_pivot_wide").items():
         assert m[".vgpr_spill_count"] == 0 and m[".sgpr_spill_count"] <= 200, name
         assert m[".private_segment_fixed_size"] <= 288, name
+
+
+def test_shallow_register_kernels_keep_their_registers(kernels):
+    """the two- and four-word kernels without matrix operands: few registers spilled"""
+    for part, spills in (("k_pivot_regILi2ELNS_4KindE1E", 60), ("k_pivot_regILi4ELNS_4KindE1E", 32)):
+        for name, m in _named(kernels, part).items():
+            assert m[".vgpr_spill_count"] <= spills, name
