@@ -514,7 +514,10 @@ struct CliqueCounts {
 //         registers at every call (R-MAT scale 22: edge tasks of 257..512 vertices
 //         at k=5 2.16 s, 1.69 s now, node tasks above 512 0.84 -> 0.73 s; 1/1024 of
 //         the edge tasks at k=8, both classes, 1.51 + 1.92 -> 1.22 + 1.58 s)
-enum Kind { MFMA, LEAN, WIDE_SCT };
+//   OPEN_SCT  the serving loop's resident kernel: as LEAN, without the step from 64-
+//         to 32-vertex words inside a walk, whose two stacks do not fit its 64
+//         registers together
+enum Kind { MFMA, LEAN, WIDE_SCT, OPEN_SCT };
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
@@ -764,7 +767,7 @@ __device__ inline uint64_t wave_total(uint64_t x, uint32_t lane_ovf, uint32_t &o
 // (close_word), and, at any h, once at most four candidates are left, which cannot hold a 5-clique.  Candidates
 // adjacent to all others lie in every maximal clique of X: they become pivots
 // together instead of one node each.  A 64-vertex subtree whose candidates
-// are at most 32 is re-encoded as a 32-vertex one.
+// are at most 32 is re-encoded as a 32-vertex one (not with OPEN_SCT).
 template <Kind KIND, class U>
 __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32_t h0, uint32_t p0, uint64_t &nodes,
                              uint32_t &ovf)
@@ -785,8 +788,8 @@ __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32
         uint32_t cx = bits_of(X);
         const uint32_t need = k - h;  // (h <= k)
         if (p + cx >= need) {
-            if (BITS == 64 && cx <= 32 && need >= 3 && cx > 0 && (!MM || need >= 5 || (uint32_t)((uint64_t)X >> 32) == 0)) {
-                if constexpr (BITS == 64) {
+            if (BITS == 64 && KIND != OPEN_SCT && cx <= 32 && need >= 3 && cx > 0 && (!MM || need >= 5 || (uint32_t)((uint64_t)X >> 32) == 0)) {
+                if constexpr (BITS == 64 && KIND != OPEN_SCT) {
                     uint32_t row1 = 0, X1 = (uint32_t)X;
                     if ((X >> 32) == 0) {
                         uint32_t up;
@@ -2245,7 +2248,7 @@ void k_pivot_reg(CountArgs a)
 constexpr uint32_t OPEN_STOP = 0xFFFFFFFFu;  // slot of a stop segment
 
 struct OpenArgs {
-    CountArgs c;              // binom, qcount / qovf per slot, acc (statistics)
+    CountArgs c;              // binom, qcount / qovf per slot
     uint64_t *counter;        // next task index
     uint64_t *known;          // task indices the device knows are published
     uint64_t *last_poll;      // wall clock of the last read of the host's total
@@ -2279,18 +2282,23 @@ __device__ inline void open_refresh(const OpenArgs &oa)
     if (h > ld_agent(oa.known)) __hip_atomic_fetch_max(oa.known, h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// the segment a wave last resolved an index in (indices a wave takes only grow)
+// The segment a wave last resolved an index in (indices a wave takes only grow;
+// desc = 0: none yet, no segment is empty).  It is in LDS, touched by lane 0
+// alone: it is needed once a task and would hold registers through the tree
+// walk.  With it there, statistics that nobody read, and the walk's step from 64- to
+// 32-vertex words, the kernel spilled 176 bytes a lane, none now: 220 queries on
+// Barabasi-Albert graphs of 3,000 to 100,000 vertices at k=4..8 5.3 -> 3.75 s, the
+// 110th answer after 1080 -> 839 ms (spills of 88 bytes still made it 890).
 struct SegCache {
-    uint64_t seg = 0, base = 0, desc = 0;
-    bool valid = false;
+    uint64_t seg, base, desc;
 };
 
 // lane 0: the segment holding published index i (segments are in base
 // order; binary search in host memory from the cached one)
 __device__ inline void open_resolve(const OpenArgs &oa, SegCache &sc, uint64_t i)
 {
-    if (sc.valid && i >= sc.base && i - sc.base < (uint32_t)sc.desc) return;
-    uint64_t lo = sc.valid ? sc.seg : 0, hi = ld_host(oa.hnseg);  // base[lo] <= i < total
+    if (i >= sc.base && i - sc.base < (uint32_t)sc.desc) return;
+    uint64_t lo = sc.seg, hi = ld_host(oa.hnseg);  // base[lo] <= i < total
     while (hi - lo > 1) {
         const uint64_t mid = (lo + hi) >> 1;
         if (ld_host(oa.hseg + 2 * mid) <= i) lo = mid;
@@ -2299,7 +2307,6 @@ __device__ inline void open_resolve(const OpenArgs &oa, SegCache &sc, uint64_t i
     sc.seg = lo;
     sc.base = ld_host(oa.hseg + 2 * lo);
     sc.desc = ld_host(oa.hseg + 2 * lo + 1);
-    sc.valid = true;
 }
 
 // flush the running count of the current slot and the tasks finished for it;
@@ -2334,6 +2341,17 @@ __device__ __attribute__((always_inline)) void open_flush(const OpenArgs &oa, Wa
     w.q = INF32;  // the slot may hold another query by the time this wave sees it again
 }
 
+// the SCT of a task of at most 64 vertices, in words of 32 where it has no more
+__device__ __attribute__((always_inline)) uint64_t open_tree(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t R,
+                                                            uint32_t h0, uint64_t &nodes, uint32_t &ovf)
+{
+    const uint32_t lane = (uint32_t)lane_id(), half = lane & 31;
+    if (R <= 32)
+        return sct_word<OPEN_SCT, uint32_t>(a, k, half < R ? (uint32_t)rows[half] : 0u, R == 32 ? ~0u : (1u << R) - 1, h0, 0u,
+                                            nodes, ovf);
+    return sct64<OPEN_SCT>(a, k, lane < R ? rows[lane] : 0ull, R == 64 ? ~0ull : (1ull << R) - 1, h0, 0u, nodes, ovf);
+}
+
 // one-word rows: every task of the graphs the resident launches take fits
 // 64 vertices, so the kernel keeps the one-word kernel's register budget
 // (eight waves per SIMD)
@@ -2348,7 +2366,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) void k_
     uint32_t *starts = reinterpret_cast<uint32_t *>(lds + L.starts);
     uint64_t *rows = lds + L.rows;
     WaveAcc w;
-    SegCache sc;
+    SegCache &sc = *reinterpret_cast<SegCache *>(lds + L.misc);
+    if (lane == 0) sc = SegCache{0, 0, 0};
     uint32_t pend = 0, seq = 0;
     uint64_t total = 0;
     Cur g{};
@@ -2403,25 +2422,24 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(8))) void k_
             total = d.total;
             seq = d.seq;
         }
-        ++w.ntask;
         ++pend;
-        const uint32_t R = stage_task(g, task, list, w.bytes);
+        uint64_t bytes = 0, nodes = 0;  // (statistics nobody asks for here)
+        const uint32_t R = stage_task(g, task, list, bytes);
         const uint32_t need = g.gran ? g.k - 2 : g.k - 1;
         if (R >= need) {
             if (g.gran && g.k == 3) {
                 run_add(w, R);
             } else {
                 __syncthreads();
-                build_rows<true>(g, list, offs, starts, nullptr, rows, R, (R + 63) / 64, w.bytes);
+                build_rows<true>(g, list, offs, starts, nullptr, rows, R, (R + 63) / 64, bytes);
                 add_checked(w.run,
-                            pivot_reg<1, LEAN>(a, g.k, rows, R, g.gran ? 2u : 1u, offs, w.nodes, w.run_ovf, 0u, nullptr),
+                            open_tree(a, g.k, rows, R, g.gran ? 2u : 1u, nodes, w.run_ovf),
                             w.run_ovf);
             }
         }
         __syncthreads();
     }
     open_flush(oa, w, pend, total, seq);
-    finish_wave(a, w);
 }
 
 // ---- the generic kernel: LDS (or HBM) bitmap, orientation or pivoting ------
@@ -3963,7 +3981,7 @@ int OpenEngine::init(int device)
         KC_HIP(hipEventCreateWithFlags(&q.done, hipEventDisableTiming));
     }
     if ((rc = qcount.ensure(8 * SLOTS)) || (rc = qovf.ensure(4 * SLOTS)) || (rc = qdone.ensure(8 * SLOTS)) ||
-        (rc = ctl.ensure(8 * CTL_WORDS * NQ)) || (rc = acc.ensure(8 * ACC)))
+        (rc = ctl.ensure(8 * CTL_WORDS * NQ)))
         return rc;
     const size_t qbytes = 16 + 16 * NSEG;  // total, nseg, then (base, slot|count) per segment
     const size_t bytes = NQ * qbytes + sizeof(OpenSlot) * SLOTS + sizeof(OpenMail) * SLOTS;
@@ -4093,7 +4111,6 @@ int OpenEngine::launch(int j)
     a.binom = binom.as<uint64_t>();
     a.binom_ovf = binom.as<uint8_t>() + (size_t)(OPEN_MAX_ROWS + 2) * (KC_MAX_K + 1) * 8;
     a.bstride = KC_MAX_K + 1;
-    a.acc = acc.as<uint64_t>();
     a.qcount = qcount.as<uint64_t>();
     a.qovf = qovf.as<uint32_t>();
     uint64_t *c = ctl.as<uint64_t>() + CTL_WORDS * j;

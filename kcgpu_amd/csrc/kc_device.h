@@ -177,7 +177,7 @@ struct OpenEngine {
     int dev = -1;
     hipStream_t adm = nullptr;       // set-up (init) only
     Queue qs[NQ];
-    DevBuf qcount, qovf, qdone, ctl, binom, acc;
+    DevBuf qcount, qovf, qdone, ctl, binom;
     uint8_t *pinned = nullptr;       // host: queues, slots, mailboxes
     uint8_t *pinned_dev = nullptr;   // the same memory's device address
     OpenSlot *hslot = nullptr;

@@ -69,3 +69,10 @@ def test_shallow_register_kernels_keep_their_registers(kernels):
     for part, spills in (("k_pivot_regILi2ELNS_4KindE1E", 60), ("k_pivot_regILi4ELNS_4KindE1E", 32)):
         for name, m in _named(kernels, part).items():
             assert m[".vgpr_spill_count"] <= spills, name
+
+
+def test_resident_launch_keeps_its_registers(kernels):
+    """the serving loop's resident kernel: eight waves per SIMD and no vector register spilled"""
+    for name, m in _named(kernels, "k_pivot_open").items():
+        assert m[".vgpr_count"] <= 64 and m[".vgpr_spill_count"] == 0, name
+        assert m[".private_segment_fixed_size"] == 0, name
