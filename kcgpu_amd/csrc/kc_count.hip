@@ -2142,6 +2142,9 @@ __device__ __attribute__((always_inline)) uint32_t next_tasks(const CountArgs &a
         tq.left = 0;
         return mine ? uni32(blockIdx.x << a.chunk_log) : INF32;
     }
+    // with fewer chunks than blocks (the host sizes a one-bin launch by the tasks
+    // before binning) the blocks past their number leave the heads alone
+    if (((uint64_t)blockIdx.x << a.chunk_log) >= a.ntasks) return INF32;
     for (;;) {
         uint32_t i = 0;
         if (lane == 0) i = atomicAdd(&a.qhead[tq.queue * QSTRIDE], 1u);
