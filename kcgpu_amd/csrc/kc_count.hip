@@ -1149,19 +1149,27 @@ __device__ uint32_t tri_lanes(const uint64_t *rows, uint32_t W, const uint64_t (
 // (WIDE_SCT: four words close h = k-4 near-cliques too; the wide kernel has the
 // registers for it, the one-wave four-word kernel keeps its budget)
 template <int S, Kind KIND>
-__device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t R, uint32_t h0,
+__device__ __attribute__((always_inline)) uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t R, uint32_t h0,
                               uint32_t *idx, uint64_t &nodes, uint32_t &ovf, uint32_t p0, uint64_t *crows, uint32_t wv = 0,
                               uint32_t nw = 1);
 
 // triangles of G[X] with X in LDS (W words): the lane walks with the words in registers
+// (inline, except the sixteen-word walk; build_rows_block likewise: what the wide
+// kernel has inline is fixed here, it decides what it spills)
 template <int S>
-__device__ uint32_t tri_lds(const uint64_t *rows, uint32_t W, const uint64_t *X, uint32_t cx, uint32_t e2,
+__device__ __attribute__((always_inline)) uint32_t tri_lds(const uint64_t *rows, uint32_t W, const uint64_t *X, uint32_t cx, uint32_t e2,
                             uint32_t *idx)
 {
     uint64_t Xr[S];
 #pragma unroll
     for (int w = 0; w < S; ++w) Xr[w] = (uint32_t)w < W ? uni64(X[w]) : 0ull;
     return tri_lanes<S>(rows, W, Xr, cx, e2, idx);
+}
+
+__device__ __attribute__((noinline)) uint32_t tri_lds16(const uint64_t *rows, uint32_t W, const uint64_t *X, uint32_t cx,
+                                                        uint32_t e2, uint32_t *idx)
+{
+    return tri_lds<16>(rows, W, X, cx, e2, idx);
 }
 
 // (inline always: as a function of its own it saved and restored its registers for
@@ -1351,7 +1359,7 @@ __device__ __attribute__((always_inline)) uint64_t pivot_count(const CountArgs &
                     const uint32_t e2 = (uint32_t)tot_s;
                     const uint32_t tri = W <= 4 ? tri_lds<4>(rows, W, X, cx, e2, cand)
                                          : W <= 8 ? tri_lds<8>(rows, W, X, cx, e2, cand)
-                                                  : tri_lds<16>(rows, W, X, cx, e2, cand);
+                                                  : tri_lds16(rows, W, X, cx, e2, cand);
                     add_checked(acc, close_k3(a, p, cx, tot_s / 2, tri, ovf), ovf);
                 } else if (h + p + max_s + 1 >= k) {
                     const uint32_t pv = INF32 - (uint32_t)(key & 0xFFFFFFFFull);
@@ -1742,7 +1750,7 @@ __device__ uint64_t compact2_and_count(const CountArgs &a, uint32_t k, const uin
 // with h0 held), each takes every nw-th branch off it, and what a chain node
 // itself adds is wave 0's.
 template <int S, Kind KIND>
-__device__ uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t R, uint32_t h0,
+__device__ __attribute__((always_inline)) uint64_t pivot_reg(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t R, uint32_t h0,
                               uint32_t *idx, uint64_t &nodes, uint32_t &ovf, uint32_t p0, uint64_t *crows, uint32_t wv,
                               uint32_t nw)
 {
@@ -2574,7 +2582,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(S == 1 ? 6 :
     finish_wave(a, w);
 }
 
-template <bool PIVOT, bool GLOBAL, bool LOCAL>
+// SMALL: the orientation's tasks of at most 128 vertices in LDS, whose rows may come
+// from the adjacency words (Chung-Lu n=200,000, k=5, edge tasks 0.95 -> 0.71 ms a
+// call, n=300,000, k=4 1.27 -> 0.61) or pair by pair.  The registers of both ways
+// cost the larger tasks, whose DFS is the time: R-MAT scale 18, node tasks at k=5
+// in degeneracy order 218 ms with them in every instance, 205 so.
+template <bool PIVOT, bool GLOBAL, bool LOCAL, bool SMALL>
 __global__ __launch_bounds__(64) void k_count(CountArgs a)
 {
     extern __shared__ uint64_t lds[];
@@ -2585,7 +2598,7 @@ __global__ __launch_bounds__(64) void k_count(CountArgs a)
     uint32_t *list = reinterpret_cast<uint32_t *>(ws + L.list);
     uint32_t *offs = reinterpret_cast<uint32_t *>(ws + L.offs);
     uint32_t *starts = reinterpret_cast<uint32_t *>(ws + L.starts);
-    uint32_t *keys = a.rmax <= PAIR_ROWS ? reinterpret_cast<uint32_t *>(ws + L.keys) : nullptr;
+    uint32_t *keys = SMALL && a.rmax <= PAIR_ROWS ? reinterpret_cast<uint32_t *>(ws + L.keys) : nullptr;
     uint64_t *rows = ws + L.rows;
     uint64_t *stk = ws + L.stk;
     uint64_t *X = ws + L.x;
@@ -2605,10 +2618,7 @@ __global__ __launch_bounds__(64) void k_count(CountArgs a)
             const Cur g = select_task(a, a.tasks[ti], w, task);
             const uint32_t k = g.k;
             ++w.ntask;
-            // (the orientation's tasks up to 128 vertices: Chung-Lu n=200,000, k=5, edge
-            // tasks 0.95 -> 0.71 ms a call, n=300,000, k=4 1.27 -> 0.61; with the four words
-            // of larger tasks too the registers cost waves: 0.75, 0.64)
-            const bool made = !PIVOT && !GLOBAL && a.rmax <= 128 && has_bits(a, g, task);
+            const bool made = SMALL && has_bits(a, g, task);
             const uint32_t R = !made          ? stage_task(g, task, list, w.bytes)
                                : a.rmax <= 64 ? rows_from_bits<1, LOCAL, false>(a, g, task, list, rows, w.bytes)
                                               : rows_from_bits<2, LOCAL, false>(a, g, task, list, rows, w.bytes);
@@ -2694,7 +2704,7 @@ __host__ __device__ inline WideLayout make_wide_layout(uint32_t rmax, uint32_t w
 
 // bitmap rows of the task by every thread of the block (build_rows with the
 // row offsets scanned by wave 0)
-__device__ void build_rows_block(const Cur &g, const uint32_t *list, uint32_t *offs, uint32_t *starts, uint64_t *rows,
+__device__ __attribute__((noinline)) void build_rows_block(const Cur &g, const uint32_t *list, uint32_t *offs, uint32_t *starts, uint64_t *rows,
                                  uint32_t R, uint32_t W, uint64_t &bytes)
 {
     const uint32_t tid = threadIdx.x, nt = blockDim.x, lane = tid & 63;
@@ -3386,18 +3396,21 @@ __global__ __launch_bounds__(BIN_T) void k_bin_scatter(BinArgs b)
 }
 
 // ---- host -------------------------------------------------------------------
-static const void *generic_kernel(bool pivot, bool global, bool local)
+static const void *generic_kernel(bool pivot, bool global, bool local, bool small)
 {
-    static const void *const k[8] = {
-        reinterpret_cast<const void *>(&k_count<false, false, false>),
-        reinterpret_cast<const void *>(&k_count<false, true, false>),
-        reinterpret_cast<const void *>(&k_count<true, false, false>),
-        reinterpret_cast<const void *>(&k_count<true, true, false>),
-        reinterpret_cast<const void *>(&k_count<false, false, true>),
-        reinterpret_cast<const void *>(&k_count<false, true, true>),
-        reinterpret_cast<const void *>(&k_count<true, false, true>),
-        reinterpret_cast<const void *>(&k_count<true, true, true>)};
-    return k[(local ? 4 : 0) + (pivot ? 2 : 0) + (global ? 1 : 0)];
+    if (pivot) {  // (per-vertex counts; the others have kernels of their own)
+        if (!local) return nullptr;
+        return global ? reinterpret_cast<const void *>(&k_count<true, true, true, false>)
+                      : reinterpret_cast<const void *>(&k_count<true, false, true, false>);
+    }
+    static const void *const k[6] = {
+        reinterpret_cast<const void *>(&k_count<false, false, false, true>),
+        reinterpret_cast<const void *>(&k_count<false, false, false, false>),
+        reinterpret_cast<const void *>(&k_count<false, true, false, false>),
+        reinterpret_cast<const void *>(&k_count<false, false, true, true>),
+        reinterpret_cast<const void *>(&k_count<false, false, true, false>),
+        reinterpret_cast<const void *>(&k_count<false, true, true, false>)};
+    return k[(local ? 3 : 0) + (global ? 2 : small ? 0 : 1)];
 }
 
 static const void *register_kernel(int c, bool deep)
@@ -3771,7 +3784,7 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         }
         if (!global && L.total * 8 > lds_cap) global = true;  // same layout in HBM
         a.nparts = np;
-        const void *kern = generic_kernel(pivot, global, lc);
+        const void *kern = generic_kernel(pivot, global, lc, c <= 1);
         variant[b] = global ? 3u : 1u;
         if (pivot && !global && c <= 2 && !lc) {
             kern = register_kernel(c, deep);
@@ -3819,6 +3832,7 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
             L.total = WL.total;
             variant[b] = global ? 5u : 4u;
         }
+        if (!kern) return fail(KC_ERR_DEVICE, "no kernel for tasks of %u vertices (internal error)", a.rmax);
         const size_t lds = global ? 0 : L.total * 8;
         if (!global) KC_HIP(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         int per_cu = 0;

@@ -76,3 +76,12 @@ def test_resident_launch_keeps_its_registers(kernels):
     for name, m in _named(kernels, "k_pivot_open").items():
         assert m[".vgpr_count"] <= 64 and m[".vgpr_spill_count"] == 0, name
         assert m[".private_segment_fixed_size"] == 0, name
+
+
+def test_generic_kernel_instances(kernels):
+    """only the instances that a launch can take; the large classes' without the small ones' registers"""
+    names = _named(kernels, "7k_countILb")
+    assert len(names) == 8
+    for part in ("7k_countILb0ELb0ELb0ELb0E", "7k_countILb0ELb1ELb0ELb0E"):
+        for name, m in _named(kernels, part).items():
+            assert m[".vgpr_count"] <= 64 and m[".private_segment_fixed_size"] == 0, name
