@@ -244,7 +244,8 @@ int build_csr_device(DeviceCtx *ctx, hipStream_t s, uint32_t n_in, size_t ne, co
 {
     if (2.0 * (double)ne >= 4294967295.0)
         return fail(KC_ERR_LIMIT, "%zu edges: %zu CSR entries exceed 32-bit offsets", ne, 2 * ne);
-    DevBuf es, ed, small;
+    DevBuf es, ed, small, deg, off, rank, tmp, ucnt, big, scan_tmp, bm;
+    StreamWait wait(s);  // (no return frees them, or the caller's rowptr and col, with a kernel running)
     int rc;
     if ((rc = es.ensure(4 * ne + 4)) || (rc = ed.ensure(4 * ne + 4)) || (rc = small.ensure(64))) return rc;
     if (ne) {
@@ -265,7 +266,6 @@ int build_csr_device(DeviceCtx *ctx, hipStream_t s, uint32_t n_in, size_t ne, co
     if (h[1] && h[0] >= nn) return fail(KC_ERR_ARG, "vertex id %u >= n=%llu", h[0], (unsigned long long)nn);
     if (nn >= 0xFFFFFFFFull) return fail(KC_ERR_LIMIT, "n=%llu does not fit 32-bit ids", (unsigned long long)nn);
     const uint32_t n = (uint32_t)nn;
-    DevBuf deg, off, rank, tmp, ucnt, big, scan_tmp;
     if ((rc = deg.ensure(4 * ((size_t)n + 1))) || (rc = off.ensure(4 * ((size_t)n + 1))) ||
         (rc = rank.ensure(8 * ne + 8)) || (rc = tmp.ensure(8 * ne + 4)) ||
         (rc = ucnt.ensure(4 * ((size_t)n + 1))) || (rc = big.ensure(4 * ((size_t)n + 1))) ||
@@ -292,12 +292,12 @@ int build_csr_device(DeviceCtx *ctx, hipStream_t s, uint32_t n_in, size_t ne, co
         // one bitmap slice per block, at most 1 GiB of them in all
         const uint64_t fit = std::max<uint64_t>(1, (1ull << 30) / (8ull * words));
         const uint32_t nb = (uint32_t)std::min<uint64_t>({(uint64_t)nbig, (uint64_t)ctx->cu, fit});
-        DevBuf bm;
         if ((rc = bm.ensure(8ull * words * nb))) return rc;
         hipLaunchKernelGGL(k_row_sort_big, dim3(nb), dim3(BUILD_T), 0, s, off.as<uint32_t>(), big.as<uint32_t>(), nbig,
                            tmp.as<uint32_t>(), ucnt.as<uint32_t>(), bm.as<uint64_t>(), words);
         KC_HIP(hipGetLastError());
-        KC_HIP(hipStreamSynchronize(s));  // bm goes out of scope
+        KC_HIP(hipStreamSynchronize(s));
+        bm.release();
     }
     if ((rc = scan_exclusive_u32(ucnt.as<uint32_t>(), rowptr.as<uint32_t>(), n, scan_tmp, s))) return rc;
     uint32_t nnz = 0;
@@ -313,6 +313,7 @@ int build_csr_device(DeviceCtx *ctx, hipStream_t s, uint32_t n_in, size_t ne, co
     uint32_t md = 0;
     KC_HIP(hipMemcpyAsync(&md, sm + 3, 4, hipMemcpyDeviceToHost, s));
     KC_HIP(hipStreamSynchronize(s));
+    wait.done();
     n_out = n;
     nnz_out = nnz;
     maxdeg_out = md;

@@ -3563,6 +3563,10 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     std::memcpy(up.data(), hq.data(), qd_bytes);
     std::memcpy(up.data() + qd_bytes, hoff.data(), off_bytes);
     std::memcpy(up.data() + qd_bytes + off_bytes, halgo.data(), nq);
+    // accumulators, per-query sums and overflow flags lie side by side: one copy back
+    std::vector<uint64_t> back((acc_bytes + q_bytes + 7) / 8);
+    uint32_t h[NS + 16] = {0};
+    StreamWait wait(s);  // no return leaves a kernel running on the caller's scratch
     KC_HIP(hipMemcpyAsync(dq, up.data(), up.size(), hipMemcpyHostToDevice, s));
     {  // counters, queue heads and per-query sums start at zero (a fill kernel, no memset node)
         const uint64_t nz = (meta_u32 * 4 + acc_bytes + q_bytes) / 4;
@@ -3657,7 +3661,6 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     } else if (one_bin) {
         bcnt[halgo[0] ? NCLASS : 0] = (uint32_t)total;  // (at most)
     } else {
-        uint32_t h[NS + 16] = {0};
         KC_HIP(hipMemcpyAsync(h, m32, sizeof h, hipMemcpyDeviceToHost, s));
         KC_HIP(hipStreamSynchronize(s));
         uint64_t tot = 0;
@@ -3682,20 +3685,6 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     // s, and the side streams start after them: sharing the device with the
     // small classes delays the wide classes' long chain walks.  With
     // grid_share > 1 (a server worker) every launch stays on s.
-    // an error after the first launch waits for every launch before it
-    // returns, so that no kernel still runs on the caller's scratch
-    auto drain = [&]() {
-        hipStreamSynchronize(s);
-        for (hipStream_t st : ctx->side) hipStreamSynchronize(st);
-    };
-#define KC_HIP_L(call)                                                                              \
-    do {                                                                                           \
-        hipError_t e_ = (call);                                                                    \
-        if (e_ != hipSuccess) {                                                                    \
-            drain();                                                                               \
-            return kc::fail(KC_ERR_DEVICE, "%s failed: %s", #call, hipGetErrorString(e_));         \
-        }                                                                                          \
-    } while (0)
     if (!triangles) evs.record(evs.go, s);
     // Side by side only when the register classes hold few tasks per CU: then
     // a class's last long tasks are a large part of its launch (Chung-Lu
@@ -3867,34 +3856,33 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         hipStream_t st = s;
         if (fan && !l.global && b % NCLASS <= 2) {
             if (!fan_recorded && !few_wide) {
-                KC_HIP_L(hipEventRecord(evs.fan, s));  // after every launch so far on s
+                KC_HIP(hipEventRecord(evs.fan, s));  // after every launch so far on s
                 fan_recorded = true;
             }
             const int si = nside++ % DeviceCtx::NSIDE;
+            wait.side = ctx->side;
             st = ctx->side[si];
             if (!side_waits[si]) {
-                KC_HIP_L(hipStreamWaitEvent(st, few_wide ? evs.go : evs.fan, 0));
+                KC_HIP(hipStreamWaitEvent(st, few_wide ? evs.go : evs.fan, 0));
                 side_waits[si] = true;
             }
         }
         bin_stream[b] = st;
         if (plan.size() > 1 && !l.global)  // (two classes may share a kernel: the last plan's limit stands)
-            KC_HIP_L(hipFuncSetAttribute(l.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.lds));
+            KC_HIP(hipFuncSetAttribute(l.kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l.lds));
         void *args[] = {&l.a};
         evs.record(evs.b0[b], st);
-        KC_HIP_L(hipLaunchKernel(l.kern, dim3(l.blocks), dim3(64 * l.nw), args, l.lds, st));
+        KC_HIP(hipLaunchKernel(l.kern, dim3(l.blocks), dim3(64 * l.nw), args, l.lds, st));
         evs.record(evs.b1[b], st);
         launched[b] = true;
     }
     for (int b = 0; b < NB; ++b)
-        if (launched[b] && bin_stream[b] != s) KC_HIP_L(hipStreamWaitEvent(s, evs.b1[b], 0));
+        if (launched[b] && bin_stream[b] != s) KC_HIP(hipStreamWaitEvent(s, evs.b1[b], 0));
     evs.record(evs.end, s);
-    // accumulators, per-query sums and overflow flags lie side by side: one copy
-    std::vector<uint64_t> back((acc_bytes + q_bytes + 7) / 8);
-    KC_HIP_L(hipMemcpyAsync(back.data(), dacc, acc_bytes + q_bytes, hipMemcpyDeviceToHost, s));
+    KC_HIP(hipMemcpyAsync(back.data(), dacc, acc_bytes + q_bytes, hipMemcpyDeviceToHost, s));
     const hipError_t se = hipStreamSynchronize(s);
     if (se != hipSuccess) return fail(KC_ERR_DEVICE, "counting kernels failed: %s", hipGetErrorString(se));
-#undef KC_HIP_L
+    wait.done();
     uint64_t hacc[NB * ACC] = {0};
     for (int b = 0; b < NB; ++b)
         for (uint32_t c = 0; c < NSTRIPE; ++c)

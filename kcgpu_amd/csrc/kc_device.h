@@ -64,6 +64,24 @@ struct DevBuf {
     };
 };
 
+// Waits for a stream (and the side streams) on the way out of a scope that queued
+// work on its own buffers, unless done() says that it has been waited for:
+// declared after those buffers, so that an early (error) return releases none
+// of them with that work still running.
+struct StreamWait {
+    hipStream_t s;
+    const hipStream_t *side = nullptr;
+    bool armed = true;
+    explicit StreamWait(hipStream_t st) : s(st) {}
+    ~StreamWait()
+    {
+        if (!armed) return;
+        hipStreamSynchronize(s);
+        for (int i = 0; side && i < DeviceCtx::NSIDE; ++i) hipStreamSynchronize(side[i]);
+    }
+    void done() { armed = false; }
+};
+
 // Exclusive scan of n uint32 counts into out[0..n] (out[n] = total); total
 // must fit 32 bits.  in and out may alias.  tmp is scratch owned by caller.
 int scan_exclusive_u32(const uint32_t *in, uint32_t *out, uint32_t n, DevBuf &tmp, hipStream_t s);

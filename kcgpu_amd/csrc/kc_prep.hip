@@ -1018,7 +1018,8 @@ struct Captured {
 static int run_peel(DeviceCtx *ctx, hipStream_t s, uint32_t n, uint32_t nnz, uint32_t maxdeg, const uint32_t *rowptr,
                     const uint32_t *col, uint32_t *prio, uint32_t *max_core)
 {
-    DevBuf deg, st, q0, q1, cnt;
+    DevBuf deg, st, q0, q1, cnt, more, ctlb;
+    StreamWait wait(s);
     int rc;
     if ((rc = deg.ensure(sizeof(int) * (size_t)n + 4)) || (rc = q0.ensure(sizeof(uint32_t) * (size_t)n + 4)) ||
         (rc = q1.ensure(sizeof(uint32_t) * (size_t)n + 4)) || (rc = cnt.ensure(sizeof(uint32_t) * 4)))
@@ -1028,7 +1029,7 @@ static int run_peel(DeviceCtx *ctx, hipStream_t s, uint32_t n, uint32_t nnz, uin
     bool coop = mode && std::strcmp(mode, "coop") == 0;
     if (!coop && !(mode && std::strcmp(mode, "step") == 0)) {
         const size_t nhub = (size_t)nnz / PEEL_HUB + 1, nl = (size_t)n / 4 + n / 16 + 2;
-        DevBuf more;  // hub queues, live lists, counters
+        // `more`: hub queues, live lists, counters
         const size_t at_list = 2 * nhub, at_shared = (at_list + nl + 1) & ~(size_t)1;
         if ((rc = more.ensure(4 * at_shared + sizeof(PeelShared)))) return rc;
         PeelRunArgs pa{};
@@ -1056,10 +1057,12 @@ static int run_peel(DeviceCtx *ctx, hipStream_t s, uint32_t n, uint32_t nnz, uin
         KC_HIP(hipMemcpyAsync(&h, pa.s, sizeof h, hipMemcpyDeviceToHost, s));
         KC_HIP(hipStreamSynchronize(s));
         if (h.done) {
+            wait.done();
             *max_core = h.max_core;
             return KC_OK;
         }
         if (!h.abort) return fail(KC_ERR_DEVICE, "peel did not converge (internal error)");
+        more.release();
     }
     if ((rc = st.ensure((size_t)n + 4))) return rc;
     int gi = (int)std::min<uint64_t>(((uint64_t)n + 255) / 256, (uint64_t)ctx->cu * 8);
@@ -1094,7 +1097,6 @@ static int run_peel(DeviceCtx *ctx, hipStream_t s, uint32_t n, uint32_t nnz, uin
         // and one 4-byte read per PEEL_STEPS peel rounds or levels.  Steps past
         // the end return at once.
         constexpr int PEEL_STEPS = 64;
-        DevBuf ctlb;
         if ((rc = ctlb.ensure(sizeof(PeelCtl)))) return rc;
         PeelCtl *ctl = ctlb.as<PeelCtl>();
         hipLaunchKernelGGL(k_peel_ctl_init, dim3(1), dim3(1), 0, s, ctl, a.cnt, n);
@@ -1126,6 +1128,7 @@ static int run_peel(DeviceCtx *ctx, hipStream_t s, uint32_t n, uint32_t nnz, uin
     uint32_t h[4];
     KC_HIP(hipMemcpyAsync(h, cnt.p, sizeof h, hipMemcpyDeviceToHost, s));
     KC_HIP(hipStreamSynchronize(s));
+    wait.done();
     if (h[3]) return fail(KC_ERR_DEVICE, "peel did not converge (internal error)");
     *max_core = h[2];
     return KC_OK;
@@ -1210,6 +1213,7 @@ int kc_orient(const kc_graph *g, int mode, kc_oriented **out)
     const uint32_t nnz = (uint32_t)g->csr.col.size();
     hipStream_t s = ctx->stream;
     DevBuf frow, fcol;
+    StreamWait wait(s);
     if ((rc = frow.ensure(sizeof(uint32_t) * ((size_t)n + 1))) || (rc = fcol.ensure(sizeof(uint32_t) * (size_t)nnz + 4)))
         return rc;
     if (hipMemcpyAsync(frow.p, g->csr.rowptr.data(), sizeof(uint32_t) * ((size_t)n + 1), hipMemcpyHostToDevice, s) !=
@@ -1217,7 +1221,9 @@ int kc_orient(const kc_graph *g, int mode, kc_oriented **out)
         (nnz && hipMemcpyAsync(fcol.p, g->csr.col.data(), sizeof(uint32_t) * (size_t)nnz, hipMemcpyHostToDevice, s) !=
                     hipSuccess))
         return fail(KC_ERR_DEVICE, "graph upload failed");
-    return orient_device_csr(ctx, n, nnz, g->max_degree, frow.as<uint32_t>(), fcol.as<uint32_t>(), mode, out);
+    rc = orient_device_csr(ctx, n, nnz, g->max_degree, frow.as<uint32_t>(), fcol.as<uint32_t>(), mode, out);
+    if (rc == KC_OK) wait.done();
+    return rc;
 }
 
 }  // extern "C"
@@ -1239,6 +1245,7 @@ int kc::orient_device_csr(DeviceCtx *ctx, uint32_t n, uint32_t nnz, uint32_t max
     hipStream_t s = o->stream;
     // every buffer is sized up front, so the launches need no host read in between
     DevBuf frow, fcol, outdeg, tmp, mx;
+    StreamWait wait(s);
     frow.view(const_cast<uint32_t *>(frow_p), sizeof(uint32_t) * ((size_t)n + 1));
     fcol.view(const_cast<uint32_t *>(fcol_p), sizeof(uint32_t) * (size_t)nnz + 4);
     const size_t np = ((size_t)n + 2047) / 2048;
@@ -1301,6 +1308,7 @@ int kc::orient_device_csr(DeviceCtx *ctx, uint32_t n, uint32_t nnz, uint32_t max
     KC_HIP(hipMemcpyAsync(&res[1], mx.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     const hipError_t se = hipStreamSynchronize(s);
     if (se != hipSuccess) return fail(KC_ERR_DEVICE, "orientation failed: %s", hipGetErrorString(se));
+    wait.done();
     if (res[0] != m_expect)
         return fail(KC_ERR_DEVICE, "orientation kept %u of %u edges (internal error)", res[0], m_expect);
     float ms = 0;
@@ -1329,9 +1337,7 @@ int kc_orient_edges(uint32_t n, size_t nedges, const uint32_t *src, const uint32
     uint32_t nv = 0, maxdeg = 0;
     uint64_t nnz = 0;
     if ((rc = build_csr_device(ctx, ctx->stream, n, nedges, src, dst, rp, col, nv, nnz, maxdeg))) return rc;
-    rc = orient_device_csr(ctx, nv, (uint32_t)nnz, maxdeg, rp.as<uint32_t>(), col.as<uint32_t>(), mode, out);
-    hipStreamSynchronize(ctx->stream);  // rp and col are freed on return
-    return rc;
+    return orient_device_csr(ctx, nv, (uint32_t)nnz, maxdeg, rp.as<uint32_t>(), col.as<uint32_t>(), mode, out);
 }
 
 // kc_graph_from_edges with the CSR built on the device and copied back
@@ -1347,12 +1353,14 @@ int kc_graph_from_edges_device(uint32_t n, size_t nedges, const uint32_t *src, c
     uint64_t nnz = 0;
     if ((rc = build_csr_device(ctx, ctx->stream, n, nedges, src, dst, rp, col, nv, nnz, maxdeg))) return rc;
     std::unique_ptr<kc_graph> g(new kc_graph);
+    StreamWait wait(ctx->stream);
     g->csr.n = nv;
     g->csr.rowptr.resize((size_t)nv + 1);
     g->csr.col.resize(nnz);
     KC_HIP(hipMemcpyAsync(g->csr.rowptr.data(), rp.p, 4 * ((size_t)nv + 1), hipMemcpyDeviceToHost, ctx->stream));
     if (nnz) KC_HIP(hipMemcpyAsync(g->csr.col.data(), col.p, 4 * nnz, hipMemcpyDeviceToHost, ctx->stream));
     KC_HIP(hipStreamSynchronize(ctx->stream));
+    wait.done();
     g->max_degree = maxdeg;
     *out = g.release();
     return KC_OK;
@@ -1382,9 +1390,16 @@ static int orient_degree_chunk(DeviceCtx *ctx, const kc_graph *const *gs, const 
     const uint64_t rp_words = (uint64_t)nrows + B, mtot = cbase[B];
     // pinned staging: full rowptrs, full cols, vbase, ebase
     const size_t stage_bytes = 4 * (rp_words + nent) + 4 * (B + 1) + 8 * B + 64;
-    uint8_t *stage = nullptr;
-    if (hipHostMalloc((void **)&stage, stage_bytes, hipHostMallocDefault) != hipSuccess)
+    struct Pinned {
+        uint8_t *p = nullptr;
+        ~Pinned()
+        {
+            if (p) hipHostFree(p);
+        }
+    } pinned;
+    if (hipHostMalloc((void **)&pinned.p, stage_bytes, hipHostMallocDefault) != hipSuccess)
         return fail(KC_ERR_NOMEM, "hipHostMalloc(%zu) failed", stage_bytes);
+    uint8_t *stage = pinned.p;
     uint32_t *h_frow = reinterpret_cast<uint32_t *>(stage);
     uint32_t *h_fcol = h_frow + rp_words;
     uint64_t *h_ebase = reinterpret_cast<uint64_t *>(stage + ((4 * (rp_words + nent) + 7) & ~(size_t)7));
@@ -1410,14 +1425,14 @@ static int orient_degree_chunk(DeviceCtx *ctx, const kc_graph *const *gs, const 
     const uint64_t a_rows = rp_words, a_col = a_rows, a_src = a_col + mtot, a_key = a_src + mtot,
                    a_words = a_key + nrows + 4;
     DevBuf din, dtmp, dscan, dmeta;
+    std::vector<uint32_t> maxout(B);
+    StreamWait wait(s);
     int rc;
     const size_t np = ((size_t)nrows + 2047) / 2048;
     if ((rc = arena->ensure(4 * a_words)) || (rc = din.ensure(4 * (rp_words + nent) + 8)) ||
         (rc = dscan.ensure(4 * (2 * (size_t)nrows + 2))) || (rc = dtmp.ensure(8 * (np + 1))) ||
-        (rc = dmeta.ensure(8 * B + 4 * (B + 1) + 4 * B + 64))) {
-        hipHostFree(stage);
+        (rc = dmeta.ensure(8 * B + 4 * (B + 1) + 4 * B + 64)))
         return rc;
-    }
     uint32_t *d_orow = arena->as<uint32_t>(), *d_ocol = d_orow + a_col, *d_osrc = d_orow + a_src,
              *d_key = d_orow + a_key;
     uint32_t *d_frow = din.as<uint32_t>(), *d_fcol = d_frow + rp_words;
@@ -1460,7 +1475,6 @@ static int orient_degree_chunk(DeviceCtx *ctx, const kc_graph *const *gs, const 
     if (captured) le = hipGraphLaunch(exec, s);
     else if ((rc = enqueue())) le = hipErrorUnknown;
     hipEventRecord(e1, s);
-    std::vector<uint32_t> maxout(B);
     if (le == hipSuccess) le = hipMemcpyAsync(maxout.data(), d_maxout, 4 * B, hipMemcpyDeviceToHost, s);
     const hipError_t se = hipStreamSynchronize(s);
     float ms = 0;
@@ -1469,7 +1483,7 @@ static int orient_degree_chunk(DeviceCtx *ctx, const kc_graph *const *gs, const 
     hipEventDestroy(e1);
     if (exec) hipGraphExecDestroy(exec);
     if (graph) hipGraphDestroy(graph);
-    hipHostFree(stage);
+    if (se == hipSuccess) wait.done();
     if (rc) return rc;
     if (le != hipSuccess || se != hipSuccess)
         return fail(KC_ERR_DEVICE, "batched orientation failed: %s", hipGetErrorString(le != hipSuccess ? le : se));
@@ -1685,6 +1699,7 @@ extern "C" int kc_oriented_load(const char *path, kc_oriented **out)
               (h.n == 0 || hipMemcpyAsync(o->key.p, key.data(), 4 * key.size(), hipMemcpyHostToDevice, s) == hipSuccess) &&
               hipStreamSynchronize(s) == hipSuccess;
     if (!up) {
+        hipStreamSynchronize(s);
         delete o;
         return fail(KC_ERR_DEVICE, "oriented-CSR upload failed");
     }
