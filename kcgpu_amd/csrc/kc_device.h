@@ -37,14 +37,15 @@ struct DeviceCtx {
 // Select and check the device (gfx950).  Returns KC_OK or KC_ERR_DEVICE.
 int device_ctx(DeviceCtx **out);
 
-// Grow-only device buffer (blocks come from and go back to a bounded pool, see
-// kc_prep.hip), or a view into memory owned elsewhere (owned =
+// Grow-only device buffer (blocks come from and go back to a bounded pool,
+// except where Unpooled says otherwise), or a view into memory owned elsewhere (owned =
 // false; ensure() on a view checks its size and never allocates).
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
     bool owned = true;
-    int dev = 0;  // device of an owned block
+    int dev = 0;         // device of an owned block
+    bool pooled = true;  // it goes to the pool on release
     int ensure(size_t want);
     void release();
     void view(void *q, size_t b)
@@ -61,6 +62,12 @@ struct DevBuf {
     struct InUse {
         InUse();
         ~InUse();
+    };
+    // While one lives, the blocks that this thread allocates bypass the pool: they
+    // are allocated and freed by the runtime, whose free waits for the device.
+    struct Unpooled {
+        Unpooled();
+        ~Unpooled();
     };
 };
 

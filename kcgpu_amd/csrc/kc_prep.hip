@@ -91,10 +91,13 @@ int device_ctx(DeviceCtx **out)
 // Device blocks that released buffers leave for the next ones, at most
 // POOL_BYTES of them over all devices: an orientation takes and gives a dozen
 // buffers, and the runtime's own allocation and free (which waits for the
-// device) took 2 to 3 ms of a 10 ms call.  Every call of the library has
-// waited for its work on a buffer before it releases it, or (on an error)
-// releases it with that work still in the library's stream, on which the next
-// owner's first use is queued too.  Blocks are given back by kc_shutdown, when
+// device) took 2 to 3 ms of a 10 ms call.  A block may be used on any stream of
+// its device next, so none is released with work on it still queued: every call
+// waits for its streams before its buffers go (StreamWait on early returns), and
+// DevBuf::InUse keeps a count's buffers in place while its launches run.  The
+// server's memory bypasses the pool (Unpooled): its graphs are read by launches
+// that outlive a query, and what it frees has to leave the device for its budget
+// to be true.  Blocks are given back by kc_shutdown, when
 // the device has no memory left, and, oldest first, when newer ones need their
 // place (a pool full of sizes that nobody asks for any more cost every call its
 // allocations again: an edge list to a count 5.1 -> 7.1 ms).
@@ -142,10 +145,13 @@ struct BlockPool {
     }
     void clear()
     {
-        std::lock_guard<std::mutex> lk(mu);
-        for (auto &b : blocks) hipFree(b.second.p);
-        blocks.clear();
-        held = 0;
+        std::multimap<std::pair<int, size_t>, Block> all;
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            all.swap(blocks);
+            held = 0;
+        }
+        for (auto &b : all) hipFree(b.second.p);
     }
 };
 BlockPool &pool()
@@ -155,7 +161,9 @@ BlockPool &pool()
 }
 }  // namespace
 
-static thread_local int t_in_use = 0;  // DevBuf::InUse of this thread
+static thread_local int t_in_use = 0, t_unpooled = 0;  // DevBuf::InUse, DevBuf::Unpooled of this thread
+DevBuf::Unpooled::Unpooled() { ++t_unpooled; }
+DevBuf::Unpooled::~Unpooled() { --t_unpooled; }
 DevBuf::InUse::InUse() { ++t_in_use; }
 DevBuf::InUse::~InUse() { --t_in_use; }
 
@@ -172,7 +180,8 @@ int DevBuf::ensure(size_t want)
     // sizes up to the pool's limit go up to the next eighth of a power of two, so
     // that graphs of about one size fit each other's blocks
     size_t b = want ? want : 256;
-    if (b <= POOL_BYTES / 4) {
+    pooled = t_unpooled == 0;
+    if (pooled && b <= POOL_BYTES / 4) {
         size_t step = 256;
         while (step * 16 <= b) step <<= 1;
         b = (b + step - 1) / step * step;
@@ -180,7 +189,7 @@ int DevBuf::ensure(size_t want)
     dev = 0;
     hipGetDevice(&dev);
     size_t got = b;
-    if ((p = pool().take(dev, b, got))) {
+    if (pooled && (p = pool().take(dev, b, got))) {
         bytes = got;
         return KC_OK;
     }
@@ -201,7 +210,7 @@ int DevBuf::ensure(size_t want)
 
 void DevBuf::release()
 {
-    if (p && owned && !pool().give(dev, p, bytes)) hipFree(p);
+    if (p && owned && !(pooled && pool().give(dev, p, bytes))) hipFree(p);
     p = nullptr;
     bytes = 0;
     owned = true;

@@ -177,6 +177,7 @@ void worker_main(kc_server *s)
     hipSetDevice(s->dev);
     hipStream_t st = nullptr;
     if (hipStreamCreate(&st) != hipSuccess) return;
+    kc::DevBuf::Unpooled own;  // (its own stream, and bytes that the budget counts)
     kc::Scratch scr;
     uint64_t held = 0;  // device bytes this worker's scratch holds between batches
     for (;;) {
@@ -411,6 +412,7 @@ int kc_server_create(const kc_server_config *cfg, kc_server **out)
     const uint64_t eng_bytes = 1ull << 20;
     if (s->cfg.budget_bytes > (64ull << 20)) {
         auto e = std::make_unique<OpenEngine>();
+        DevBuf::Unpooled own;
         if ((rc = e->init(s->dev))) {
             delete s;
             return rc;
@@ -440,7 +442,11 @@ int kc_server_add_graph(kc_server *s, const kc_graph *g, int orient_mode, uint32
         s->resident_bytes += foot;  // reserve before the upload
     }
     kc_oriented *o = nullptr;
-    int rc = kc_orient(g, orient_mode, &o);
+    int rc;
+    {
+        DevBuf::Unpooled own;  // (the graph, and the orientation's transient buffers, are in the budget)
+        rc = kc_orient(g, orient_mode, &o);
+    }
     std::lock_guard<std::mutex> lk(s->mu);
     if (rc) {
         s->resident_bytes -= foot;
