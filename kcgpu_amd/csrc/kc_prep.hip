@@ -792,8 +792,11 @@ __global__ void k_peel_ctl_round(PeelCtl *ctl, uint32_t *cnt, uint32_t maxdeg)
 // stores past the L1 and the XCD's L2), so a barrier only waits for this
 // thread's own accesses.  Counters that all blocks read after a barrier sit in
 // three slots taken in turn; a slot is cleared one phase before it is filled.
-// A wait is bounded: when the other blocks do not arrive (the device holds
-// no room for them) every block leaves and the host steps the peel.
+// A wait is bounded: when the other blocks do not arrive every block leaves and
+// the host steps the peel from the start.  At the first barrier they may be
+// missing because the device has no room for them (other launches hold it):
+// that wait is a few milliseconds.  Past it all of them are resident, and the
+// limit is only there to end a launch that something else has stopped.
 // ---------------------------------------------------------------------------
 struct PeelShared {
     unsigned long long arrive;
@@ -810,7 +813,7 @@ struct PeelRunArgs {
     uint32_t *hubs[2];
     uint32_t *list[2];  // n/4, n/16
     PeelShared *s;
-    uint64_t wait_ticks;
+    uint64_t first_ticks, wait_ticks;  // limits of the first and of the later waits (0: give up at once)
 };
 
 constexpr uint32_t PEEL_SHORT = 64, PEEL_HUB = 4096;
@@ -876,6 +879,7 @@ __global__ __launch_bounds__(PEEL_T) void k_peel_run(PeelRunArgs a)
     const uint32_t wave = tid >> 6, nwave = nthr >> 6;
     PeelShared *s = a.s;
     unsigned long long target = 0;
+    uint64_t limit = a.first_ticks;
     auto barrier = [&]() {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_s_waitcnt(0);  // this thread's stores and atomics are done
@@ -884,17 +888,19 @@ __global__ __launch_bounds__(PEEL_T) void k_peel_run(PeelRunArgs a)
         if (threadIdx.x == 0) {
             __hip_atomic_fetch_add(&s->arrive, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const uint64_t t0 = wall_clock64();
-            uint32_t fine = 1;
-            while (__hip_atomic_load(&s->arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-                if (wall_clock64() - t0 > a.wait_ticks || ld_dev(&s->abort)) {
+            uint32_t fine = limit ? 1 : 0;
+            if (!fine) st_dev(&s->abort, 1u);
+            while (fine && __hip_atomic_load(&s->arrive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
+                if (wall_clock64() - t0 > limit || ld_dev(&s->abort)) {
                     st_dev(&s->abort, 1u);
                     fine = 0;
-                    break;
+                } else {
+                    __builtin_amdgcn_s_sleep(1);
                 }
-                __builtin_amdgcn_s_sleep(1);
             }
             ok = fine;
         }
+        limit = a.wait_ticks;
         __syncthreads();
         const bool r = ok != 0;
         __syncthreads();  // (ok is written again by the next barrier)
@@ -1054,7 +1060,15 @@ static int run_peel(DeviceCtx *ctx, hipStream_t s, uint32_t n, uint32_t nnz, uin
         pa.list[0] = pa.hubs[0] + at_list;
         pa.list[1] = pa.list[0] + n / 4 + 1;
         pa.s = reinterpret_cast<PeelShared *>(more.as<uint32_t>() + at_shared);
-        pa.wait_ticks = 2000000000ull;  // 20 s at 100 MHz
+        // ticks of 10 ns: 10 ms (and 1 ns a vertex, for the pass before it), then 5 s;
+        // KC_PEEL_WAIT_US=first,later sets them (a test of the way out has no other)
+        pa.first_ticks = 1000000ull + n / 10;
+        pa.wait_ticks = 500000000ull;
+        if (const char *e = std::getenv("KC_PEEL_WAIT_US")) {
+            char *end = nullptr;
+            pa.first_ticks = pa.wait_ticks = 100 * std::strtoull(e, &end, 10);
+            if (*end == ',') pa.wait_ticks = 100 * std::strtoull(end + 1, nullptr, 10);
+        }
         const int gb = (int)std::max<uint64_t>(1, std::min<uint64_t>(((uint64_t)n + PEEL_T - 1) / PEEL_T, PEEL_BLOCKS));
         hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, reinterpret_cast<uint32_t *>(pa.s),
                            (uint32_t)(sizeof(PeelShared) / 4), 0u);
