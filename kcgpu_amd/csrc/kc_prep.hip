@@ -1030,8 +1030,9 @@ struct Captured {
     }
 };
 
+// words: n + 1 words that the caller has no use for until the peel is done
 static int run_peel(DeviceCtx *ctx, hipStream_t s, uint32_t n, uint32_t nnz, uint32_t maxdeg, const uint32_t *rowptr,
-                    const uint32_t *col, uint32_t *prio, uint32_t *max_core)
+                    const uint32_t *col, uint32_t *prio, uint32_t *words, uint32_t *max_core)
 {
     DevBuf deg, st, q0, q1, cnt, more, ctlb;
     StreamWait wait(s);
@@ -1043,10 +1044,11 @@ static int run_peel(DeviceCtx *ctx, hipStream_t s, uint32_t n, uint32_t nnz, uin
     const char *mode = std::getenv("KC_PEEL_MODE");
     bool coop = mode && std::strcmp(mode, "coop") == 0;
     if (!coop && !(mode && std::strcmp(mode, "step") == 0)) {
-        const size_t nhub = (size_t)nnz / PEEL_HUB + 1, nl = (size_t)n / 4 + n / 16 + 2;
-        // `more`: hub queues, live lists, counters
-        const size_t at_list = 2 * nhub, at_shared = (at_list + nl + 1) & ~(size_t)1;
-        if ((rc = more.ensure(4 * at_shared + sizeof(PeelShared)))) return rc;
+        // the live lists (n/4 and n/16 entries) go into `words`; with degrees and queues
+        // it is 12 bytes a vertex and 1/512 byte an entry for the hub queues (the
+        // stepped peel takes 13 a vertex)
+        const size_t nhub = std::min<size_t>(n, (size_t)nnz / PEEL_HUB) + 1;
+        if ((rc = more.ensure(8 * nhub + sizeof(PeelShared)))) return rc;
         PeelRunArgs pa{};
         pa.n = n;
         pa.rowptr = rowptr;
@@ -1055,11 +1057,11 @@ static int run_peel(DeviceCtx *ctx, hipStream_t s, uint32_t n, uint32_t nnz, uin
         pa.prio = prio;
         pa.q[0] = q0.as<uint32_t>();
         pa.q[1] = q1.as<uint32_t>();
+        pa.list[0] = words;
+        pa.list[1] = words + n / 4 + 1;
         pa.hubs[0] = more.as<uint32_t>();
         pa.hubs[1] = pa.hubs[0] + nhub;
-        pa.list[0] = pa.hubs[0] + at_list;
-        pa.list[1] = pa.list[0] + n / 4 + 1;
-        pa.s = reinterpret_cast<PeelShared *>(more.as<uint32_t>() + at_shared);
+        pa.s = reinterpret_cast<PeelShared *>(pa.hubs[1] + nhub);
         // ticks of 10 ns: 10 ms (and 1 ns a vertex, for the pass before it), then 5 s;
         // KC_PEEL_WAIT_US=first,later sets them (a test of the way out has no other)
         pa.first_ticks = 1000000ull + n / 10;
@@ -1292,7 +1294,7 @@ int kc::orient_device_csr(DeviceCtx *ctx, uint32_t n, uint32_t nnz, uint32_t max
     uint32_t max_core = 0;
     if (mode == KC_ORIENT_DEGEN && n > 0 &&
         (rc = run_peel(ctx, s, n, nnz, maxdeg, frow.as<uint32_t>(), fcol.as<uint32_t>(), o->key.as<uint32_t>(),
-                       &max_core)))
+                       outdeg.as<uint32_t>(), &max_core)))
         return rc;
     // keep flags, per-row counts, scan, stable compaction, max out-degree
     // (plain launches: instantiating, launching and destroying a graph of these

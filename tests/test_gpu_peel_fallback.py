@@ -28,3 +28,24 @@ def test_peel_gives_up_and_is_stepped(n, m, hub, wait, monkeypatch):
     monkeypatch.delenv("KC_PEEL_WAIT_US")
     o = G.orient("degen")  # the waits hold again, on the same device blocks
     assert (o.export()[2] == prio).all() and o.info()["max_core"] == core
+
+
+# where the peel's lists and hub queues lie: the smallest graphs, and hubs at both sides of the room for their queues
+@pytest.mark.parametrize("n,hubs", [(1, 0), (2, 1), (3, 1), (4, 2), (5, 3), (9000, 1), (4200, 4200), (6500, 900)])
+def test_peel_of_smallest_and_hub_graphs(n, hubs):
+    """`hubs` vertices joined to every other vertex: with 4,200 of 4,200 the rows of all are above 4,096 entries"""
+    if hubs == n:
+        a, b = np.triu_indices(n, 1)
+    else:
+        a = np.repeat(np.arange(hubs), n)
+        b = np.tile(np.arange(n), hubs)
+        keep = a < b
+        a, b = a[keep], b[keep]
+    G = K.Graph.from_edges(a.astype(np.uint32), b.astype(np.uint32), n)
+    o = G.orient("degen")
+    rp, col, key = o.export()
+    if hubs < n or n == 1:
+        prio, core = O.peel_priority(G.csr()[0].astype(np.uint64), G.csr()[1])
+        assert (key == prio).all() and o.info()["max_core"] == core
+    else:  # a clique goes in one round at level n - 1, which empties the graph and assigns nothing
+        assert int(rp[-1]) == a.size and o.info()["max_core"] == n - 1 and (key == 2 * a.size).all()
