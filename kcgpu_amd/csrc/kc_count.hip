@@ -3566,6 +3566,13 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     // accumulators, per-query sums and overflow flags lie side by side: one copy back
     std::vector<uint64_t> back((acc_bytes + q_bytes + 7) / 8);
     uint32_t h[NS + 16] = {0};
+    struct WordsUse {
+        AdjWords *w = nullptr;
+        ~WordsUse()
+        {
+            if (w) w->put();
+        }
+    } wu;
     StreamWait wait(s);  // no return leaves a kernel running on the caller's scratch
     KC_HIP(hipMemcpyAsync(dq, up.data(), up.size(), hipMemcpyHostToDevice, s));
     {  // counters, queue heads and per-query sums start at zero (a fill kernel, no memset node)
@@ -3598,12 +3605,14 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     // (lists of at most MERGE_OUT are sooner merged by a lane an edge, and binned:
     // 23,936 edges with lists of at most 8, 47 us a call against 59)
     constexpr uint32_t MERGE_OUT = 32;
-    constexpr uint64_t BITS_BYTES = 2ull << 30;
+    // (KC_WORDS_MIB sets the bytes of adjacency words a handle may keep, 0: none)
+    uint64_t bits_limit = 2ull << 30;
+    if (const char *e = std::getenv("KC_WORDS_MIB")) bits_limit = std::strtoull(e, nullptr, 10) << 20;
     const bool lists = nq == 1 && any_edge && max_out > MERGE_OUT;
     const bool triangles = lists && kmax == 3 && !local && total > 0;
     // The adjacency words (rows_from_bits) of one query on a graph with
     // long lists: they belong to the handle's scratch like the sizes, and are
-    // made by the pass that makes those, of a whole count and within BITS_BYTES.
+    // made by the pass that makes those, of a whole count and within bits_limit.
     // With lists of at most MERGE_OUT the pass costs the first call more than a
     // later one gains (BA n=200,000: 0.63 -> 0.84 and 0.52 -> 0.41 ms); with longer
     // ones both gain (Chung-Lu n=300,000, 2 M edges: pass 0.36 ms, the launches of a
@@ -3612,18 +3621,24 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     // server's workers keep to the memory they declared.
     const uint64_t nedge = qs[0].o->m;
     const uint64_t bits_bytes = nedge * sizeof(uint64_t) * std::min<uint64_t>(BITS_ROW / 64, ((uint64_t)max_out + 63) / 64);
-    const bool with_bits = nq == 1 && max_out > MERGE_OUT && !triangles && !(any_edge && kmax == 3) && nedge > 0 &&
-                           !scr.fixed && grid_share <= 1 && scr.may_grow && hq[0].sample <= 1 &&
-                           bits_bytes <= BITS_BYTES && scr.bits.ensure(bits_bytes) == KC_OK;
-    const bool bits_cached = with_bits && scr.bits_uid == qs[0].o->uid;
-    if (with_bits && !bits_cached) scr.bits_uid = 0;
+    // Where the device has no room for them the lists are used, and a later
+    // allocation of this call or of another may take them back.
+    if (nq == 1 && max_out > MERGE_OUT && !triangles && !(any_edge && kmax == 3) && nedge > 0 && !scr.fixed &&
+        grid_share <= 1 && scr.words && hq[0].sample <= 1 && bits_bytes <= bits_limit && scr.words->take()) {
+        wu.w = scr.words;
+        if (wu.w->bits.bytes < bits_bytes) wu.w->uid = 0;
+    }
+    const bool with_bits = wu.w && wu.w->bits.try_ensure(bits_bytes);
+    const bool bits_cached = with_bits && wu.w->uid == qs[0].o->uid;
+    if (wu.w && !bits_cached) wu.w->uid = 0;
+    uint64_t *const bits = with_bits ? wu.w->bits.as<uint64_t>() : nullptr;
     BinArgs ba{dq, dalgo, doff, nq, pivot_top2, total, any_edge ? scr.size.as<uint32_t>() : nullptr, sub_cnt, bin_max,
                sub_pos, sub_off, scr.tasks.as<uint64_t>(), any_pivot ? scr.binom.as<uint64_t>() : nullptr, brows, bstride};
     if (total > 0) {
         if ((lists && (triangles || !sizes_cached)) || (with_bits && !bits_cached)) {
             EdgeArgs ea{hq[0].rowptr, hq[0].col, hq[0].src, (uint32_t)nedge, hq[0].sample, hq[0].offset,
                         halgo[0] ? pivot_top2 : CLASS_ROWS[2], triangles ? 1u : 0u, any_edge ? scr.size.as<uint32_t>() : nullptr,
-                        dacc + (halgo[0] ? NCLASS * NSTRIPE * ACC : 0), with_bits && !bits_cached ? scr.bits.as<uint64_t>() : nullptr};
+                        dacc + (halgo[0] ? NCLASS * NSTRIPE * ACC : 0), bits_cached ? nullptr : bits};
             const unsigned eb = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((nedge + 255) / 256, (uint64_t)ctx->cu * 8));
             if (triangles) evs.record(evs.go, s);
             if (ea.bits) hipLaunchKernelGGL(k_edge_sizes<true>, dim3(eb), dim3(256), 0, s, ea);
@@ -3655,7 +3670,7 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         scr.size_uid = qs[0].o->uid;
         scr.size_total = total;
     }
-    if (with_bits) scr.bits_uid = qs[0].o->uid;
+    if (with_bits) wu.w->uid = qs[0].o->uid;
     uint32_t bcnt[NB] = {0}, bmax[NB] = {0}, boff[NB] = {0};
     if (triangles) {
     } else if (one_bin) {
@@ -3751,7 +3766,7 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         a.qhead = qhead + (size_t)b * NQUEUE * QSTRIDE;
         a.acc = dacc + (size_t)b * NSTRIPE * ACC;
         a.acc_mask = NSTRIPE - 1;
-        a.bits = with_bits ? scr.bits.as<uint64_t>() : nullptr;
+        a.bits = bits;
         a.bits_m = nedge;
         a.qcount = qcount;
         a.single = nq == 1;
@@ -3847,6 +3862,13 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
             slice_bytes = std::max<size_t>(slice_bytes, blocks * L.total * 8);
         }
         plan.push_back(Launch{a, kern, b, (uint32_t)blocks, nw, lds, global});
+    }
+    if (slice_bytes && !scr.gscr.try_ensure(slice_bytes, true) && with_bits) {
+        // the words of this very call stand in the way: the lists do
+        KC_HIP(hipStreamSynchronize(s));
+        wu.w->uid = 0;
+        wu.w->bits.release();
+        for (Launch &l : plan) l.a.bits = nullptr;
     }
     if (slice_bytes && (rc = scr.gscr.ensure(slice_bytes))) return rc;
     DevBuf::InUse in_use;  // from here to the wait below no buffer of this thread may move
@@ -4293,7 +4315,7 @@ static int count_tasks(const kc_oriented *o, const kc_query *q, uint32_t stride,
     std::vector<QueryRun> qs{run};
     std::vector<kc_result> res;
     LaunchStats ls;
-    om->scr.may_grow = true;
+    om->scr.words = &om->words;
     rc = run_queries(om->scr, om->stream, qs, res, &ls);
     if (rc) return rc;
     fill_result(r, res[0], ls);
@@ -4340,7 +4362,7 @@ extern "C" int kc_count_local(const kc_oriented *o, const kc_query *q, uint64_t 
     std::vector<QueryRun> qs{QueryRun{o, qq}};
     std::vector<kc_result> res;
     LaunchStats ls;
-    om->scr.may_grow = true;
+    om->scr.words = &om->words;
     rc = run_queries(om->scr, om->stream, qs, res, &ls, om->scr.local.as<uint64_t>());
     if (rc) return rc;
     if (n) {

@@ -47,6 +47,9 @@ struct DevBuf {
     int dev = 0;         // device of an owned block
     bool pooled = true;  // it goes to the pool on release
     int ensure(size_t want);
+    // the same for a block that a call can do without, with no error left behind;
+    // insist: as ensure(), with pooled blocks and idle adjacency words given up for it
+    bool try_ensure(size_t want, bool insist = false);
     void release();
     void view(void *q, size_t b)
     {
@@ -93,19 +96,34 @@ struct StreamWait {
 // must fit 32 bits.  in and out may alias.  tmp is scratch owned by caller.
 int scan_exclusive_u32(const uint32_t *in, uint32_t *out, uint32_t n, DevBuf &tmp, hipStream_t s);
 
+// The adjacency words of a handle's graph, which counts are faster with and right
+// without: any allocation of the process that finds the device full takes them
+// from the handles that are not counting.
+struct AdjWords {
+    DevBuf bits;
+    uint64_t uid = 0;  // the oriented graph they are of (0: none)
+    // a count that uses them, or who takes them: take() before any use of the members
+    bool take() { return !busy.exchange(true, std::memory_order_acquire); }
+    void put() { busy.store(false, std::memory_order_release); }
+    AdjWords();
+    ~AdjWords();
+
+private:
+    std::atomic<bool> busy{false};
+};
+
 // scratch of one launch sequence (grow-only), or views into a fixed region
 // (fixed = true: ensure() never allocates, run_queries creates no events)
 struct Scratch {
-    DevBuf tasks, meta, binom, gscr, size, qdesc, local, bits;
+    DevBuf tasks, meta, binom, gscr, size, qdesc, local;
     bool fixed = false;
-    bool may_grow = false;  // a handle's own: pivoting may keep the adjacency words of the tasks in `bits`
+    AdjWords *words = nullptr;  // a handle's own counts may keep the adjacency words of its tasks
     // what `size` holds when it was filled for one query of edge tasks: the
     // oriented graph (its uid) and the task count; an edge task's size
     // |N+(u) & N+(v)| does not depend on k, so the next query on that graph
     // reuses it
     uint64_t size_uid = 0;
     uint64_t size_total = 0;
-    uint64_t bits_uid = 0;  // likewise the oriented graph of `bits`
 };
 
 // a number no other oriented graph of the process carries
@@ -247,6 +265,7 @@ struct kc_oriented {
     std::shared_ptr<kc::DevBuf> arena;  // owner of rowptr/col/src/key when they are views (batched orientation)
     // count scratch (grow-only, reused across calls on this handle)
     kc::Scratch scr, batch_scr;
+    kc::AdjWords words;
     std::vector<uint32_t> h_rowptr_cache;  // filled lazily by host-side autotune
     ~kc_oriented();
 };

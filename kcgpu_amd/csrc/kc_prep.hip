@@ -102,6 +102,26 @@ int device_ctx(DeviceCtx **out)
 // place (a pool full of sizes that nobody asks for any more cost every call its
 // allocations again: an edge list to a count 5.1 -> 7.1 ms).
 namespace {
+// device memory the library holds, pooled blocks included; KC_DEVICE_LIMIT_MIB
+// bounds it (an allocation beyond it fails as on a full device)
+std::atomic<size_t> g_held{0};
+
+hipError_t raw_alloc(void **p, size_t bytes)
+{
+    if (const char *e = std::getenv("KC_DEVICE_LIMIT_MIB"))
+        if (g_held.load() + bytes > (std::strtoull(e, nullptr, 10) << 20)) return hipErrorOutOfMemory;
+    const hipError_t rc = hipMalloc(p, bytes);
+    if (rc == hipSuccess) g_held += bytes;
+    else (void)hipGetLastError();
+    return rc;
+}
+
+void raw_free(void *p, size_t bytes)
+{
+    hipFree(p);
+    g_held -= bytes;
+}
+
 constexpr size_t POOL_BYTES = (size_t)512 << 20;
 struct BlockPool {
     std::mutex mu;
@@ -127,20 +147,20 @@ struct BlockPool {
     bool give(int dev, void *p, size_t bytes)
     {
         if (bytes > POOL_BYTES / 4) return false;
-        std::vector<void *> old;
+        std::vector<std::pair<void *, size_t>> old;
         {
             std::lock_guard<std::mutex> lk(mu);
             while (held + bytes > POOL_BYTES) {
                 auto it = std::min_element(blocks.begin(), blocks.end(),
                                            [](const auto &a, const auto &b) { return a.second.seq < b.second.seq; });
-                old.push_back(it->second.p);
+                old.emplace_back(it->second.p, it->first.second);
                 held -= it->first.second;
                 blocks.erase(it);
             }
             blocks.emplace(std::make_pair(dev, bytes), Block{p, seq++});
             held += bytes;
         }
-        for (void *o : old) hipFree(o);  // (waits for the device: not under the lock)
+        for (auto &o : old) raw_free(o.first, o.second);  // (waits for the device: not under the lock)
         return true;
     }
     void clear()
@@ -151,7 +171,7 @@ struct BlockPool {
             all.swap(blocks);
             held = 0;
         }
-        for (auto &b : all) hipFree(b.second.p);
+        for (auto &b : all) raw_free(b.second.p, b.first.second);
     }
 };
 BlockPool &pool()
@@ -159,13 +179,94 @@ BlockPool &pool()
     static BlockPool *p = new BlockPool;  // (never destroyed: buffers may be released late)
     return *p;
 }
+
+struct WordsList {
+    std::mutex mu;
+    std::vector<AdjWords *> all;
+};
+WordsList &words_list()
+{
+    static WordsList *p = new WordsList;  // (likewise)
+    return *p;
+}
+
+// free the adjacency words of every handle that is not counting; false when there were none
+bool drop_words()
+{
+    std::vector<std::pair<void *, size_t>> gone;
+    {
+        WordsList &l = words_list();
+        std::lock_guard<std::mutex> lk(l.mu);
+        for (AdjWords *w : l.all) {
+            if (!w->take()) continue;
+            if (w->bits.p) gone.emplace_back(w->bits.p, w->bits.bytes);
+            w->bits.p = nullptr;
+            w->bits.bytes = 0;
+            w->uid = 0;
+            w->put();
+        }
+    }
+    for (auto &g : gone) raw_free(g.first, g.second);
+    return !gone.empty();
+}
 }  // namespace
+
+AdjWords::AdjWords()
+{
+    WordsList &l = words_list();
+    std::lock_guard<std::mutex> lk(l.mu);
+    l.all.push_back(this);
+}
+
+AdjWords::~AdjWords()
+{
+    WordsList &l = words_list();
+    std::lock_guard<std::mutex> lk(l.mu);
+    l.all.erase(std::find(l.all.begin(), l.all.end(), this));
+}
 
 static thread_local int t_in_use = 0, t_unpooled = 0;  // DevBuf::InUse, DevBuf::Unpooled of this thread
 DevBuf::Unpooled::Unpooled() { ++t_unpooled; }
 DevBuf::Unpooled::~Unpooled() { --t_unpooled; }
 DevBuf::InUse::InUse() { ++t_in_use; }
 DevBuf::InUse::~InUse() { --t_in_use; }
+
+// an owned block of at least want bytes in p, or p = null
+static hipError_t acquire(DevBuf &d, size_t want)
+{
+    d.owned = true;
+    // sizes up to the pool's limit go up to the next eighth of a power of two, so
+    // that graphs of about one size fit each other's blocks
+    size_t b = want ? want : 256;
+    d.pooled = t_unpooled == 0;
+    if (d.pooled && b <= POOL_BYTES / 4) {
+        size_t step = 256;
+        while (step * 16 <= b) step <<= 1;
+        b = (b + step - 1) / step * step;
+    }
+    d.dev = 0;
+    hipGetDevice(&d.dev);
+    d.bytes = b;
+    if (d.pooled && (d.p = pool().take(d.dev, b, d.bytes))) return hipSuccess;
+    const hipError_t e = raw_alloc(&d.p, b);
+    if (e != hipSuccess) {
+        d.p = nullptr;
+        d.bytes = 0;
+    }
+    return e;
+}
+
+bool DevBuf::try_ensure(size_t want, bool insist)
+{
+    if (p && want <= bytes) return true;
+    if (p && (!owned || t_in_use)) return false;
+    release();
+    if (acquire(*this, want) == hipSuccess) return true;
+    if (!insist) return false;
+    pool().clear();
+    if (acquire(*this, want) == hipSuccess) return true;
+    return drop_words() && acquire(*this, want) == hipSuccess;
+}
 
 int DevBuf::ensure(size_t want)
 {
@@ -175,42 +276,12 @@ int DevBuf::ensure(size_t want)
     }
     if (want <= bytes && p && owned) return KC_OK;
     if (p && t_in_use) return fail(KC_ERR_DEVICE, "a buffer in use by a launch would move (internal error)");
-    release();
-    owned = true;
-    // sizes up to the pool's limit go up to the next eighth of a power of two, so
-    // that graphs of about one size fit each other's blocks
-    size_t b = want ? want : 256;
-    pooled = t_unpooled == 0;
-    if (pooled && b <= POOL_BYTES / 4) {
-        size_t step = 256;
-        while (step * 16 <= b) step <<= 1;
-        b = (b + step - 1) / step * step;
-    }
-    dev = 0;
-    hipGetDevice(&dev);
-    size_t got = b;
-    if (pooled && (p = pool().take(dev, b, got))) {
-        bytes = got;
-        return KC_OK;
-    }
-    hipError_t e = hipMalloc(&p, b);
-    if (e != hipSuccess) {
-        pool().clear();
-        (void)hipGetLastError();
-        e = hipMalloc(&p, b);
-    }
-    if (e != hipSuccess) {
-        p = nullptr;
-        bytes = 0;
-        return fail(KC_ERR_NOMEM, "hipMalloc(%zu) failed: %s", b, hipGetErrorString(e));
-    }
-    bytes = b;
-    return KC_OK;
+    return try_ensure(want, true) ? KC_OK : fail(KC_ERR_NOMEM, "no room for %zu bytes on the device", want);
 }
 
 void DevBuf::release()
 {
-    if (p && owned && !(pooled && pool().give(dev, p, bytes))) hipFree(p);
+    if (p && owned && !(pooled && pool().give(dev, p, bytes))) raw_free(p, bytes);
     p = nullptr;
     bytes = 0;
     owned = true;

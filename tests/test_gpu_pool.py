@@ -1,7 +1,9 @@
 """GPU: which device memory the library keeps and which it gives back."""
 import ctypes
 import time
+from math import comb
 
+import numpy as np
 import pytest
 
 import kcgpu_amd as K
@@ -55,3 +57,52 @@ def test_graphs_of_the_calls_beside_a_server_are_pooled():
             assert all(srv.wait(x).count == exp for x in t)
     finally:
         srv.close()
+
+
+def _pairs_graph(parts):
+    """all edges between `parts` pairs of vertices but none inside a pair"""
+    a, b = np.triu_indices(2 * parts, 1)
+    keep = a // 2 != b // 2
+    return K.Graph.from_edges(a[keep].astype(np.uint32), b[keep].astype(np.uint32), 2 * parts)
+
+
+def test_adjacency_words_never_make_a_call_fail(monkeypatch):
+    """on a full device (KC_DEVICE_LIMIT_MIB) a count that fits without adjacency words fits with them allowed, its own
+    or another handle's, and every count that succeeds is right"""
+    parts, k = 530, 4
+    G = _pairs_graph(parts)  # 18 MB of words, 200 MB of slices for its tasks above 512 vertices
+    other = K.Graph.generate(K.GEN_CHUNG_LU, seed=8, n=300_000, m=1_900_000, gamma=2.1, max_degree=6000)
+
+    def fits(limit, words):
+        monkeypatch.setenv("KC_WORDS_MIB", words)
+        monkeypatch.setenv("KC_DEVICE_LIMIT_MIB", str(limit))
+        o = None
+        try:
+            o = G.orient("degree")
+            for _ in range(2):
+                assert o.count(k, "pivot", "node").count == comb(parts, k) << k
+            return True
+        except K.KCError as e:
+            assert e.code == K.KC_ERR_NOMEM
+            return False
+        finally:
+            if o:
+                o.close()
+
+    least = next(x for x in range(0, 4096, 32) if fits(x, "0"))
+    for limit in range(max(0, least - 32), least + 40, 2):  # on both sides of what it needs
+        without = fits(limit, "0")
+        assert fits(limit, "2048") or not without, limit
+
+    monkeypatch.delenv("KC_DEVICE_LIMIT_MIB")
+    monkeypatch.setenv("KC_WORDS_MIB", "0")
+    o = other.orient("degen")
+    exp = o.count(6, "pivot", "edge").count
+    least = next(x for x in range(0, 4096, 4) if fits(x, "0"))
+    for _ in range(2):  # now it holds 60 MB of words, until the other graph's count wants them
+        monkeypatch.delenv("KC_DEVICE_LIMIT_MIB")
+        monkeypatch.setenv("KC_WORDS_MIB", "2048")
+        assert o.count(6, "pivot", "edge").count == exp
+        assert fits(least, "0")
+    monkeypatch.setenv("KC_DEVICE_LIMIT_MIB", str(least))
+    assert o.count(6, "pivot", "edge").count == exp and o.count(6, "pivot", "node").count == exp
