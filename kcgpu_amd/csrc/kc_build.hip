@@ -6,7 +6,8 @@
 //
 // Steps: degree histogram (both endpoints of every non-loop edge), exclusive
 // scan into row offsets, scatter of both directions to the places the
-// histogram's atomics gave (unordered within a row), a per-row sort that also removes
+// histogram's atomics gave (unordered within a row; where the device has no room
+// for those places, through per-row atomic cursors), a per-row sort that also removes
 // duplicates, a scan of the unique counts and a compaction into the final
 // CSR.  Rows of at most SMALL_ROW entries are sorted by one wave each with a
 // bitonic network in LDS; longer rows (hubs of power-law graphs, up to
@@ -60,7 +61,8 @@ __global__ __launch_bounds__(BUILD_T) void k_edge_max(const uint32_t *s, const u
 
 // The degree histogram's atomics hand every edge end its place in its row,
 // which the scatter then needs no atomic for (2.3 M edges of an R-MAT graph:
-// two passes of atomics, 1.01 ms each -> 1.01 + 0.05).
+// two passes of atomics, 1.01 ms each -> 1.01 + 0.05).  rank = null: not kept, the
+// scatter takes the places from cursors (off, then) with atomics of its own.
 __global__ __launch_bounds__(BUILD_T) void k_edge_degree(const uint32_t *s, const uint32_t *d, uint64_t ne,
                                                          uint32_t *deg, uint2 *rank)
 {
@@ -68,19 +70,24 @@ __global__ __launch_bounds__(BUILD_T) void k_edge_degree(const uint32_t *s, cons
         const uint32_t u = s[i], v = d[i];
         if (u == v) continue;
         const uint32_t ru = atomicAdd(&deg[u], 1u), rv = atomicAdd(&deg[v], 1u);
-        rank[i] = make_uint2(ru, rv);
+        if (rank) rank[i] = make_uint2(ru, rv);
     }
 }
 
 __global__ __launch_bounds__(BUILD_T) void k_edge_scatter(const uint32_t *s, const uint32_t *d, uint64_t ne,
-                                                          const uint32_t *off, const uint2 *rank, uint32_t *tmp)
+                                                          uint32_t *off, const uint2 *rank, uint32_t *tmp)
 {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < ne; i += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t u = s[i], v = d[i];
         if (u == v) continue;
-        const uint2 r = rank[i];
-        tmp[off[u] + r.x] = v;
-        tmp[off[v] + r.y] = u;
+        if (rank) {
+            const uint2 r = rank[i];
+            tmp[off[u] + r.x] = v;
+            tmp[off[v] + r.y] = u;
+        } else {
+            tmp[atomicAdd(&off[u], 1u)] = v;
+            tmp[atomicAdd(&off[v], 1u)] = u;
+        }
     }
 }
 
@@ -267,18 +274,25 @@ int build_csr_device(DeviceCtx *ctx, hipStream_t s, uint32_t n_in, size_t ne, co
     if (nn >= 0xFFFFFFFFull) return fail(KC_ERR_LIMIT, "n=%llu does not fit 32-bit ids", (unsigned long long)nn);
     const uint32_t n = (uint32_t)nn;
     if ((rc = deg.ensure(4 * ((size_t)n + 1))) || (rc = off.ensure(4 * ((size_t)n + 1))) ||
-        (rc = rank.ensure(8 * ne + 8)) || (rc = tmp.ensure(8 * ne + 4)) ||
+        (rc = tmp.ensure(8 * ne + 4)) ||
         (rc = ucnt.ensure(4 * ((size_t)n + 1))) || (rc = big.ensure(4 * ((size_t)n + 1))) ||
         (rc = rowptr.ensure(4 * ((size_t)n + 1))))
         return rc;
+    // (8 bytes an edge that an edge list too large for them does without)
+    const bool ranked = rank.try_ensure(8 * ne + 8);
     const int gn = (int)std::max<uint64_t>(1, std::min<uint64_t>(((uint64_t)n + BUILD_T - 1) / BUILD_T, (uint64_t)ctx->cu * 16));
     hipLaunchKernelGGL(k_build_fill, dim3(gn), dim3(BUILD_T), 0, s, deg.as<uint32_t>(), (uint64_t)n + 1, 0u);
     if (ne) hipLaunchKernelGGL(k_edge_degree, dim3(ge), dim3(BUILD_T), 0, s, S, D, (uint64_t)ne, deg.as<uint32_t>(),
-                               rank.as<uint2>());
+                               ranked ? rank.as<uint2>() : nullptr);
     KC_HIP(hipGetLastError());
     if ((rc = scan_exclusive_u32(deg.as<uint32_t>(), off.as<uint32_t>(), n, scan_tmp, s))) return rc;
-    if (ne) hipLaunchKernelGGL(k_edge_scatter, dim3(ge), dim3(BUILD_T), 0, s, S, D, (uint64_t)ne, off.as<uint32_t>(),
-                               rank.as<uint2>(), tmp.as<uint32_t>());
+    uint32_t *at = off.as<uint32_t>();
+    if (!ranked) {  // the cursors: a copy of the offsets in `big`, which is not in use yet
+        at = big.as<uint32_t>();
+        KC_HIP(hipMemcpyAsync(at, off.p, 4 * (size_t)n, hipMemcpyDeviceToDevice, s));
+    }
+    if (ne) hipLaunchKernelGGL(k_edge_scatter, dim3(ge), dim3(BUILD_T), 0, s, S, D, (uint64_t)ne, at,
+                               ranked ? rank.as<uint2>() : nullptr, tmp.as<uint32_t>());
     // rows: distinct sorted values at each row's start, counts in ucnt
     const int gw = (int)std::max<uint64_t>(1, std::min<uint64_t>(((uint64_t)n + 3) / 4, (uint64_t)ctx->cu * 8));
     if (n) hipLaunchKernelGGL(k_row_sort_small, dim3(gw), dim3(BUILD_T), 0, s, off.as<uint32_t>(), n,

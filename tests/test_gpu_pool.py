@@ -106,3 +106,25 @@ def test_adjacency_words_never_make_a_call_fail(monkeypatch):
         assert fits(least, "0")
     monkeypatch.setenv("KC_DEVICE_LIMIT_MIB", str(least))
     assert o.count(6, "pivot", "edge").count == exp and o.count(6, "pivot", "node").count == exp
+
+
+def test_edge_list_that_leaves_no_room_for_the_ranks(monkeypatch):
+    """the CSR build with and without the places of the edge ends: from the least memory it takes upwards"""
+    r = np.random.default_rng(3)
+    ne, n = 1_000_003, 60_000
+    s, d = (np.minimum(r.zipf(1.4, ne), n) - 1).astype(np.uint32), r.integers(0, n, ne, dtype=np.uint32)
+    exp = K.Graph.from_edges(s, d, n).csr()
+
+    def fits(limit):
+        monkeypatch.setenv("KC_DEVICE_LIMIT_MIB", str(limit))
+        try:
+            rp, col = K.Graph.from_edges_device(s, d, n).csr()
+        except K.KCError as e:
+            assert e.code == K.KC_ERR_NOMEM
+            return False
+        assert (rp == exp[0]).all() and (col == exp[1]).all()
+        return True
+
+    least = next(x for x in range(0, 4096, 1) if fits(x))
+    for limit in range(least, least + 14):  # (8 MB of ranks)
+        assert fits(limit), limit
