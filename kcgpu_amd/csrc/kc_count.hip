@@ -778,7 +778,7 @@ __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32
     k = uni32(k);
     U X = BITS == 64 ? (U)uni64(X0) : (U)uni32((uint32_t)X0);
     U tC = 0, tB = 0, stkC = 0, stkB = 0;
-    uint32_t tM = 0, stkM = 0;  // h | p << 8 | pivot << 20
+    uint32_t tM = 0, stkM = 0;  // h | p << 8 | pivot << 24 (p < 2^16, pivot < 256)
     bool open = false;
     int t = -1;
     uint32_t h = uni32(h0), p = uni32(p0);
@@ -840,7 +840,7 @@ __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32
                             open = true;
                             tC = X;
                             tB = X & ~rdlane(row, pv) & ~((U)1 << pv);
-                            tM = h | (p << 8) | (pv << 20);
+                            tM = h | (p << 8) | (pv << 24);
                         }
                     }
                 }
@@ -867,7 +867,7 @@ __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32
             open = true;
         }
         h = tM & 0xFF;
-        p = (tM >> 8) & 0xFFF;
+        p = (tM >> 8) & 0xFFFF;
         if (tB) {
             const uint32_t b = low_bit(tB);
             X = tC & rdlane(row, b);
@@ -875,7 +875,7 @@ __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32
             tB &= tB - 1;
             ++h;
         } else {  // the pivot branch replaces its level
-            X = tC & rdlane(row, tM >> 20);
+            X = tC & rdlane(row, tM >> 24);
             ++p;
             open = false;
         }
@@ -939,7 +939,7 @@ __device__ uint64_t sct_local(const CountArgs &a, uint32_t k, const uint64_t (&r
         H.w[o] = P.w[o] = tC.w[o] = tB.w[o] = tH.w[o] = tP.w[o] = 0;
         stkC.w[o] = stkB.w[o] = stkH.w[o] = stkP.w[o] = 0;
     }
-    uint32_t tM = 0, stkM = 0;  // h | p << 8 | pivot << 20
+    uint32_t tM = 0, stkM = 0;  // h | p << 8 | pivot << 24 (p < 2^16, pivot < 256)
     bool open = false;
     int t = -1;
     uint32_t h = uni32(h0), p = 0;
@@ -1059,7 +1059,7 @@ __device__ uint64_t sct_local(const CountArgs &a, uint32_t k, const uint64_t (&r
                         tH.w[o] = H.w[o];
                         tP.w[o] = P.w[o];
                     }
-                    tM = h | (p << 8) | (pv << 20);
+                    tM = h | (p << 8) | (pv << 24);
                 }
             }
         }
@@ -1078,13 +1078,13 @@ __device__ uint64_t sct_local(const CountArgs &a, uint32_t k, const uint64_t (&r
             open = true;
         }
         h = tM & 0xFF;
-        p = (tM >> 8) & 0xFFF;
+        p = (tM >> 8) & 0xFFFF;
         H = tH;
         P = tP;
         uint64_t left = tB.w[0];
         if (S > 1) left |= tB.w[S - 1];
         const bool held = left != 0;
-        uint32_t v = tM >> 20;
+        uint32_t v = tM >> 24;
         if (held) v = tB.w[0] ? (uint32_t)__builtin_ctzll(tB.w[0]) : 64u + (uint32_t)__builtin_ctzll(tB.w[S - 1]);
 #pragma unroll
         for (int o = 0; o < S; ++o) {
@@ -1852,7 +1852,7 @@ __device__ __attribute__((always_inline)) uint64_t pivot_reg(const CountArgs &a,
                         stkC[w] = (lane == (uint32_t)t) ? X[w] : stkC[w];
                         stkB[w] = (lane == (uint32_t)t) ? bw : stkB[w];
                     }
-                    const uint32_t M = h | (p << 8) | (pv << 20);
+                    const uint32_t M = h | (p << 8) | (pv << 24);
                     stkM = (lane == (uint32_t)t) ? M : stkM;
                 }
             }
@@ -1866,7 +1866,7 @@ __device__ __attribute__((always_inline)) uint64_t pivot_reg(const CountArgs &a,
             B[w] = rdlane64(stkB[w], (uint32_t)t);
         }
         const uint32_t M = (uint32_t)__builtin_amdgcn_readlane((int)stkM, t);
-        const uint32_t hh = M & 0xFF, pp = (M >> 8) & 0xFFF, pv = M >> 20;
+        const uint32_t hh = M & 0xFF, pp = (M >> 8) & 0xFFFF, pv = M >> 24;
         uint32_t b = INF32;
 #pragma unroll
         for (int w = S - 1; w >= 0; --w) {
