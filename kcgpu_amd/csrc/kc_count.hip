@@ -788,7 +788,7 @@ __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32
         uint32_t cx = bits_of(X);
         const uint32_t need = k - h;  // (h <= k)
         if (p + cx >= need) {
-            if (BITS == 64 && KIND != OPEN_SCT && cx <= 32 && need >= 3 && cx > 0 && (!MM || need >= 5 || (uint32_t)((uint64_t)X >> 32) == 0)) {
+            if (BITS == 64 && KIND != OPEN_SCT && cx <= 32 && need >= 3 && cx > 0) {
                 if constexpr (BITS == 64 && KIND != OPEN_SCT) {
                     uint32_t row1 = 0, X1 = (uint32_t)X;
                     if ((X >> 32) == 0) {
@@ -3527,20 +3527,15 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
     // per query: two sums, then a flag (the sums of a single query are in the accumulators)
     const size_t q_bytes = sizeof(uint64_t) * 2 * nq + sizeof(uint32_t) * nq;
     bool any_pivot = false, any_edge = false, one_algo = true;
-    // Five or more vertices below the root of some pivoting task: its tree is walked,
-    // and most of the time goes to closing its nodes, for which the two- and
-    // four-word kernels have the matrix cores.  With fewer, most roots close by
-    // themselves; the operands' registers then only cost waves and spills.  Edge
-    // tasks, ms, without / with matrix cores: Chung-Lu n=1.7M k=5 17.5 / 19.9, k=6
-    // 26.6 / 30.7, k=7 79 / 73, k=8 434 / 357; R-MAT scale 22 k=5, 65..128 vertices 341
-    // / 476, 129..256 982 / 1196; k=8, 1 of 1024, both 165 / 138.
-    bool deep = false;
+    // The most vertices below the root of a pivoting task (it decides whether the two-
+    // and four-word kernels have the matrix cores, below)
+    uint32_t depth = 0;
     uint32_t max_out = 0;  // bounds every task's size
     for (uint32_t i = 0; i < nq; ++i) {
         any_pivot |= halgo[i] != 0;
         any_edge |= hq[i].gran == KC_GRAN_EDGE;
         one_algo &= halgo[i] == halgo[0];
-        deep |= halgo[i] && hq[i].k >= (hq[i].gran == KC_GRAN_EDGE ? 7u : 6u);
+        if (halgo[i]) depth = std::max(depth, hq[i].k - std::min(hq[i].k, hq[i].gran == KC_GRAN_EDGE ? 2u : 1u));
         max_out = std::max(max_out, qs[i].o->max_out);
     }
     const uint32_t bstride = kmax + 1, brows = max_out + 2;
@@ -3791,7 +3786,18 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         const void *kern = generic_kernel(pivot, global, lc, c <= 1);
         variant[b] = global ? 3u : 1u;
         if (pivot && !global && c <= 2 && !lc) {
-            kern = register_kernel(c, deep);
+            // With five or more vertices below the roots the tree is walked, and most of
+            // the time goes to closing its nodes: on the matrix cores.  With fewer, most
+            // roots close by themselves, and the operands' registers only cost waves and
+            // spills.  Edge tasks, ms, without / with matrix cores: Chung-Lu n=1.7M k=5
+            // 17.5 / 19.9, k=6 26.6 / 30.7, k=7 79 / 71, k=8 434 / 345; R-MAT scale 22 k=5,
+            // 65..128 vertices 341 / 476, 129..256 982 / 1196; k=8, 1 of 1024, both 165 / 138.
+            // At just five a launch with a slot for every task is over with its longest,
+            // whose closures then wait for the matrix cores instead of other waves' (node
+            // tasks at k=6: R-MAT scale 14, 5 tasks per CU, 1.39 / 1.74; one random graph of
+            // 300 vertices, density 0.5, 3.63 / 4.82).
+            constexpr uint32_t SLOTS_PER_CU = 16;
+            kern = register_kernel(c, depth > 5 || (depth == 5 && bcnt[b] >= SLOTS_PER_CU * (uint32_t)ctx->cu));
             L = make_layout(a.rmax, a.wmax, 0, 0, true);
             variant[b] = 2u;
         }
