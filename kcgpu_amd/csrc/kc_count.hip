@@ -3786,18 +3786,25 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
         const void *kern = generic_kernel(pivot, global, lc, c <= 1);
         variant[b] = global ? 3u : 1u;
         if (pivot && !global && c <= 2 && !lc) {
-            // With five or more vertices below the roots the tree is walked, and most of
-            // the time goes to closing its nodes: on the matrix cores.  With fewer, most
-            // roots close by themselves, and the operands' registers only cost waves and
-            // spills.  Edge tasks, ms, without / with matrix cores: Chung-Lu n=1.7M k=5
-            // 17.5 / 19.9, k=6 26.6 / 30.7, k=7 79 / 71, k=8 434 / 345; R-MAT scale 22 k=5,
-            // 65..128 vertices 341 / 476, 129..256 982 / 1196; k=8, 1 of 1024, both 165 / 138.
-            // At just five a launch with a slot for every task is over with its longest,
-            // whose closures then wait for the matrix cores instead of other waves' (node
-            // tasks at k=6: R-MAT scale 14, 5 tasks per CU, 1.39 / 1.74; one random graph of
-            // 300 vertices, density 0.5, 3.63 / 4.82).
-            constexpr uint32_t SLOTS_PER_CU = 16;
-            kern = register_kernel(c, depth > 5 || (depth == 5 && bcnt[b] >= SLOTS_PER_CU * (uint32_t)ctx->cu));
+            // Six or more vertices below the roots: the tree is walked, and most of the time
+            // goes to closing its nodes, on the matrix cores.  Up to three: most roots close
+            // by themselves, and the operands' registers only cost waves and spills.  Between
+            // them it turns with the tasks: at four, closures of a few long tasks are shorter
+            // on the matrix cores, with many tasks the waves count; at five the few tasks'
+            // nodes spend their time above the closures, except edge tasks', whose sets are
+            // dense.  ms without / with matrix cores, and tasks of the class per CU:
+            //   <= 3  R-MAT scale 22 edge k=5, 65..128 vertices 341 / 476, 129..256 982 / 1196
+            //   4     random graph, 300 vertices, node k=5 (0.6) 0.63 / 0.49, R-MAT scale 14
+            //         node (4.9) 0.42 / 0.35, Chung-Lu n=300,000 edge k=6 (20) 0.87 / 0.81, R-MAT
+            //         scale 18 node (35) 2.18 / 2.32, Chung-Lu n=1.7M edge (1087) 26.7 / 30.0
+            //   5     random graph, 300 vertices, node k=6 (0.6) 3.52 / 4.71, R-MAT scale 14 node
+            //         (4.9) 1.29 / 1.64, scale 15 node (7.1) 2.85 / 2.65, Chung-Lu n=1M edge k=7
+            //         (543) 26.6 / 24.4, R-MAT scale 14 edge (2.5) 0.97 / 0.79
+            //   >= 6  R-MAT scale 14 node k=7 6.3 / 5.2, Chung-Lu n=1.7M edge k=8 434 / 345
+            const uint32_t cu = (uint32_t)ctx->cu;
+            constexpr uint32_t MANY_AT_4 = 24, MANY_AT_5 = 7;  // tasks per CU
+            kern = register_kernel(c, depth >= 6 || (depth == 5 && (any_edge || bcnt[b] >= MANY_AT_5 * cu)) ||
+                                          (depth == 4 && bcnt[b] < MANY_AT_4 * cu));
             L = make_layout(a.rmax, a.wmax, 0, 0, true);
             variant[b] = 2u;
         }
