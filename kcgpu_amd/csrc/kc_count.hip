@@ -514,10 +514,13 @@ struct CliqueCounts {
 //         registers at every call (R-MAT scale 22: edge tasks of 257..512 vertices
 //         at k=5 2.16 s, 1.69 s now, node tasks above 512 0.84 -> 0.73 s; 1/1024 of
 //         the edge tasks at k=8, both classes, 1.51 + 1.92 -> 1.22 + 1.58 s)
+//   WIDE_DEEP  the same for deep trees: with the matrix cores, all its register walks
+//         functions of their own (it spills 55 registers around the calls)
 //   OPEN_SCT  the serving loop's resident kernel: as LEAN, without the step from 64-
 //         to 32-vertex words inside a walk, whose two stacks do not fit its 64
 //         registers together
-enum Kind { MFMA, LEAN, WIDE_SCT, OPEN_SCT };
+enum Kind { MFMA, LEAN, WIDE_SCT, OPEN_SCT, WIDE_DEEP };
+__host__ __device__ constexpr bool wide_kind(Kind k) { return k == WIDE_SCT || k == WIDE_DEEP; }
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
@@ -773,7 +776,7 @@ __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32
                              uint32_t &ovf)
 {
     constexpr uint32_t BITS = 8 * sizeof(U);
-    constexpr bool MM = KIND == MFMA;
+    constexpr bool MM = KIND == MFMA || KIND == WIDE_DEEP;
     const uint32_t lane = (uint32_t)lane_id(), v = lane & (BITS - 1);
     k = uni32(k);
     U X = BITS == 64 ? (U)uni64(X0) : (U)uni32((uint32_t)X0);
@@ -845,7 +848,7 @@ __device__ uint64_t sct_word(const CountArgs &a, uint32_t k, U row, U X0, uint32
                     }
                 }
                 if (close) {
-                    const CloseTerm<KIND == WIDE_SCT> term(a, need, p);
+                    const CloseTerm<wide_kind(KIND)> term(a, need, p);
                     CliqueCounts c{0, 0, 0};
                     if (cx >= 2 && need >= 3) {
                         c = close_word<MM>(X, row, cx, need > 3);
@@ -891,10 +894,11 @@ __device__ inline uint64_t sct64(const CountArgs &a, uint32_t k, uint64_t row, u
 {
     return sct_word<KIND, uint64_t>(a, k, row, X0, h0, p0, nodes, ovf);
 }
+template <Kind KIND>
 __device__ __attribute__((noinline)) uint64_t sct64_wide(const CountArgs &a, uint32_t k, uint64_t row, uint64_t X0,
                                                          uint32_t h0, uint32_t p0, uint64_t &nodes, uint32_t &ovf)
 {
-    return sct64<WIDE_SCT>(a, k, row, X0, h0, p0, nodes, ovf);
+    return sct64<KIND>(a, k, row, X0, h0, p0, nodes, ovf);
 }
 
 // A set of task vertices as S uniform words.
@@ -1153,6 +1157,15 @@ __device__ __attribute__((always_inline)) uint64_t pivot_reg(const CountArgs &a,
                               uint32_t *idx, uint64_t &nodes, uint32_t &ovf, uint32_t p0, uint64_t *crows, uint32_t wv = 0,
                               uint32_t nw = 1);
 
+// the register walks of the deep block-wide kernel, functions of their own
+template <int S>
+__device__ __attribute__((noinline)) uint64_t pivot_deep(const CountArgs &a, uint32_t k, const uint64_t *rows, uint32_t R,
+                                                         uint32_t h0, uint32_t *idx, uint64_t &nodes, uint32_t &ovf,
+                                                         uint32_t p0, uint64_t *crows)
+{
+    return pivot_reg<S, WIDE_DEEP>(a, k, rows, R, h0, idx, nodes, ovf, p0, crows);
+}
+
 // triangles of G[X] with X in LDS (W words): the lane walks with the words in registers
 // (inline, except the sixteen-word walk; build_rows_block likewise: what the wide
 // kernel has inline is fixed here, it decides what it spills)
@@ -1174,7 +1187,7 @@ __device__ __attribute__((noinline)) uint32_t tri_lds16(const uint64_t *rows, ui
 
 // (inline always: as a function of its own it saved and restored its registers for
 // every entry of the wide kernel)
-template <bool LOCAL, bool WIDE = false>
+template <bool LOCAL, bool WIDE = false, Kind KIND = WIDE_SCT>
 __device__ __attribute__((always_inline)) uint64_t pivot_count(const CountArgs &a, uint32_t P, uint32_t k, const uint64_t *rows, uint64_t *stk,
                                 uint64_t *X, Scal *scal, uint32_t *cand, uint32_t R, uint32_t W, uint32_t h0,
                                 uint64_t &nodes, uint32_t &ovf, uint64_t *lacc, uint32_t p0 = 0, bool init_x = true,
@@ -1250,7 +1263,7 @@ __device__ __attribute__((always_inline)) uint64_t pivot_count(const CountArgs &
                     row1 = (lane == j) ? col : row1;
                 }
                 uint32_t lo = 0;
-                const uint64_t part = sct64_wide(a, k, row1, cx >= 64 ? ~0ull : ((1ull << cx) - 1), h, p, nodes, lo);
+                const uint64_t part = sct64_wide<KIND>(a, k, row1, cx >= 64 ? ~0ull : ((1ull << cx) - 1), h, p, nodes, lo);
                 add_checked(acc, wave_total(part, lo, ovf), ovf);
                 --my_nodes;  // counted again as the subtree's root
             } else if (!LOCAL && crows4 && cx > 128 && cx <= 256 && h + 3 <= k && h + p + cx >= k) {
@@ -1274,7 +1287,8 @@ __device__ __attribute__((always_inline)) uint64_t pivot_count(const CountArgs &
                 }
                 sync_tree<WIDE>();
                 uint32_t lo = 0;
-                const uint64_t part = pivot_reg<4, WIDE_SCT>(a, k, crows4, cx, h, cand, nodes, lo, p, crows2);
+                const uint64_t part = KIND == WIDE_DEEP ? pivot_deep<4>(a, k, crows4, cx, h, cand, nodes, lo, p, crows2)
+                                                       : pivot_reg<4, WIDE_SCT>(a, k, crows4, cx, h, cand, nodes, lo, p, crows2);
                 add_checked(acc, wave_total(part, lo, ovf), ovf);
                 --my_nodes;
             } else if (!LOCAL && crows2 && cx <= 128 && h + 3 <= k && h + p + cx >= k) {
@@ -1291,7 +1305,8 @@ __device__ __attribute__((always_inline)) uint64_t pivot_count(const CountArgs &
                 }
                 sync_tree<WIDE>();
                 uint32_t lo = 0;
-                const uint64_t part = pivot_reg<2, WIDE_SCT>(a, k, crows2, cx, h, cand, nodes, lo, p, nullptr);
+                const uint64_t part = KIND == WIDE_DEEP ? pivot_deep<2>(a, k, crows2, cx, h, cand, nodes, lo, p, nullptr)
+                                                       : pivot_reg<2, WIDE_SCT>(a, k, crows2, cx, h, cand, nodes, lo, p, nullptr);
                 add_checked(acc, wave_total(part, lo, ovf), ovf);
                 --my_nodes;
             } else if (h + p + cx >= k) {
@@ -1475,7 +1490,8 @@ __device__ uint64_t compact_and_count(const CountArgs &a, uint32_t k, const uint
         }
     }
     const uint64_t X1 = cx >= 64 ? ~0ull : ((1ull << cx) - 1);
-    return KIND == WIDE_SCT ? sct64_wide(a, k, row1, X1, h, p, nodes, ovf) : sct64<KIND>(a, k, row1, X1, h, p, nodes, ovf);
+    if constexpr (wide_kind(KIND)) return sct64_wide<KIND>(a, k, row1, X1, h, p, nodes, ovf);
+    else return sct64<KIND>(a, k, row1, X1, h, p, nodes, ovf);
 }
 
 // Triangles of G[X] for X of up to 64*S vertices (rows of stride W in LDS) by
@@ -1742,7 +1758,8 @@ __device__ uint64_t compact2_and_count(const CountArgs &a, uint32_t k, const uin
         }
     }
     sync_tree<true>();
-    return pivot_reg<2, KIND>(a, k, crows, cx, h, idx, nodes, ovf, p, nullptr, wv, nw);
+    if constexpr (KIND == WIDE_DEEP) return pivot_deep<2>(a, k, crows, cx, h, idx, nodes, ovf, p, nullptr);
+    else return pivot_reg<2, KIND>(a, k, crows, cx, h, idx, nodes, ovf, p, nullptr, wv, nw);
 }
 
 // nw > 1: this wave is number wv of nw that walk the same subtree, each with
@@ -1831,14 +1848,14 @@ __device__ __attribute__((always_inline)) uint64_t pivot_reg(const CountArgs &a,
                 }
                 uint32_t e2 = 0;  // twice the edges of G[X]
                 if (need <= 4) e2 = wave_sum32(lsum);
-                const bool near = (S == 2 || (S == 4 && KIND == WIDE_SCT)) && need == 4 && 4 * (uint64_t)e2 >= 3ull * cx * (cx - 1);
+                const bool near = (S == 2 || (S == 4 && wide_kind(KIND))) && need == 4 && 4 * (uint64_t)e2 >= 3ull * cx * (cx - 1);
                 if (near || need <= 3 || cx == 0) {
                     if (!solo) break;  // (a chain node that closes ends the chain: the wave's branches are done)
                     // closed forms: h >= k-3, and h = k-4 over a near-clique (complement
                     // density <= 1/4)
-                    const CloseTerm<KIND == WIDE_SCT> term(a, need, p);
+                    const CloseTerm<wide_kind(KIND)> term(a, need, p);
                     CliqueCounts c{0, 0, 0};
-                    if (near && cx) c = k34_complement_rows<S, KIND == MFMA>(rows, W, X, cx);
+                    if (near && cx) c = k34_complement_rows<S, KIND == MFMA || KIND == WIDE_DEEP>(rows, W, X, cx);
                     else if (need >= 2) c.e = e2 / 2;
                     if (need == 3 && cx) c.c3 = tri_lanes<S>(rows, W, X, cx, e2, idx);
                     term.add(acc, ovf, cx, c);
@@ -2843,7 +2860,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4))) vo
     finish_wave(a, w);
 }
 
-template <bool GLOBAL>
+template <bool GLOBAL, Kind KIND>
 __global__ __launch_bounds__(512) void k_pivot_wide(CountArgs a)
 {
     extern __shared__ uint64_t lds[];
@@ -2986,7 +3003,7 @@ __global__ __launch_bounds__(512) void k_pivot_wide(CountArgs a)
                 }
             }
             const uint32_t h = end ? h0 : h0 + 1;
-            run_add(w, pivot_count<false, true>(a, g.psize, k, rows, stk, X, scal, cand, R, W, h, w.nodes, w.run_ovf,
+            run_add(w, pivot_count<false, true, KIND>(a, g.psize, k, rows, stk, X, scal, cand, R, W, h, w.nodes, w.run_ovf,
                                                 nullptr, j, false, crows2, crows4));
         }
         __syncthreads();
@@ -3844,8 +3861,15 @@ int run_queries(Scratch &scr, hipStream_t s, const std::vector<QueryRun> &qs, st
                 nw = 8;
                 WL = make_wide_layout(a.rmax, a.wmax, a.levels, nw, a.chain);
             }
-            kern = global ? reinterpret_cast<const void *>(&k_pivot_wide<true>)
-                          : reinterpret_cast<const void *>(&k_pivot_wide<false>);
+            static const void *const wide[4] = {reinterpret_cast<const void *>(&k_pivot_wide<false, WIDE_SCT>),
+                                                reinterpret_cast<const void *>(&k_pivot_wide<true, WIDE_SCT>),
+                                                reinterpret_cast<const void *>(&k_pivot_wide<false, WIDE_DEEP>),
+                                                reinterpret_cast<const void *>(&k_pivot_wide<true, WIDE_DEEP>)};
+            // (the matrix cores from six vertices below the roots, above 512 vertices from
+            // seven.  ms without / with: R-MAT scale 18, node tasks of 257..512, k=7 126 / 111,
+            // k=8 634 / 429; R-MAT scale 22, 1 of 2048 node tasks at k=7, 257..512 784 / 811,
+            // 513..1024 15,780 / 16,860; 1 of 8192 edge tasks at k=9, both 18,090 / 15,230)
+            kern = wide[(depth >= (c == 3 ? 6u : 7u) ? 2 : 0) + (global ? 1 : 0)];
             L.total = WL.total;
             variant[b] = global ? 5u : 4u;
         }

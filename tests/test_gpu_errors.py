@@ -10,7 +10,7 @@ from oracle import oracle as O
 pytestmark = pytest.mark.gpu
 
 
-def _write_oriented(path, rowptr, col, key, max_out):
+def write_oriented(path, rowptr, col, key, max_out):
     """an oriented-CSR cache file (format of Oriented.save)"""
     h = 14695981039346656037
     for b in b"".join(np.ascontiguousarray(x, dtype="<u4").tobytes() for x in (rowptr, col, key)):
@@ -29,7 +29,7 @@ def test_refused_count_leaves_nothing_running(tmp_path):
     rowptr[0] = 0
     key = np.ones(leaves + 1, np.uint32)
     key[0] = 0
-    _write_oriented(tmp_path / "star.kco", rowptr, np.arange(1, leaves + 1, dtype=np.uint32), key, leaves)
+    write_oriented(tmp_path / "star.kco", rowptr, np.arange(1, leaves + 1, dtype=np.uint32), key, leaves)
     G = K.Graph.generate(K.GEN_CHUNG_LU, seed=5, n=20_000, m=130_000, gamma=2.1, max_degree=900)
     rp, col = G.csr()
     orp, oc = O.orient(rp.astype(np.uint64), col, O.peel_priority(rp.astype(np.uint64), col)[0])
